@@ -9,7 +9,7 @@
 namespace pale {
 
 constexpr uint32_t kTile = 1024;       // compaction / scan tile (256 threads x 4)
-constexpr uint32_t kTraceBlock = 128;  // threads per traversal workgroup
+constexpr uint32_t kTraceBlock = kStackStride;  // threads per traversal workgroup
 // The layer walk's tiles are split into this many contiguous regions, one
 // cursor each; a workgroup starts in region blockIdx.x % kTraceRegions (its
 // XCD under round-robin dispatch) so each XCD's L2 serves one part of the
@@ -32,7 +32,7 @@ struct DevState {
     uint32_t evPool;       // adjoint events waiting for the transport
     uint32_t resv;         // this bounce may pass the photon capacity
     uint32_t bigCells;     // photon cells too large for the per-wave sort
-    uint32_t pad32;
+    uint32_t traceNext;    // next ray of the queue to trace (photon and adjoint traces)
     unsigned long long photonQ, gatherQ, adjointQ, deposits, events, pad;
     // Counting mode, per kernel class (photon, gather, adjoint): popped
     // nodes, AABB tests, primitive tests, gathers, gather cells, non-empty

@@ -11,6 +11,7 @@
 #include <mutex>
 #include <algorithm>
 #include <cstddef>
+#include <vector>
 
 #include "pale_kernels.h"
 
@@ -49,6 +50,12 @@ __device__ __forceinline__ void flushWork(const Work& w, DevState* st, int cls) 
     }
 }
 
+__device__ __forceinline__ void addWork(Work& w, const Work& q) {
+    w.pops += q.pops;
+    w.aabb += q.aabb;
+    w.prims += q.prims;
+}
+
 // Exclusive scan over a 256-thread block; `total` receives the block sum.
 __device__ __forceinline__ uint32_t blockExclusiveScan(uint32_t v, uint32_t& total) {
     __shared__ uint32_t waveTotals[kScanThreads / 64 + 1];
@@ -83,17 +90,16 @@ __device__ __forceinline__ uint32_t loadCount(const uint32_t* count, uint32_t ma
 }
 
 __device__ __forceinline__ LaneStack laneStack(uint2* lds, uint32_t depth) {
-    return LaneStack{(LdsUint2*)(lds + threadIdx.x), blockDim.x, depth, nullptr, 0u, depth};
+    return LaneStack{(LdsUint2*)(lds + threadIdx.x), depth, nullptr, depth};
 }
 
-// The layer walk's stack: its first inLds entries in LDS, the rest in the
-// spill area (entry k of lane l at spill[(k - inLds) * lanes + l]), so that
-// more waves fit on a CU; spill == nullptr: all in LDS.
+// A trace's stack: its first inLds entries in LDS, the rest in the lane's part
+// of the spill area, so that more waves fit on a CU; spill == nullptr: all in
+// LDS.
 __device__ __forceinline__ LaneStack walkStack(uint2* lds, uint32_t depth, uint2* spill, uint32_t inLds) {
     if (!spill) return laneStack(lds, depth);
-    const uint32_t lanes = gridDim.x * blockDim.x;
-    return LaneStack{(LdsUint2*)(lds + threadIdx.x), blockDim.x, depth, spill + blockIdx.x * blockDim.x + threadIdx.x,
-                     lanes, inLds};
+    const uint32_t l = blockIdx.x * kTraceBlock + threadIdx.x;
+    return LaneStack{(LdsUint2*)(lds + threadIdx.x), depth, spill + (size_t)l * (depth - inLds), inLds};
 }
 
 __device__ __forceinline__ float4 f4(F3 v, float w) { return make_float4(v.x, v.y, v.z, w); }
@@ -118,6 +124,7 @@ __global__ void k_iota(uint32_t* p, uint32_t n) {
 // always draws; a bounce draws only if its queue is not empty.
 __global__ void k_seed_next(DevState* st, const uint32_t* table, uint32_t len, int bounce) {
     if (blockIdx.x != 0 || threadIdx.x != 0) return;
+    st->traceNext = 0;
     if (bounce >= 0 && st->qCount == 0) {
         st->live = 0;
         return;
@@ -163,8 +170,47 @@ __global__ void k_event_pool_add(DevState* st, uint32_t cap) {
 }
 
 __global__ void k_set_queue(DevState* st, const uint32_t* src) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) st->qCount = *src;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        st->qCount = *src;
+        st->traceNext = 0;
+    }
 }
+
+// ------------------------------------------------------- queue traces --
+// Rays of a queue for the waves of a persistent grid: a wave claims 64
+// consecutive rays at a time and gives them to its lanes as they fall idle.
+struct QueueCursor {
+    uint32_t* next;             // shared by the grid, zero at the start of a launch
+    uint32_t end;               // rays to hand out
+    uint32_t at = 0, to = 0;    // the wave's claimed, untaken rays
+    bool empty = false;
+
+    __device__ QueueCursor(uint32_t* n, uint32_t e) : next(n), end(e) {}
+    // Every lane of the wave calls it; false: no ray for this lane now (t
+    // stays as it is).
+    __device__ __forceinline__ bool take(bool want, uint32_t& t) {
+        const unsigned long long need = __ballot(want);
+        if (!need || empty) return false;
+        const uint32_t lane = laneId();
+        if (at >= to) {
+            const uint32_t leader = (uint32_t)__ffsll((long long)need) - 1u;
+            uint32_t base = 0;
+            if (lane == leader) base = atomicAdd(next, 64u);
+            base = __shfl(base, (int)leader, 64);
+            if (base >= end) {
+                empty = true;
+                return false;
+            }
+            at = base;
+            to = min(base + 64u, end);
+        }
+        const uint32_t mine = at + (uint32_t)__popcll(need & ((1ull << lane) - 1ull));
+        const bool got = want && mine < to;
+        if (got) t = mine;
+        at = min(at + (uint32_t)__popcll(need), to);
+        return got;
+    }
+};
 
 // ---------------------------------------------------------- emission --
 // launchRayGenEmitterKernel (PrimalKernels.cpp:13-62)
@@ -184,21 +230,35 @@ __global__ __launch_bounds__(256) void k_emit(DevScene S, const DevState* st, ui
 }
 
 // ---------------------------------------------------- photon bounce --
-// launchIntersectKernel (PrimalKernels.cpp:65-321) for one queue.
+// launchIntersectKernel (PrimalKernels.cpp:65-321) for one queue: the hit of
+// ray i, its deposit and the ray that goes on.
 template <bool kCount>
-__global__ __launch_bounds__(kTraceBlock) void k_photon_trace(DevScene S, DevState* st, RayQueue in,
-                                                              RayQueue out, uint8_t* extFlags, PhotonArrays dep,
-                                                              uint8_t* depFlags, TraceParams tp, Reservoir rs) {
-    extern __shared__ uint2 s_stack[];
-    const LaneStack stk = walkStack(s_stack, S.stackDepth, tp.spill, tp.inLds);
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t n = st->live ? st->qCount : 0u;
-    const bool active = i < n;
-    const bool resv = st->resv != 0u;
+struct PhotonJob {
+    static constexpr bool kGoesOn = false;
+    const DevScene& S;
+    const RayQueue &in, &out;
+    const PhotonArrays& dep;
+    const TraceParams& tp;
+    const Reservoir& rs;
+    uint8_t *extFlags, *depFlags;
+    uint32_t number;  // seed of the launch
+    bool resv;
+    QueueCursor queue;
+    uint32_t i = 0;
     Work w{};
-    if (active) {
+
+    __device__ __forceinline__ bool drained() const { return queue.empty; }
+    __device__ __forceinline__ bool fetch(bool idle, F3& o, F3& d) {
+        if (!queue.take(idle, i)) return false;
+        o = ld3(in.o[i]);
+        d = ld3(in.d[i]);
+        return true;
+    }
+    __device__ __forceinline__ bool finish(bool done, const JobHit& h, const Work& wl, F3&, F3&) {
+        if (!done) return false;
+        if (kCount) addWork(w, wl);
         uint8_t ef = 0, df = 0;
-        Rng rng(perItemSeed(st->number, i));
+        Rng rng(perItemSeed(number, i));
         // depositPhotonSurface past capacity (KernelHelpers.h:1705-1718): the
         // attempt index comes from the probe pass; accept with probability
         // cap / (attempt + 1), then pick the slot (two draws of this item).
@@ -215,10 +275,9 @@ __global__ __launch_bounds__(kTraceBlock) void k_photon_trace(DevScene S, DevSta
         };
         if (resv) rs.slot[i] = kNoSlot;
         const float4 o4 = in.o[i], d4 = in.d[i], T4 = in.T[i];
-        const F3 o = ld3(o4), d = ld3(d4), T = ld3(T4);
+        const F3 d = ld3(d4), T = ld3(T4);
         const uint32_t bounce = f2u(d4.w);
-        Hit h;
-        if (intersectScene<kCount>(S, o, d, stk, h, w)) {
+        if (h.inst != kInvalid) {
             const DevInstance& I = S.inst[h.inst];
             F3 no = mk3(0, 0, 0), nT = mk3(0, 0, 0), ndir = d;
             bool spawn = false;
@@ -238,11 +297,12 @@ __global__ __launch_bounds__(kTraceBlock) void k_photon_trace(DevScene S, DevSta
             } else {
                 const float u = rng.nextFloat();
                 const SurfelShade sh = S.shade[h.prim];
+                const float hAlpha = jobAlpha(S, h);
                 if (u < tp.qNull) {
-                    const float att = 1.0f - h.alpha * sh.opacity;
-                    const float w = att / tp.qNull;
+                    const float att = 1.0f - hAlpha * sh.opacity;
+                    const float wn = att / tp.qNull;
                     no = h.pos + d * 1e-5f;
-                    nT = T * w;
+                    nT = T * wn;
                     spawn = true;
                 } else if (u < tp.qNull + tp.qReflect) {
                     const F3 nc = mk3(sh.nsx, sh.nsy, sh.nsz);
@@ -259,7 +319,7 @@ __global__ __launch_bounds__(kTraceBlock) void k_photon_trace(DevScene S, DevSta
                     sampleUniformHemi(rng, on, ndir, pdf);
                     const float cosT = fmaxf(0.0f, dot(ndir, on));
                     const F3 fs = (sh.alpha_r * mk3(sh.ar, sh.ag, sh.ab)) * kInvPi;
-                    const float alpha = h.alpha * sh.opacity;
+                    const float alpha = hAlpha * sh.opacity;
                     const F3 w = divs(((alpha / tp.qReflect) * fs) * cosT, pdf);
                     no = h.pos + on * 1e-5f;
                     nT = T * w;
@@ -273,7 +333,7 @@ __global__ __launch_bounds__(kTraceBlock) void k_photon_trace(DevScene S, DevSta
                     sampleUniformHemi(rng, on, ndir, pdf);
                     const float cosT = fmaxf(0.0f, dot(ndir, on));
                     const F3 fs = (0.0f * mk3(sh.ar, sh.ag, sh.ab)) * kInvPi;  // alpha_t = 0
-                    const float alpha = h.alpha * sh.opacity;
+                    const float alpha = hAlpha * sh.opacity;
                     const F3 w = divs(((alpha / tp.qReflect) * fs) * cosT, pdf);
                     no = h.pos + (-on) * 1e-5f;
                     nT = T * w;
@@ -289,9 +349,27 @@ __global__ __launch_bounds__(kTraceBlock) void k_photon_trace(DevScene S, DevSta
         }
         extFlags[i] = ef;
         depFlags[i] = df;
+        return false;
     }
-    waveCount(active, &st->photonQ);
-    if (kCount) flushWork(w, st, kWorkPhoton);
+};
+
+template <bool kCount, bool kTopLds>
+__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_photon_trace(
+    DevScene S, DevState* st, RayQueue in, RayQueue out, uint8_t* extFlags, PhotonArrays dep, uint8_t* depFlags,
+    TraceParams tp, Reservoir rs) {
+    extern __shared__ uint2 s_stack[];
+    __shared__ TopLds sTop;
+    if (kTopLds) loadTopLds(S, sTop);
+    const LaneStack stk = walkStack(s_stack, S.stackDepth, tp.spill, tp.inLds);
+    const uint32_t n = st->live ? st->qCount : 0u;
+    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&st->photonQ, (unsigned long long)n);
+    PhotonJob<kCount> job{S,  in,       out,      dep,        tp,          rs, extFlags, depFlags, st->number,
+                          st->resv != 0u, QueueCursor(&st->traceNext, n)};
+    if (kTopLds)
+        traceWave<kCount>(S, sTop, stk, job);
+    else
+        traceWave<kCount>(S, TopGlobal{S.tlas, S.inst}, stk, job);
+    if (kCount) flushWork(job.w, st, kWorkPhoton);
 }
 
 // Reservoir mode of one bounce: on when the deposits so far plus one per
@@ -717,6 +795,204 @@ struct BatchMap {
 
 // Slots a wave of the layer walk claims at a time from its region.
 constexpr uint32_t kWalkUnit = 64;
+// Entries a wave claims at a time, and the slot of an entry it left unused.
+constexpr uint32_t kEntryClaim = 512;
+constexpr uint32_t kNoSlotOfEntry = 0xFFFFFFFFu;
+
+// The layers of a pixel, one closest-hit query each: a lane appends the entry
+// of its hit and goes on behind it until its pixel ends, then draws another.
+template <bool kCount, typename Map, typename Top>
+struct CameraJob {
+    static constexpr bool kGoesOn = true;
+    const DevScene& S;
+    const Top& top;
+    DevState* st;
+    const Map& map;
+    const PixelArrays& px;
+    const EntryArrays& ent;
+    uint32_t cap;
+    uint32_t* cursor;
+    uint32_t tiles, region;
+    uint32_t emptyRegions = 0;
+    uint32_t chunkNext = 0, chunkEnd = 0;  // the wave's claimed, untaken slots
+    bool exhausted = false;
+    // Entries are claimed entClaim at a time: one claim per entry append made
+    // every wave wait for an atomic on the one counter of the grid, and with
+    // queries that end a few lanes at a time the walk took 58 ms that way
+    // against 38 ms (1M surfels, 800x800, 16 shared-seed passes).  What a wave
+    // has claimed and not used when it ends is marked as holes (leaveHoles).
+    uint32_t entClaim;
+    uint32_t entNext = 0, entEnd = 0;
+    uint32_t layers = 0;
+    uint32_t pixel = 0, r = 0, layer = 0;
+    float tr = 1.0f;
+    Work w{};
+
+    __device__ __forceinline__ bool drained() const { return exhausted; }
+
+    __device__ __forceinline__ void leaveHoles() const {
+        for (uint32_t e = entNext + laneId(); e < min(entEnd, cap); e += 64u)
+            ent.qb[e] = make_float4(0.0f, 0.0f, u2f(kNoSlotOfEntry), 0.0f);
+    }
+
+    // Draws pixels for the idle lanes until each has one or the slots run out
+    // (a lane that drew a finished pixel, or none, draws again).
+    __device__ __forceinline__ bool fetch(bool idle, F3& o, F3& d) {
+        const uint32_t lane = laneId();
+        bool got = false;
+        while (!exhausted) {
+            const unsigned long long need = __ballot(idle && !got);
+            if (!need) break;
+            // The wave claims a whole 64-slot unit (a few pixels in all their
+            // passes) of its region and keeps what its lanes have not taken
+            // for its next draws: its lanes stay on neighbouring rays.
+            // Claiming only what the lanes need interleaves the waves' draws
+            // and scatters each wave over many pixels (the walk took 17 %
+            // longer, 28 % with decorrelated passes).
+            if (chunkNext >= chunkEnd) {
+                // Slots [lo, hi) of the current region; cursor[region] counts
+                // the slots drawn from it this round.
+                const uint32_t lo = (uint32_t)(((uint64_t)region * tiles) / kTraceRegions) * 64u;
+                const uint32_t hi = (uint32_t)(((uint64_t)(region + 1u) * tiles) / kTraceRegions) * 64u;
+                const uint32_t leader = (uint32_t)__ffsll((long long)need) - 1u;
+                uint32_t base = 0;
+                if (lane == leader) base = lo + atomicAdd(cursor + region, kWalkUnit);
+                base = __shfl(base, (int)leader, 64);
+                if (base >= hi) {
+                    // Used up (it stays so): the next region, done after all.
+                    if (++emptyRegions == kTraceRegions) exhausted = true;
+                    region = (region + 1u) % kTraceRegions;
+                    continue;
+                }
+                chunkNext = base;
+                chunkEnd = min(base + kWalkUnit, hi);
+                if (*reinterpret_cast<volatile const uint32_t*>(&st->overflow) != 0u) {
+                    exhausted = true;
+                    break;
+                }
+            }
+            if (idle && !got) {
+                const uint32_t slot = chunkNext + (uint32_t)__popcll(need & ((1ull << lane) - 1ull));
+                uint32_t p = 0;
+                if (slot < chunkEnd && map.locate(slot, p) && f2u(px.cs[p].w) == kPixActive) {
+                    pixel = p;
+                    got = true;
+                    const float4 a = px.ot[p], b = px.dl[p];
+                    o = mk3(a.x, a.y, a.z);
+                    tr = a.w;
+                    d = mk3(b.x, b.y, b.z);
+                    layer = f2u(b.w);
+                    r = 0;
+                }
+            }
+            chunkNext = min(chunkNext + (uint32_t)__popcll(need), chunkEnd);
+        }
+        return got;
+    }
+
+    __device__ __forceinline__ bool finish(bool done, const JobHit& h, const Work& wl, F3& o, F3& d) {
+        const uint32_t lane = laneId();
+        const bool want = done && h.inst != kInvalid;
+        bool terminal = true, gather = false;
+        F3 q = mk3(0, 0, 0), n = mk3(0, 0, 0), k = mk3(0, 0, 0), nextO = o;
+        float wgt = 0.0f, nextTr = tr;
+        if (want) {
+            const DevInstance& I = top.inst[h.inst];
+            if (I.type == kGeoCloud) {
+                const SurfelShade sh = S.shade[h.prim];
+                n = mk3(sh.nsx, sh.nsy, sh.nsz);
+                if (dot(n, -d) < 0.0f) n = -n;
+                q = h.pos;
+                gather = true;
+                k = (sh.alpha_r * mk3(sh.ar, sh.ag, sh.ab)) * kInvPi;
+                const float ae = sh.opacity * jobAlpha(S, h);
+                wgt = tr * ae;
+                nextTr = tr * (1.0f - ae);
+                nextO = h.pos + d * 1e-4f;
+                terminal = false;
+            } else {
+                const DevMaterial m = S.mats[I.material];
+                const F3 base = mk3(m.r, m.g, m.b);
+                wgt = tr;
+                if (m.power > 0.0f) {
+                    k = vmin(base * m.power, mk3(1.0f, 1.0f, 1.0f));
+                } else {
+                    q = h.pos;
+                    n = hitNormal(S, h);
+                    gather = true;
+                    k = base * kInvPi;
+                }
+            }
+        }
+        // Append of the entries, in lane order: from the wave's claimed
+        // range, then from a new one.
+        const unsigned long long m = __ballot(want);
+        uint32_t e = 0xFFFFFFFFu;
+        if (m) {
+            const uint32_t count = (uint32_t)__popcll(m), mine = (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+            const uint32_t left = entEnd - entNext, taken = min(count, left);
+            e = entNext + mine;
+            entNext += taken;
+            if (taken < count) {
+                const uint32_t leader = (uint32_t)__ffsll((long long)m) - 1u, claim = max(entClaim, count - taken);
+                uint32_t base = 0;
+                if (lane == leader) base = atomicAdd(&st->entries, claim);
+                base = __builtin_amdgcn_readfirstlane(__shfl(base, (int)leader, 64));
+                if (mine >= taken) e = base + (mine - taken);
+                entNext = base + (count - taken);
+                entEnd = base + claim;
+            }
+        }
+        bool full = false, more = false;
+        if (done) {
+            if (want && e >= cap) {
+                // No room: stop before this layer, resume next round.
+                px.ot[pixel] = f4(o, tr);
+                px.dl[pixel] = f4(d, u2f(layer));
+                st->overflow = 1u;
+                px.cnt[pixel] = r;
+                full = true;
+            } else {
+                ++layers;
+                if (kCount) addWork(w, wl);
+                if (want) {
+                    ent.qa[e] = f4(q, n.x);
+                    ent.qb[e] = make_float4(n.y, n.z, u2f(pixel), u2f(r | (gather ? 0u : kEntryNoGather)));
+                    ent.comp[e] = f4(k, wgt);
+                    ++r;
+                    ++layer;
+                }
+                if (terminal) {
+                    px.cnt[pixel] = r;
+                    px.cs[pixel].w = u2f(kPixFinished);
+                } else {
+                    o = nextO;
+                    tr = nextTr;
+                    more = true;
+                }
+            }
+        }
+        if (__any(full)) exhausted = true;
+        return more;
+    }
+};
+
+template <bool kCount, typename Map, typename Top>
+__device__ __forceinline__ void camTrace(const DevScene& S, const Top& top, DevState* st, const Map& map,
+                                         const PixelArrays& px, const EntryArrays& ent, uint32_t cap, uint32_t* cursor,
+                                         const LaneStack& stk) {
+    CameraJob<kCount, Map, Top> job{S, top, st, map, px, ent, cap, cursor, map.slots() >> 6, blockIdx.x % kTraceRegions};
+    // At most an eighth of the buffer is claimed ahead; below 64 entries a
+    // wave claims what it appends.
+    const uint32_t waves = gridDim.x * (kTraceBlock / 64u);
+    const uint32_t share = min(cap / (8u * waves), kEntryClaim);
+    job.entClaim = share < 64u ? 0u : share;
+    traceWave<kCount>(S, top, stk, job);
+    job.leaveHoles();
+    const uint32_t ws = waveSum(job.layers);
+    if (laneId() == 0 && ws) atomicAdd(&st->gatherQ, (unsigned long long)ws);
+    if (kCount) flushWork(job.w, st, kWorkGather);
+}
 
 template <bool kCount, typename Map, bool kTopLds>
 __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_cam_trace(
@@ -726,164 +1002,10 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(4))
     __shared__ TopLds sTop;
     if (kTopLds) loadTopLds(S, sTop);
     const LaneStack stk = walkStack(s_stack, S.stackDepth, spill, inLds);
-    const uint32_t lane = laneId();
-    const uint32_t slots = map.slots();
-    const uint32_t tiles = slots >> 6;
-    uint32_t region = blockIdx.x % kTraceRegions, emptyRegions = 0;
-    uint32_t chunkNext = 0, chunkEnd = 0;  // the wave's claimed, untaken slots
-    uint32_t layers = 0;
-    Work w{};
-    bool active = false, exhausted = false;
-    uint32_t pixel = 0, r = 0, layer = 0;
-    F3 o = mk3(0, 0, 0), d = mk3(0, 0, 0);
-    float tr = 1.0f;
-    while (true) {
-        if (!exhausted) {
-            const unsigned long long need = __ballot(!active);
-            if (need) {
-                // Slots [lo, hi) of the current region; cursor[region] counts
-                // the slots drawn from it this round.
-                const uint32_t lo = (uint32_t)(((uint64_t)region * tiles) / kTraceRegions) * 64u;
-                const uint32_t hi = (uint32_t)(((uint64_t)(region + 1u) * tiles) / kTraceRegions) * 64u;
-                // The wave claims a whole 64-slot unit (a few pixels in all
-                // their passes) and keeps what its lanes have not taken for
-                // its next draws: its lanes stay on neighbouring rays.
-                // Claiming only what the lanes need interleaves the waves'
-                // draws and scatters each wave over many pixels (the walk
-                // took 17 % longer, 28 % with decorrelated passes).
-                if (chunkNext >= chunkEnd) {
-                    const uint32_t leader = (uint32_t)__ffsll((long long)need) - 1u;
-                    uint32_t base = 0;
-                    if (lane == leader) base = lo + atomicAdd(cursor + region, kWalkUnit);
-                    base = __shfl(base, (int)leader, 64);
-                    if (base >= hi) {
-                        // Used up (it stays so): the next region, done after all.
-                        if (++emptyRegions == kTraceRegions) exhausted = true;
-                        region = (region + 1u) % kTraceRegions;
-                    } else {
-                        chunkNext = base;
-                        chunkEnd = min(base + kWalkUnit, hi);
-                        if (*reinterpret_cast<volatile const uint32_t*>(&st->overflow) != 0u) exhausted = true;
-                    }
-                }
-                if (chunkNext < chunkEnd) {
-                    if (!active) {
-                        const uint32_t slot = chunkNext + (uint32_t)__popcll(need & ((1ull << lane) - 1ull));
-                        uint32_t p = 0;
-                        if (slot < chunkEnd && map.locate(slot, p) && f2u(px.cs[p].w) == kPixActive) {
-                            pixel = p;
-                            active = true;
-                            const float4 a = px.ot[p], b = px.dl[p];
-                            o = mk3(a.x, a.y, a.z);
-                            tr = a.w;
-                            d = mk3(b.x, b.y, b.z);
-                            layer = f2u(b.w);
-                            r = 0;
-                        }
-                    }
-                    chunkNext = min(chunkNext + (uint32_t)__popcll(need), chunkEnd);
-                }
-            }
-        }
-        if (!__any(active)) {
-            // Every lane drew a finished pixel (or none): draw again until the
-            // slots run out or the entry buffer has filled.  Leaving here
-            // earlier would strand the pixels no other wave draws.
-            if (exhausted) break;
-            continue;
-        }
-        // One layer: closest hit, then the entry it contributes.
-        bool want = false, terminal = true, gather = false;
-        F3 q = mk3(0, 0, 0), n = mk3(0, 0, 0), k = mk3(0, 0, 0), nextO = o;
-        float wgt = 0.0f, nextTr = tr;
-        Work wl{};
-        if (active) {
-            Hit h;
-            const bool hit = kTopLds ? intersectSceneTop<kCount, 2>(S, sTop, o, d, stk, h, wl)
-                                     : intersectSceneTop<kCount, 2>(S, TopGlobal{S.tlas, S.inst}, o, d, stk, h, wl);
-            if (hit) {
-                const DevInstance& I = kTopLds ? sTop.inst[h.inst] : S.inst[h.inst];
-                want = true;
-                if (I.type == kGeoCloud) {
-                    const SurfelShade sh = S.shade[h.prim];
-                    n = mk3(sh.nsx, sh.nsy, sh.nsz);
-                    if (dot(n, -d) < 0.0f) n = -n;
-                    q = h.pos;
-                    gather = true;
-                    k = (sh.alpha_r * mk3(sh.ar, sh.ag, sh.ab)) * kInvPi;
-                    const float ae = sh.opacity * h.alpha;
-                    wgt = tr * ae;
-                    nextTr = tr * (1.0f - ae);
-                    nextO = h.pos + d * 1e-4f;
-                    terminal = false;
-                } else {
-                    const DevMaterial m = S.mats[I.material];
-                    const F3 base = mk3(m.r, m.g, m.b);
-                    wgt = tr;
-                    if (m.power > 0.0f) {
-                        k = vmin(base * m.power, mk3(1.0f, 1.0f, 1.0f));
-                    } else {
-                        q = h.pos;
-                        n = hitNormal(S, h);
-                        gather = true;
-                        k = base * kInvPi;
-                    }
-                }
-            }
-        }
-        // Wave-aggregated append of the entries of this iteration.
-        const unsigned long long m = __ballot(want);
-        uint32_t e = 0xFFFFFFFFu;
-        if (m) {
-            const uint32_t leader = (uint32_t)__ffsll((long long)m) - 1u;
-            uint32_t base = 0;
-            if (lane == leader) base = atomicAdd(&st->entries, (uint32_t)__popcll(m));
-            base = __shfl(base, (int)leader, 64);
-            if (want) e = base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-        }
-        bool full = false;
-        if (active) {
-            bool finished = false;
-            if (want && e >= cap) {
-                // No room: stop before this layer, resume next round.
-                px.ot[pixel] = f4(o, tr);
-                px.dl[pixel] = f4(d, u2f(layer));
-                st->overflow = 1u;
-                px.cnt[pixel] = r;
-                active = false;
-                full = true;
-            } else {
-                ++layers;
-                if (kCount) {
-                    w.pops += wl.pops;
-                    w.aabb += wl.aabb;
-                    w.prims += wl.prims;
-                }
-                if (want) {
-                    ent.qa[e] = f4(q, n.x);
-                    ent.qb[e] = make_float4(n.y, n.z, u2f(pixel), u2f(r | (gather ? 0u : kEntryNoGather)));
-                    ent.comp[e] = f4(k, wgt);
-                    ++r;
-                    ++layer;
-                }
-                if (terminal) {
-                    finished = true;
-                } else {
-                    o = nextO;
-                    tr = nextTr;
-                }
-            }
-            if (finished) {
-                px.cnt[pixel] = r;
-                px.cs[pixel].w = u2f(kPixFinished);
-                active = false;
-            }
-        }
-        if (__any(full)) exhausted = true;
-    }
-    const uint32_t ws = waveSum(layers);
-    if (lane == 0 && ws) atomicAdd(&st->gatherQ, (unsigned long long)ws);
-    if (kCount) flushWork(w, st, kWorkGather);
+    if (kTopLds)
+        camTrace<kCount>(S, sTop, st, map, px, ent, cap, cursor, stk);
+    else
+        camTrace<kCount>(S, TopGlobal{S.tlas, S.inst}, st, map, px, ent, cap, cursor, stk);
 }
 
 // The lanes of a wave that hold the same key, wherever they sit: the lowest
@@ -929,10 +1051,12 @@ __global__ __launch_bounds__(256) void k_entry_key(GridParams g, const DevState*
         uint32_t c = kNoCell;
         if (i < n) {
             const float4 b = ent.qb[i];
-            const uint32_t tag = f2u(b.w);
-            const uint32_t pos = px.off[f2u(b.z)] + (tag & ~kEntryNoGather);
+            const uint32_t tag = f2u(b.w), slot = f2u(b.z);
+            const uint32_t pos = slot == kNoSlotOfEntry ? 0u : px.off[slot] + (tag & ~kEntryNoGather);
             ent.pos[i] = pos;
-            if (tag & kEntryNoGather) {
+            if (slot == kNoSlotOfEntry) {
+                // claimed and not used by its wave
+            } else if (tag & kEntryNoGather) {
                 const float4 k = ent.comp[i];
                 ent.contrib[pos] = f4(k.w * mk3(k.x, k.y, k.z), 0.0f);
             } else {
@@ -1087,7 +1211,10 @@ __global__ __launch_bounds__(256) void k_adj_raygen(DevCamera cam, const float* 
                                                     PendingArrays pend, DevState* st, uint32_t seed) {
     const uint32_t npx = cam.W * cam.H;
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i == 0) st->qCount = npx;
+    if (i == 0) {
+        st->qCount = npx;
+        st->traceNext = 0;
+    }
     if (i >= npx) return;
     Rng rng(perItemSeed((uint64_t)seed, i));
     const float jx = rng.nextFloat() - 0.5f;
@@ -1105,7 +1232,10 @@ __global__ __launch_bounds__(256) void k_adj_raygen(DevCamera cam, const float* 
 __global__ __launch_bounds__(256) void k_adj_raygen_batch(BatchDesc b, const float* dloss, RayQueue q,
                                                           PendingArrays pend, DevState* st) {
     const uint32_t t = blockIdx.x * 4u + (threadIdx.x >> 6);
-    if (blockIdx.x == 0 && threadIdx.x == 0) st->qCount = b.hdr->nSlots;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        st->qCount = b.hdr->nSlots;
+        st->traceNext = 0;
+    }
     if (t >= b.hdr->nTiles) return;
     uint32_t seg, pxx, pxy;
     const BatchSeg* sp;
@@ -1161,44 +1291,52 @@ __global__ __launch_bounds__(64) void k_group_lanes(const uint32_t* segFirst, co
     }
 }
 
-// launchAdjointIntersectKernel (AdjointKernels.cpp:87-386) for one queue.
-// Capped at 128 VGPRs (4 waves per SIMD): it needs 125 without spills since
-// the hit's alpha is a call (uncapped it took 129, and 3 waves per SIMD ran
-// 5-8 % slower).
+// launchAdjointIntersectKernel (AdjointKernels.cpp:87-386) for one queue: the
+// hit of ray i, the pending event it completes, the event it makes and the
+// ray that goes on.
 template <bool kCount>
-__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_adj_trace(DevScene S, DevState* st, uint32_t bounceIndex,
-                                                           RayQueue in, RayQueue out, uint8_t* extFlags,
-                                                           EventArrays ev, uint8_t* evFlags, PendingArrays pend,
-                                                           uint32_t pendCap, TraceParams tp) {
-    extern __shared__ uint2 s_stack[];
-    const LaneStack stk = walkStack(s_stack, S.stackDepth, tp.spill, tp.inLds);
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t n = st->qCount;
-    uint32_t i = t;
-    bool active = t < n;
-    if (tp.groups) {
-        // Lane t -> (view group, segment, rank) -> queue index.
-        active = false;
-        uint32_t lo = 0, hi = tp.nGroups;  // last group whose first lane <= t
-        while (hi - lo > 1u) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (tp.groups[mid].z <= t)
-                lo = mid;
-            else
-                hi = mid;
-        }
-        const uint4 gr = tp.nGroups ? tp.groups[lo] : make_uint4(0u, 0u, 0u, 0u);
-        const uint32_t local = t - gr.z;
-        if (t >= gr.z && local < gr.y * gr.w) {
-            const uint32_t s = tp.groupSegs[gr.x + local % gr.y], r = local / gr.y;
-            if (r < tp.segEnd[s] - tp.segFirst[s]) {
-                i = tp.segFirst[s] + r;
-                active = true;
-            }
-        }
-    }
+struct AdjointJob {
+    static constexpr bool kGoesOn = false;
+    const DevScene& S;
+    const RayQueue &in, &out;
+    const EventArrays& ev;
+    const PendingArrays& pend;
+    const TraceParams& tp;
+    uint8_t *extFlags, *evFlags;
+    uint32_t bounceIndex, pendCap;
+    QueueCursor queue;  // of queue indices, or of lanes of the view groups
+    uint32_t i = 0;
     Work w{};
-    if (active) {
+
+    __device__ __forceinline__ bool drained() const { return queue.empty; }
+    __device__ __forceinline__ bool fetch(bool idle, F3& o, F3& d) {
+        uint32_t t;
+        if (!queue.take(idle, t)) return false;
+        i = t;
+        if (tp.groups) {
+            // Place t -> (view group, segment, rank) -> queue index.
+            uint32_t lo = 0, hi = tp.nGroups;  // last group whose first place <= t
+            while (hi - lo > 1u) {
+                const uint32_t mid = (lo + hi) >> 1;
+                if (tp.groups[mid].z <= t)
+                    lo = mid;
+                else
+                    hi = mid;
+            }
+            const uint4 gr = tp.groups[lo];
+            const uint32_t local = t - gr.z;
+            if (t < gr.z || local >= gr.y * gr.w) return false;
+            const uint32_t s = tp.groupSegs[gr.x + local % gr.y], r = local / gr.y;
+            if (r >= tp.segEnd[s] - tp.segFirst[s]) return false;
+            i = tp.segFirst[s] + r;
+        }
+        o = ld3(in.o[i]);
+        d = ld3(in.d[i]);
+        return true;
+    }
+    __device__ __forceinline__ bool finish(bool done, const JobHit& h, const Work& wl, F3&, F3&) {
+        if (!done) return false;
+        if (kCount) addWork(w, wl);
         uint8_t ef = 0, vf = 0;
         const float4 o4 = in.o[i], d4 = in.d[i], T4 = in.T[i];
         const uint32_t seg = f2u(T4.w);
@@ -1211,10 +1349,10 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(4))
         const uint32_t dpx = !tp.debug ? 0u
                              : tp.segs ? tp.segs[seg].pixOffset + (path - tp.segs[seg].slotBase)
                                        : tp.debugBase + path;
-        Hit h;
-        if (intersectScene<kCount>(S, o, d, stk, h, w)) {
+        if (h.inst != kInvalid) {
             const DevInstance& I = S.inst[h.inst];
             const bool cloud = I.type == kGeoCloud;
+            const float hAlpha = cloud ? jobAlpha(S, h) : 0.0f;
             F3 on, ng = mk3(0, 0, 0), dir;
             float pdf;
             SurfelShade sh{};
@@ -1244,7 +1382,7 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(4))
                     ev.e0[i] = f4(h.pos, u2f(kind));
                     if (reflectDone) {
                         ev.e1[i] = f4(on, u2f(h.prim));
-                        ev.e2[i] = f4(Tp, h.alpha);
+                        ev.e2[i] = f4(Tp, hAlpha);
                         ev.e3[i] = make_float4(u2f(S.inst[p2.y].material), pdf, endCos, invS);
                         if (tp.fullGradients || tp.debug) {  // this ray hit the endpoint surfel
                             ev.e4[i] = f4(o, 0.0f);
@@ -1288,27 +1426,27 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(4))
             } else {
                 const float u = rng.nextFloat();
                 if (u < tp.qNull) {
-                    const float att = 1.0f - h.alpha * sh.opacity;
-                    const float w = att / tp.qNull;
+                    const float att = 1.0f - hAlpha * sh.opacity;
+                    const float wn = att / tp.qNull;
                     no = h.pos + d * 1e-5f;
                     ndir = d;
-                    nT = T * w;
+                    nT = T * wn;
                     spawn = true;
                     newKind = kNullT;
                     pT = divs(T, tp.qNull);
-                    pAlpha = h.alpha;
+                    pAlpha = hAlpha;
                     pIds = make_uint2(h.prim, kInvalid);
                 } else if (u < tp.qNull + tp.qReflect) {
                     const F3 fs = (sh.alpha_r * mk3(sh.ar, sh.ag, sh.ab)) * kInvPi;
                     const float cosT = fmaxf(0.0f, dot(dir, on));
-                    const float alpha = h.alpha * sh.opacity;
+                    const float alpha = hAlpha * sh.opacity;
                     const F3 mult = divs((alpha / tp.qReflect) * (fs * cosT), pdf);
                     no = h.pos + on * 1e-5f;
                     nT = T * mult;
                     spawn = true;
                     projection = bounceIndex == 0;
                 } else if (u < tp.qNull + tp.qReflect + tp.qTransmit) {
-                    const float alpha = h.alpha * sh.opacity;
+                    const float alpha = hAlpha * sh.opacity;
                     const float w = (alpha * 0.0f) / tp.qTransmit;  // alpha_t = 0
                     const F3 nc = mk3(sh.nsx, sh.nsy, sh.nsz);
                     const float sc = dot(nc, -d);
@@ -1334,7 +1472,7 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(4))
                 if (projection && path < pendCap) {
                     ev.e0[i] = f4(h.pos, u2f(kProjection));
                     ev.e1[i] = f4(on, u2f(h.prim));
-                    ev.e2[i] = f4(divs(T, tp.qReflect), h.alpha);
+                    ev.e2[i] = f4(divs(T, tp.qReflect), hAlpha);
                     ev.e3[i] = make_float4(0.0f, 0.0f, 0.0f, invS);
                     if (tp.fullGradients || tp.debug) {
                         ev.e4[i] = f4(o, 0.0f);
@@ -1350,9 +1488,32 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(4))
         }
         extFlags[i] = ef;
         evFlags[i] = vf;
+        return false;
     }
-    waveCount(active, &st->adjointQ);
-    if (kCount) flushWork(w, st, kWorkAdjoint);
+};
+
+template <bool kCount, bool kTopLds>
+__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_adj_trace(
+    DevScene S, DevState* st, uint32_t bounceIndex, RayQueue in, RayQueue out, uint8_t* extFlags, EventArrays ev,
+    uint8_t* evFlags, PendingArrays pend, uint32_t pendCap, TraceParams tp) {
+    extern __shared__ uint2 s_stack[];
+    __shared__ TopLds sTop;
+    if (kTopLds) loadTopLds(S, sTop);
+    const LaneStack stk = walkStack(s_stack, S.stackDepth, tp.spill, tp.inLds);
+    const uint32_t n = st->qCount;
+    uint32_t end = n;
+    if (tp.groups) {
+        const uint4 last = tp.nGroups ? tp.groups[tp.nGroups - 1u] : make_uint4(0u, 0u, 0u, 0u);
+        end = last.z + last.y * last.w;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&st->adjointQ, (unsigned long long)n);
+    AdjointJob<kCount> job{S,  in,       out,     ev,          pend,    tp,
+                           extFlags, evFlags, bounceIndex, pendCap, QueueCursor(&st->traceNext, end)};
+    if (kTopLds)
+        traceWave<kCount>(S, sTop, stk, job);
+    else
+        traceWave<kCount>(S, TopGlobal{S.tlas, S.inst}, stk, job);
+    if (kCount) flushWork(job.w, st, kWorkAdjoint);
 }
 
 // Counting sort of the pooled events by the photon-grid cell of their
@@ -1667,6 +1828,32 @@ void launchEmit(hipStream_t s, const DevScene& S, DevState* st, uint32_t P, floa
                 uint8_t* flags) {
     if (P) k_emit<<<blocks(P, 256), 256, 0, s>>>(S, st, P, invEmitted, staged, flags);
 }
+// Persistent grid of a trace kernel: as many workgroups as fit on the device.
+// Renderers on several host threads share the cache.
+static uint32_t traceGrid(const void* kernel, size_t lds) {
+    struct Entry {
+        const void* kernel;
+        size_t lds;
+        int dev;
+        uint32_t grid;
+    };
+    static std::mutex lock;
+    static std::vector<Entry> cache;  // a few kernels, one LDS size per stack depth
+    int dev = 0, cus = 0, perCu = 0;
+    (void)hipGetDevice(&dev);
+    std::lock_guard<std::mutex> guard(lock);
+    for (const Entry& e : cache)
+        if (e.kernel == kernel && e.lds == lds && e.dev == dev) return e.grid;
+    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCu, kernel, kTraceBlock, lds);
+    cache.push_back(Entry{kernel, lds, dev, (uint32_t)std::max(1, cus) * (uint32_t)std::max(1, perCu)});
+    return cache.back().grid;
+}
+template <bool kCount, typename Map, bool kTopLds>
+static uint32_t camTraceGrid(size_t lds) {
+    return traceGrid(reinterpret_cast<const void*>(&k_cam_trace<kCount, Map, kTopLds>), lds);
+}
+
 void launchPhotonTrace(hipStream_t s, const DevScene& S, DevState* st, uint32_t maxRays, RayQueue in,
                        RayQueue staged, uint8_t* extFlags, PhotonArrays dep, uint8_t* depFlags, TraceParams tp,
                        Reservoir rs, uint32_t* tiles, bool count) {
@@ -1684,10 +1871,11 @@ void launchPhotonTrace(hipStream_t s, const DevScene& S, DevState* st, uint32_t 
         k_resv_rank<<<nt, kScanThreads, 0, s>>>(depFlags, st, tiles, rs.attempt);
     }
     const size_t lds = tp.spill ? (size_t)tp.inLds * sizeof(uint2) * kTraceBlock : stackBytes(S);
-    if (count)
-        k_photon_trace<true><<<g, kTraceBlock, lds, s>>>(S, st, in, staged, extFlags, dep, depFlags, tp, rs);
-    else
-        k_photon_trace<false><<<g, kTraceBlock, lds, s>>>(S, st, in, staged, extFlags, dep, depFlags, tp, rs);
+    const bool top = topFitsLds(S);
+    const auto k = count ? (top ? &k_photon_trace<true, true> : &k_photon_trace<true, false>)
+                         : (top ? &k_photon_trace<false, true> : &k_photon_trace<false, false>);
+    const uint32_t pg = min(traceGrid(reinterpret_cast<const void*>(k), lds), blocks(maxRays, kTraceBlock));
+    k<<<pg, kTraceBlock, lds, s>>>(S, st, in, staged, extFlags, dep, depFlags, tp, rs);
 }
 void launchReservoirWrite(hipStream_t s, DevState* st, uint32_t maxRays, Reservoir rs, PhotonArrays dep,
                           PhotonArrays raw) {
@@ -1741,25 +1929,6 @@ void launchBuildGrid(hipStream_t s, const GridParams& g, DevState* st, uint32_t 
     k_cell_sort<<<blocks(g.total, 256), 256, 0, s>>>(g.total, cellStart, sortedIdx, st, cellId);
     k_cell_sort_big<<<min(pb, 2048u), 256, 0, s>>>(st, cellId, cellStart, sortedIdx);
     k_cell_payload<<<pb, 256, 0, s>>>(st, cap, sortedIdx, raw, sorted);
-}
-
-// Persistent grid of the camera trace: as many workgroups as fit on the device.
-// Renderers on several host threads share the cache.
-template <bool kCount, typename Map, bool kTopLds>
-static uint32_t camTraceGrid(size_t lds) {
-    static std::mutex lock;
-    static uint32_t cached[2] = {0, 0};
-    static size_t cachedLds[2] = {0, 0};
-    const int k = kCount ? 1 : 0;
-    std::lock_guard<std::mutex> guard(lock);
-    if (cached[k] && cachedLds[k] == lds) return cached[k];
-    int dev = 0, cus = 0, perCu = 0;
-    (void)hipGetDevice(&dev);
-    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCu, k_cam_trace<kCount, Map, kTopLds>, kTraceBlock, lds);
-    cached[k] = (uint32_t)std::max(1, cus) * (uint32_t)std::max(1, perCu);
-    cachedLds[k] = lds;
-    return cached[k];
 }
 
 void launchExclusiveScan(hipStream_t s, const uint32_t* in, uint32_t* out, uint32_t n, uint32_t* tiles,
@@ -1904,14 +2073,12 @@ void launchAdjTrace(hipStream_t s, const DevScene& S, DevState* st, uint32_t max
                     RayQueue staged, uint8_t* extFlags, EventArrays ev, uint8_t* evFlags, PendingArrays pend,
                     TraceParams tp, bool count) {
     if (!maxRays) return;
-    const dim3 g(blocks(maxRays, kTraceBlock));
     const size_t lds = tp.spill ? (size_t)tp.inLds * sizeof(uint2) * kTraceBlock : stackBytes(S);
-    if (count)
-        k_adj_trace<true><<<g, kTraceBlock, lds, s>>>(S, st, bounce, in, staged, extFlags, ev, evFlags, pend,
-                                                      maxRays, tp);
-    else
-        k_adj_trace<false><<<g, kTraceBlock, lds, s>>>(S, st, bounce, in, staged, extFlags, ev, evFlags, pend,
-                                                       maxRays, tp);
+    const bool top = topFitsLds(S);
+    const auto k = count ? (top ? &k_adj_trace<true, true> : &k_adj_trace<true, false>)
+                         : (top ? &k_adj_trace<false, true> : &k_adj_trace<false, false>);
+    const uint32_t g = min(traceGrid(reinterpret_cast<const void*>(k), lds), blocks(maxRays, kTraceBlock));
+    k<<<g, kTraceBlock, lds, s>>>(S, st, bounce, in, staged, extFlags, ev, evFlags, pend, maxRays, tp);
 }
 void launchEventSort(hipStream_t s, const GridParams& g, DevState* st, uint32_t poolCap, EventArrays ev,
                      uint32_t* cell, uint32_t* sorted, uint32_t* cellCount, uint32_t* cellStart, uint32_t* tiles,

@@ -1,0 +1,105 @@
+"""The wave-level traversal at its edges, against the oracle: queues of fewer
+rays than a wave, of one wave and around multiples of 64 (claims of a queue),
+clouds of one leaf, of a few leaves and of leaves with fewer than four
+surfels, a top level too large for its copy in LDS, degenerate surfels (NaN
+normals, whose tests accept a NaN distance), and entry buffers that waves
+claim ahead of use and that overflow.
+
+Hits, deposits and images are the same expressions in the same order on both
+sides (bit-exact); gradients within 1e-4 of the largest (order of FP32
+atomics), the repository's bars.
+"""
+import numpy as np
+import pytest
+
+from differentiablepointrendering_amd import scene
+
+pytestmark = pytest.mark.gpu
+
+
+def _pair(spec, settings):
+    from differentiablepointrendering_amd.pale import Renderer
+    from oracle.oracle import Oracle
+
+    print(f"case: n={len(spec.points['position'])} meshes={len(spec.meshes)} settings={settings}", flush=True)
+    return Renderer.from_spec(spec, settings), Oracle.from_spec(spec, settings)
+
+
+def _check(gpu, orc, backward=True):
+    a, b = gpu.render_forward()["camera1_raw"], orc.render_forward()["camera1_raw"]
+    pa, pb = gpu.photons(), orc.photons()
+    assert pa["count"] == pb["count"] and pa["attempted"] == pb["attempted"]
+    for k in ("position", "power", "direction"):
+        assert np.array_equal(pa[k], pb[k]), k
+    assert np.array_equal(a, b, equal_nan=True)
+    if backward:
+        dl = (a[..., :3] / a[..., :3].size).astype(np.float32)
+        g = gpu.render_backward({"camera1": dl})[0]["opacity"]
+        want = orc.render_backward({"camera1": dl})
+        assert np.allclose(g, want, rtol=1e-4, atol=1e-4 * (float(np.abs(want).max()) or 1.0))
+
+
+@pytest.mark.parametrize("photons", [1, 63, 64, 65, 127, 129, 1000])
+@pytest.mark.parametrize("size", [(1, 1), (9, 7), (65, 1)])
+def test_queue_sizes(photons, size):
+    spec = scene.config_scene(0, n=700, width=size[0], height=size[1])
+    gpu, orc = _pair(spec, dict(photons=photons, gather_passes=2, adjoint_passes=2))
+    _check(gpu, orc)
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 11, 13, 50])
+def test_leaf_sizes(n):
+    pts = scene.uniform_surfels(n, seed=3, scale_lo=0.3, scale_hi=0.6)[0]
+    spec = scene.SceneSpec([scene.light_quad()], [scene.default_camera(40, 24)], pts,
+                           dict(photons=3000, bounces=4, forward_passes=2, gather_passes=3, adjoint_bounces=4,
+                                adjoint_passes=2, seed=5, gather_radius=0.2, spp_decorrelate=1))
+    gpu, orc = _pair(spec, {})
+    _check(gpu, orc)
+
+
+@pytest.mark.parametrize("meshes", [7, 8, 20])
+def test_top_level_beside_its_lds_copy(meshes):
+    spec = scene.config_scene(0, n=300, width=40, height=32)
+    for i in range(meshes - 1):
+        a = 2.0 * np.pi * i / (meshes - 1)
+        spec.meshes.append(scene.quad_mesh(f"q{i}", (1.2 * np.cos(a), -1.1 + 0.02 * i, 1.2 * np.sin(a)),
+                                           scene.FACING_UP, 0.25, (0.6, 0.5, 0.4)))
+    gpu, orc = _pair(spec, dict(photons=4000, gather_passes=2, adjoint_passes=2))
+    _check(gpu, orc)
+
+
+def test_degenerate_surfels_accept_nan_distances():
+    pts = scene.uniform_surfels(40, seed=4, scale_lo=0.2, scale_hi=0.4)[0]
+    pts["tangent_v"][[3, 17, 18]] = pts["tangent_u"][[3, 17, 18]]  # no plane: normalize(0)
+    spec = scene.SceneSpec([scene.light_quad()], [scene.default_camera(24, 24)], pts, {})
+    gpu, orc = _pair(spec, dict(photons=100))
+    rng = np.random.default_rng(1)
+    o = rng.uniform(-1.5, 1.5, size=(3000, 3)).astype(np.float32)
+    d = rng.normal(size=(3000, 3)).astype(np.float32)
+    a, b = gpu.trace_rays(o, d), orc.trace(o, d)
+    for k in ("instance", "primitive"):
+        assert np.array_equal(a[k], b[k]), k
+    # The same through the wave traversal: one-layer photon map over the cloud.
+    gpu, orc = _pair(spec, dict(photons=2000, bounces=1, forward_passes=1, gather_passes=1))
+    gpu.build_photon_map()
+    orc.build_photon_map()
+    pa, pb = gpu.photons(), orc.photons()
+    assert pa["count"] == pb["count"]
+    assert np.array_equal(pa["position"], pb["position"], equal_nan=True)
+
+
+@pytest.mark.parametrize("budget", [8, 9, 16, 60])
+def test_entry_claims_and_their_holes(budget):
+    pts = scene.uniform_surfels(30_000, seed=6, scale_lo=0.03, scale_hi=0.08)[0]  # about 20 layers per pixel
+    spec = scene.SceneSpec([scene.light_quad()], [scene.default_camera(150, 90)], pts,
+                           dict(photons=5000, bounces=3, forward_passes=1, gather_passes=3, adjoint_passes=1,
+                                gather_radius=0.05, spp_decorrelate=1))
+    from differentiablepointrendering_amd.pale import Renderer
+
+    print(f"case: entries per pixel {budget}", flush=True)
+    want = Renderer.from_spec(spec, dict(gather_entry_budget=1)).render_forward()["camera1_raw"]  # claims nothing ahead
+    r = Renderer.from_spec(spec, dict(gather_entry_budget=budget))
+    got = r.render_forward()["camera1_raw"]
+    rounds = r.stats()["camera_rounds"]
+    assert np.array_equal(got, want)
+    assert rounds > 1 if budget < 10 else rounds >= 1

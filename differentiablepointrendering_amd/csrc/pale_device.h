@@ -35,12 +35,13 @@ struct DevScene {
 };
 
 struct DevGrid {
-    const float4* posPow;  // sorted photons: position, power.x
-    const float4* dirPow;  // incoming direction, power.y
-    const float* powZ;     // power.z
+    const float4* posPow;  // sorted photons: position, power.x / (pi radius^2)
+    const float4* dirPow;  // incoming direction, power.y / (pi radius^2)
+    const float* powZ;     // power.z / (pi radius^2)
     const uint32_t* cellStart;  // exclusive prefix over cells, total+1 entries
     float ox, oy, oz;
     float cx, cy, cz;
+    float inv;  // 1 / the cell size
     int rx, ry, rz;
     float radius;
     const uint32_t* attempted;  // deposits attempted (T), device memory
@@ -963,36 +964,59 @@ __device__ __forceinline__ void worldToCell(const DevGrid& g, F3 p, int& x, int&
     z = min(max((int)floorf(f.z), 0), g.rz - 1);
 }
 
-// Cells of one grid row (cy, cz) that can hold a photon within radius r of
-// q: the row is skipped when its y-z extent lies farther than r from q, and
-// otherwise the x range shrinks to the chord of the sphere.  Every bound is
-// widened by a margin (1e-3 of a cell plus 2e-6 of the coordinates) that
-// exceeds the binary32 rounding of worldToCell and of the distance test by
-// orders of magnitude, and boundary cells, which also hold the photons that
-// worldToCell clamps into them, extend to infinity.  A photon in a skipped
-// cell therefore fails the reference's d2 > r2 test, so skipping it leaves
-// the sum unchanged.
-__device__ __forceinline__ bool rowSpan(const DevGrid& g, F3 q, float r2, int cy, int cz, int lx, int hx, int& ax,
-                                        int& bx) {
-    auto axisGap = [](float qc, float o, float c, int i, int res, float m) {
-        const float lo = (i == 0) ? -INFINITY : o + (float)i * c - m;
-        const float hi = (i == res - 1) ? INFINITY : o + (float)(i + 1) * c + m;
-        return fmaxf(fmaxf(lo - qc, qc - hi), 0.0f);
-    };
-    const float my = 1e-3f * g.cy + 2e-6f * (fabsf(q.y) + fabsf(g.oy) + g.radius);
-    const float mz = 1e-3f * g.cz + 2e-6f * (fabsf(q.z) + fabsf(g.oz) + g.radius);
-    const float dy = axisGap(q.y, g.oy, g.cy, cy, g.ry, my);
-    const float dz = axisGap(q.z, g.oz, g.cz, cz, g.rz, mz);
-    const float room = r2 * 1.001f - (dy * dy + dz * dz);
-    if (!(room >= 0.0f)) return false;
-    const float hw = sqrtf(room);
-    const float mx = 1e-3f * g.cx + 2e-6f * (fabsf(q.x) + fabsf(g.ox) + g.radius);
-    const float fa = floorf((q.x - hw - mx - g.ox) / g.cx);
-    const float fb = floorf((q.x + hw + mx - g.ox) / g.cx);
-    ax = (fa > (float)lx) ? (int)fa : lx;
-    bx = (fb < (float)hx) ? (int)fb : hx;
-    return ax <= bx;
-}
+// Rows of the grid that can hold a photon within radius r of a point of the
+// box [qlo, qhi] (one point: qlo = qhi): a row (cy, cz) is skipped when its
+// y-z extent lies farther than r from the box, and otherwise its x range
+// shrinks to the chords of the sphere.  Every bound is widened by a margin,
+// 1e-3 of a cell plus 2e-6 of the coordinates, far above the binary32 rounding
+// of worldToCell, of the distance test and of the bounds themselves (a dozen
+// roundings of 6e-8 relative to the coordinates), and boundary cells, which
+// also hold the photons that worldToCell clamps into them, extend to infinity.
+// A photon in a skipped cell therefore fails the reference's d2 > r2 test, so
+// skipping it leaves the sum unchanged.  Nothing here enters a sum, so the
+// bounds need no correctly rounded operations: with an IEEE square root and
+// two IEEE divisions per row the 25 rows of a gather cost more vector
+// instructions than its photons.
+struct GridRows {
+    float c, inv;          // cell size, 1 / cell size
+    float ylo, yhi, zlo, zhi;  // gaps to the faces of cell 0: ylo + i c and yhi - i c to cell i's
+    float x0, x1;          // the box's x range, widened, in cells
+    float room;            // r^2 and a little
+
+    __device__ __forceinline__ GridRows(const DevGrid& g, F3 qlo, F3 qhi, float r2) {
+        c = g.cx;
+        inv = g.inv;
+        const float m = 1e-3f * c;
+        const float mx = m + 2e-6f * (fmaxf(fabsf(qlo.x), fabsf(qhi.x)) + fabsf(g.ox) + g.radius);
+        const float my = m + 2e-6f * (fmaxf(fabsf(qlo.y), fabsf(qhi.y)) + fabsf(g.oy) + g.radius);
+        const float mz = m + 2e-6f * (fmaxf(fabsf(qlo.z), fabsf(qhi.z)) + fabsf(g.oz) + g.radius);
+        ylo = g.oy - my - qhi.y;
+        yhi = qlo.y - g.oy - my - c;
+        zlo = g.oz - mz - qhi.z;
+        zhi = qlo.z - g.oz - mz - c;
+        x0 = (qlo.x - mx - g.ox) * inv;
+        x1 = (qhi.x + mx - g.ox) * inv;
+        room = r2 * 1.001f;
+    }
+    __device__ __forceinline__ float gap(float lo, float hi, int i, int res) const {
+        const float t = (float)i * c;
+        const float a = i == 0 ? 0.0f : lo + t, b = i == res - 1 ? 0.0f : hi - t;
+        return fmaxf(fmaxf(a, b), 0.0f);
+    }
+    // what slice cz leaves of room
+    __device__ __forceinline__ float slice(const DevGrid& g, int cz) const {
+        const float d = gap(zlo, zhi, cz, g.rz);
+        return room - d * d;
+    }
+    __device__ __forceinline__ bool span(const DevGrid& g, float left, int cy, int lx, int hx, int& ax, int& bx) const {
+        const float d = gap(ylo, yhi, cy, g.ry);
+        const float rest = left - d * d;
+        const float hw = __builtin_amdgcn_sqrtf(fmaxf(rest, 0.0f)) * inv;
+        ax = max((int)floorf(x0 - hw), lx);
+        bx = min((int)floorf(x1 + hw), hx);
+        return rest >= 0.0f && ax <= bx;
+    }
+};
 
 typedef __attribute__((address_space(4))) const float4 ConstF4;
 typedef __attribute__((address_space(4))) const float ConstF;
@@ -1009,30 +1033,14 @@ __device__ __forceinline__ float waveMaxF(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
 }
 
-// rowSpan for every point of the box [qlo, qhi]: the row is skipped only
-// when its extent lies farther than r from the whole box, and the x range
-// covers the chords of all its points (every bound and margin is monotone in
-// the point, so the span contains each point's own span).
-__device__ __forceinline__ bool rowSpanBox(const DevGrid& g, F3 qlo, F3 qhi, float r2, int cy, int cz, int lx,
-                                           int hx, int& ax, int& bx) {
-    auto axisGap = [](float ql, float qh, float o, float c, int i, int res, float m) {
-        const float lo = (i == 0) ? -INFINITY : o + (float)i * c - m;
-        const float hi = (i == res - 1) ? INFINITY : o + (float)(i + 1) * c + m;
-        return fmaxf(fmaxf(lo - qh, ql - hi), 0.0f);
-    };
-    const float my = 1e-3f * g.cy + 2e-6f * (fmaxf(fabsf(qlo.y), fabsf(qhi.y)) + fabsf(g.oy) + g.radius);
-    const float mz = 1e-3f * g.cz + 2e-6f * (fmaxf(fabsf(qlo.z), fabsf(qhi.z)) + fabsf(g.oz) + g.radius);
-    const float dy = axisGap(qlo.y, qhi.y, g.oy, g.cy, cy, g.ry, my);
-    const float dz = axisGap(qlo.z, qhi.z, g.oz, g.cz, cz, g.rz, mz);
-    const float room = r2 * 1.001f - (dy * dy + dz * dz);
-    if (!(room >= 0.0f)) return false;
-    const float hw = sqrtf(room);
-    const float mx = 1e-3f * g.cx + 2e-6f * (fmaxf(fabsf(qlo.x), fabsf(qhi.x)) + fabsf(g.ox) + g.radius);
-    const float fa = floorf((qlo.x - hw - mx - g.ox) / g.cx);
-    const float fb = floorf((qhi.x + hw + mx - g.ox) / g.cx);
-    ax = (fa > (float)lx) ? (int)fa : lx;
-    bx = (fb < (float)hx) ? (int)fb : hx;
-    return ax <= bx;
+// A photon's tests and its part of the sum (its power is stored divided by
+// the disc's area, k_cell_payload).
+__device__ __forceinline__ void gatherPhoton(F3& E, F3 q, F3 n, float r2, const float4& pp, const float4& dp, float pz) {
+    const F3 dd = mk3(pp.x, pp.y, pp.z) - q;
+    // dot(n, -dir) == dot(-n, dir) exactly (negation is exact).
+    const float cosine = dot(n, -mk3(dp.x, dp.y, dp.z));
+    const float d2 = dot(dd, dd);
+    if (!(cosine < 0.0f) && !(d2 > r2)) E = E + mk3(pp.w, dp.w, pz);
 }
 
 // The gather of a full wave whose points share one cell box and lie close
@@ -1043,25 +1051,20 @@ __device__ __forceinline__ bool rowSpanBox(const DevGrid& g, F3 qlo, F3 qhi, flo
 // photons of its own box that pass its tests, in the same order as the
 // per-lane walk, so the sums are the same to the bit.
 constexpr float kWaveSpread = 0.5f;
-__device__ F3 gatherWave(const DevGrid& g, F3 q, F3 n, F3 qlo, F3 qhi, float r2, float invArea, int lx, int ly,
-                         int lz, int hx, int hy, int hz) {
+__device__ F3 gatherWave(const DevGrid& g, F3 q, F3 n, F3 qlo, F3 qhi, float r2, int lx, int ly, int lz, int hx,
+                         int hy, int hz) {
     F3 E = mk3(0, 0, 0);
-    auto addPhoton = [&](const float4& pp, const float4& dp, float pz) {
-        const F3 dd = mk3(pp.x, pp.y, pp.z) - q;
-        const float cosine = dot(n, -mk3(dp.x, dp.y, dp.z));
-        if (cosine < 0.0f) return;
-        const float d2 = dot(dd, dd);
-        if (d2 > r2) return;
-        E = E + mk3(pp.w, dp.w, pz) * invArea;
-    };
+    auto addPhoton = [&](const float4& pp, const float4& dp, float pz) { gatherPhoton(E, q, n, r2, pp, dp, pz); };
+    const GridRows rows(g, qlo, qhi, r2);
     const ConstF4* pos = (const ConstF4*)g.posPow;
     const ConstF4* dir = (const ConstF4*)g.dirPow;
     const ConstF* pzs = (const ConstF*)g.powZ;
     const ConstU32* cs = (const ConstU32*)g.cellStart;
     for (int cz = lz; cz <= hz; ++cz) {
+        const float left = rows.slice(g, cz);
         for (int cy = ly; cy <= hy; ++cy) {
             int ax, bx;
-            if (!rowSpanBox(g, qlo, qhi, r2, cy, cz, lx, hx, ax, bx)) continue;
+            if (!rows.span(g, left, cy, lx, hx, ax, bx)) continue;
             ax = __builtin_amdgcn_readfirstlane(ax);
             bx = __builtin_amdgcn_readfirstlane(bx);
             const uint32_t row = (uint32_t)((cz * g.ry + cy) * g.rx);
@@ -1095,9 +1098,9 @@ __device__ F3 gatherWave(const DevGrid& g, F3 q, F3 n, F3 qlo, F3 qhi, float r2,
 // stored sorted by (cell, deposit index), so the cells of one grid row form
 // one contiguous range; summation order equals the reference's cell-by-cell,
 // photon-by-photon order.  Cells that cannot hold an accepted photon are not
-// scanned (rowSpan).  Memory-level parallelism: the row bounds of a whole
+// scanned (GridRows).  Memory-level parallelism: the row bounds of a whole
 // z-slice are loaded before any photon of that slice, and photons are loaded
-// four at a time (added in order).  Counting mode counts the reference's
+// two at a time (added in order).  Counting mode counts the reference's
 // cells and photons (the whole box), not the scanned ones.  kWave (the
 // camera gather, whose waves hold cell-sorted points, with shared seeds
 // often the same point several times): a wave whose points share a cell box
@@ -1110,7 +1113,6 @@ __device__ F3 gatherIrradiance(const DevGrid& g, F3 q, F3 n, Work& w) {
     if (!g.valid) return mk3(0, 0, 0);
     const float r = g.radius;
     const float r2 = r * r;
-    const float invArea = 1.0f / (kPi * r2);
     int lx, ly, lz, hx, hy, hz;
     worldToCell(g, q - mk3(r, r, r), lx, ly, lz);
     worldToCell(g, q + mk3(r, r, r), hx, hy, hz);
@@ -1126,22 +1128,16 @@ __device__ F3 gatherIrradiance(const DevGrid& g, F3 q, F3 n, Work& w) {
             const F3 qhi = mk3(waveMaxF(q.x), waveMaxF(q.y), waveMaxF(q.z));
             const F3 ext = qhi - qlo;
             if (fmaxf(fmaxf(ext.x, ext.y), ext.z) <= kWaveSpread * r) {
-                E = gatherWave(g, q, n, qlo, qhi, r2, invArea, ulx, uly, ulz, uhx, uhy, uhz);
+                E = gatherWave(g, q, n, qlo, qhi, r2, ulx, uly, ulz, uhx, uhy, uhz);
                 waveDone = true;
             }
         }
     }
     if (!waveDone) {
-    auto addPhoton = [&](const float4& pp, const float4& dp, float pz) {
-        const F3 dd = mk3(pp.x, pp.y, pp.z) - q;
-        // dot(n, -dir) == dot(-n, dir) exactly (negation is exact).
-        const float cosine = dot(n, -mk3(dp.x, dp.y, dp.z));
-        if (cosine < 0.0f) return;
-        const float d2 = dot(dd, dd);
-        if (d2 > r2) return;
-        E = E + mk3(pp.w, dp.w, pz) * invArea;
-    };
+    auto addPhoton = [&](const float4& pp, const float4& dp, float pz) { gatherPhoton(E, q, n, r2, pp, dp, pz); };
+    const GridRows rows(g, q, q, r2);
     for (int cz = lz; cz <= hz; ++cz) {
+        const float left = rows.slice(g, cz);
         for (int cy0 = ly; cy0 <= hy; cy0 += kSliceRows) {
             uint32_t ra[kSliceRows], rb[kSliceRows];
 #pragma unroll
@@ -1149,7 +1145,7 @@ __device__ F3 gatherIrradiance(const DevGrid& g, F3 q, F3 n, Work& w) {
                 const int cy = cy0 + k;
                 ra[k] = rb[k] = 0u;
                 int ax, bx;
-                if (cy <= hy && rowSpan(g, q, r2, cy, cz, lx, hx, ax, bx)) {
+                if (cy <= hy && rows.span(g, left, cy, lx, hx, ax, bx)) {
                     const uint32_t row = (uint32_t)((cz * g.ry + cy) * g.rx);
                     ra[k] = g.cellStart[row + ax];
                     rb[k] = g.cellStart[row + bx + 1];
@@ -1165,16 +1161,16 @@ __device__ F3 gatherIrradiance(const DevGrid& g, F3 q, F3 n, Work& w) {
                 }
                 uint32_t j = ra[k];
                 const uint32_t b = rb[k];
-                for (; j + 4 <= b; j += 4) {
-                    const float4 p0 = g.posPow[j], p1 = g.posPow[j + 1], p2 = g.posPow[j + 2], p3 = g.posPow[j + 3];
-                    const float4 d0 = g.dirPow[j], d1 = g.dirPow[j + 1], d2 = g.dirPow[j + 2], d3 = g.dirPow[j + 3];
-                    const float z0 = g.powZ[j], z1 = g.powZ[j + 1], z2 = g.powZ[j + 2], z3 = g.powZ[j + 3];
+                // Two at a time, then the last: rows hold few photons (2 to 3
+                // of the 1M-surfel workload's map).
+                for (; j + 2 <= b; j += 2) {
+                    const float4 p0 = g.posPow[j], p1 = g.posPow[j + 1];
+                    const float4 d0 = g.dirPow[j], d1 = g.dirPow[j + 1];
+                    const float z0 = g.powZ[j], z1 = g.powZ[j + 1];
                     addPhoton(p0, d0, z0);
                     addPhoton(p1, d1, z1);
-                    addPhoton(p2, d2, z2);
-                    addPhoton(p3, d3, z3);
                 }
-                for (; j < b; ++j) addPhoton(g.posPow[j], g.dirPow[j], g.powZ[j]);
+                if (j < b) addPhoton(g.posPow[j], g.dirPow[j], g.powZ[j]);
             }
         }
     }

@@ -227,10 +227,11 @@ void launchCompactEvents(hipStream_t s, const uint8_t* flags, const uint32_t* co
                          uint32_t* tiles, DevState* st, EventArrays src, EventArrays pool, uint32_t poolCap);
 void launchFinishPhotonBounce(hipStream_t s, DevState* st, uint32_t cap);
 void launchSetQueue(hipStream_t s, DevState* st, const uint32_t* src);
-// Photon grid (counting sort by cell, stable in deposit order).
+// Photon grid (counting sort by cell, stable in deposit order); the sorted
+// powers are divided by the area of the gather's disc.
 void launchBuildGrid(hipStream_t s, const GridParams& g, DevState* st, uint32_t photonCap, PhotonArrays raw,
                      PhotonArrays sorted, uint32_t* cellId, uint32_t* sortedIdx, uint32_t* cellCount,
-                     uint32_t* cellStart, uint32_t* tiles, uint32_t* scratchTotal);
+                     uint32_t* cellStart, uint32_t* tiles, uint32_t* scratchTotal, float radius);
 // Exclusive scan of n values into out[0..n] (out[n] = total).
 void launchExclusiveScan(hipStream_t s, const uint32_t* in, uint32_t* out, uint32_t n, uint32_t* tiles,
                          uint32_t* scratchTotal);

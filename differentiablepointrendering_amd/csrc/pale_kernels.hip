@@ -695,15 +695,21 @@ __global__ __launch_bounds__(256) void k_cell_sort_big(const DevState* st, const
     }
 }
 
+// The gather's copy: photons in cell order, their power times 1 / (pi r^2),
+// the factor that every gather applies to it.
 __global__ __launch_bounds__(256) void k_cell_payload(const DevState* st, uint32_t cap, const uint32_t* sortedIdx,
-                                                      PhotonArrays raw, PhotonArrays sorted) {
+                                                      PhotonArrays raw, PhotonArrays sorted, float radius) {
     const uint32_t n = min(st->photonCount, cap);
     const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= n) return;
     const uint32_t k = sortedIdx[j];
-    sorted.posPow[j] = raw.posPow[k];
-    sorted.dirPow[j] = raw.dirPow[k];
-    sorted.powZ[j] = raw.powZ[k];
+    const float invArea = 1.0f / (kPi * (radius * radius));
+    float4 p = raw.posPow[k], d = raw.dirPow[k];
+    p.w *= invArea;
+    d.w *= invArea;
+    sorted.posPow[j] = p;
+    sorted.dirPow[j] = d;
+    sorted.powZ[j] = raw.powZ[k] * invArea;
 }
 
 // ---------------------------------------------------- camera gather --
@@ -1094,8 +1100,15 @@ __global__ __launch_bounds__(256) void k_entry_scatter(const DevState* st, uint3
 // One irradiance gather per entry in cell order; the entry's contribution
 // w * (E * k) goes to its place in the slot's layer list (the products the
 // reference's loop forms, PrimalKernels.cpp:583-585, :620, :626-628).
+//
+// Bound by vector instructions (issued in 80-89 % of the cycles with shared
+// seeds, 60-64 % with independent samples), then by the latency of the rows'
+// dependent loads: 5 waves per SIMD (at most 96 VGPRs) instead of 4.  12.2 ->
+// 8.8 ms and 18.1 -> 14.0 ms for the 102 M gathers of the 1M-surfel step: row
+// bounds without IEEE divisions and square roots (GridRows; -1.0, -1.8 ms),
+// photons two at a time instead of four (-1.6 ms), the fifth wave (-0.6 ms).
 template <bool kCount>
-__global__ __launch_bounds__(256) void k_entry_gather(DevGrid G, DevState* st, const uint32_t* nGather,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k_entry_gather(DevGrid G, DevState* st, const uint32_t* nGather,
                                                       EntryArrays ent) {
     // One lane per entry (a one-shot grid over the capacity): gathers vary
     // in cost, and fresh waves take the place of finished ones, which a
@@ -1915,7 +1928,7 @@ void launchSetQueue(hipStream_t s, DevState* st, const uint32_t* src) { k_set_qu
 
 void launchBuildGrid(hipStream_t s, const GridParams& g, DevState* st, uint32_t cap, PhotonArrays raw,
                      PhotonArrays sorted, uint32_t* cellId, uint32_t* sortedIdx, uint32_t* cellCount,
-                     uint32_t* cellStart, uint32_t* tiles, uint32_t* scratchTotal) {
+                     uint32_t* cellStart, uint32_t* tiles, uint32_t* scratchTotal, float radius) {
     const uint32_t pb = blocks(cap, 256);
     k_cell_count<<<pb, 256, 0, s>>>(g, st, cap, raw.posPow, cellId, cellCount);
     const uint32_t nt = blocks(g.total, kTile);
@@ -1928,7 +1941,7 @@ void launchBuildGrid(hipStream_t s, const GridParams& g, DevState* st, uint32_t 
     launchFill(s, reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(st) + offsetof(DevState, bigCells)), 1, 0u);
     k_cell_sort<<<blocks(g.total, 256), 256, 0, s>>>(g.total, cellStart, sortedIdx, st, cellId);
     k_cell_sort_big<<<min(pb, 2048u), 256, 0, s>>>(st, cellId, cellStart, sortedIdx);
-    k_cell_payload<<<pb, 256, 0, s>>>(st, cap, sortedIdx, raw, sorted);
+    k_cell_payload<<<pb, 256, 0, s>>>(st, cap, sortedIdx, raw, sorted, radius);
 }
 
 void launchExclusiveScan(hipStream_t s, const uint32_t* in, uint32_t* out, uint32_t n, uint32_t* tiles,

@@ -516,6 +516,7 @@ struct pale_handle {
         g.oy = grid.oy;
         g.oz = grid.oz;
         g.cx = g.cy = g.cz = grid.cell;
+        g.inv = 1.0f / grid.cell;
         g.rx = grid.rx;
         g.ry = grid.ry;
         g.rz = grid.rz;
@@ -1043,7 +1044,7 @@ struct pale_handle {
         launchBuildGrid(stream, grid, st, photonCap, pa(rawPosPow, rawDirPow, rawPowZ),
                         pa(srtPosPow, srtDirPow, srtPowZ), cellId.as<uint32_t>(), sortedIdx.as<uint32_t>(),
                         cellCount.as<uint32_t>(), cellStart.as<uint32_t>(), gridTiles.as<uint32_t>(),
-                        gridTotal.as<uint32_t>());
+                        gridTotal.as<uint32_t>(), radius);
         tEnd(tg);
         mapValid = true;
     }

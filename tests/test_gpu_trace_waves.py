@@ -103,3 +103,37 @@ def test_entry_claims_and_their_holes(budget):
     rounds = r.stats()["camera_rounds"]
     assert np.array_equal(got, want)
     assert rounds > 1 if budget < 10 else rounds >= 1
+
+
+@pytest.mark.parametrize("radius", [0.004, 0.02, 0.11, 0.7])
+@pytest.mark.parametrize("offset", [0.0, 37.0])
+def test_gather_rows_against_all_photons(radius, offset):
+    """The row bounds of the gather skip no accepted photon: irradiance at
+    points around the photons, at cell faces, at distance r of a photon and
+    outside the grid equals the oracle's walk over the reference's whole box,
+    also far from the origin, where the coordinates' rounding is a larger part
+    of a cell."""
+    pts = scene.uniform_surfels(2000, seed=8, scale_lo=0.05, scale_hi=0.1)[0]
+    pts["position"] = (pts["position"] + np.float32(offset)).astype(np.float32)
+    light = scene.light_quad()
+    light.object_to_world[:3, 3] += offset
+    light.world_to_object = np.linalg.inv(light.object_to_world.astype(np.float64)).astype(np.float32)
+    spec = scene.SceneSpec([light], [scene.default_camera(8, 8)], pts, {})
+    gpu, orc = _pair(spec, dict(photons=4000 if radius > 0.5 else 20_000, bounces=3, forward_passes=1,
+                                gather_radius=radius))
+    gpu.build_photon_map()
+    orc.build_photon_map()
+    p = gpu.photons()["position"]
+    rng = np.random.default_rng(2)
+    near = p[rng.integers(0, len(p), 3000)]
+    d = rng.normal(size=(3000, 3))
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    on = near + radius * d * rng.choice([0.3, 0.999999, 1.0, 1.000001, 1.4], size=(3000, 1))
+    cell = 0.5 * radius
+    lo = p.min(axis=0)
+    faces = lo + np.round((near - lo) / cell) * cell
+    out = near + 4.0 * (near - p.mean(axis=0))
+    q = np.concatenate([near, on, faces, out]).astype(np.float32)
+    n = rng.normal(size=q.shape)
+    n = (n / np.linalg.norm(n, axis=1, keepdims=True)).astype(np.float32)
+    assert np.array_equal(gpu.gather_irradiance(q, n), orc.gather(q, n))

@@ -81,9 +81,10 @@ struct PendingArrays {
     float4* p4;
 };
 
-// Camera gather, per pixel: ot = ray origin + throughput tr, dl = direction +
-// next layer (bits), cs = accumulated colour + status (bits), cnt = entries
-// of this round, off = their first slot in the ordered list.
+// Camera gather, per pixel: ot = origin of the next layer's ray + transmittance
+// tr of the layers composited so far, dl = direction, cs = accumulated colour +
+// status (bits), cnt = entries of this round, off = their first slot in the
+// ordered list.
 struct PixelArrays {
     float4* ot;
     float4* dl;
@@ -124,21 +125,18 @@ struct BatchDesc {
     const DevCamera* cams;  // per view
 };
 
-// Camera-gather entries (one per layer): qa = gather point + normal.x,
-// qb = normal.y, normal.z, pixel (bits), index in the pixel's round (bits,
-// top bit = no gather); comp = colour factor k + weight w; E = irradiance;
-// ord = entries in (pixel, layer) order; cell / sorted = counting sort of
-// the gather entries by grid cell.
-// Camera-gather entries of one round, in append order: qa = gather point +
-// normal.x, qb = normal.yz, slot, layer tag; comp = colour factor k and
-// weight w.  pos[i] = place of entry i in its slot's layer-ordered list
-// (slot offset + layer); contrib holds each entry's w * (E * k) at that place,
-// so a slot's layers are contiguous for the in-order sum.  cell / sorted:
-// the counting sort of the gather entries by photon-grid cell.
+// Camera-gather entries of one round, one per layer, in append order: the hit
+// as the walk found it.  qa = hit point + squared radius in the surfel's
+// support (a mesh: its instance, bits), qb = ray direction + primitive (bits),
+// qs = slot, layer of the round (top bit: a mesh).  pos[i] = place of entry i
+// in its slot's layer-ordered list (slot offset + layer); contrib holds at
+// that place each entry's radiance E * k and alpha * opacity, so a slot's
+// layers are contiguous for the in-order composite.  cell / sorted: the
+// counting sort of the gather entries by photon-grid cell.
 struct EntryArrays {
     float4* qa;
     float4* qb;
-    float4* comp;
+    uint2* qs;
     float4* contrib;
     uint32_t* pos;
     uint32_t* cell;
@@ -241,14 +239,14 @@ void launchCamInit(hipStream_t s, const DevCamera& cam, const DevState* st, uint
 // Layer walk: the first inLds stack entries of a lane (default
 // kWalkLdsEntries) in LDS, the rest in a spill area of
 // walkSpillBytes(S, inLds) (null: the whole stack in LDS).
-constexpr uint32_t kWalkLdsEntries = 16;
+constexpr uint32_t kWalkLdsEntries = 12;
 size_t walkSpillBytes(const DevScene& S, uint32_t inLds);
 void launchCamTrace(hipStream_t s, const DevScene& S, DevState* st, uint32_t npx, uint32_t width, PixelArrays px,
                     EntryArrays ent, uint32_t cap, uint32_t* cursor, uint2* spill, uint32_t inLds, bool count);
-void launchEntrySort(hipStream_t s, const GridParams& g, DevState* st, uint32_t cap, PixelArrays px,
+void launchEntrySort(hipStream_t s, const DevScene& S, const GridParams& g, DevState* st, uint32_t cap, PixelArrays px,
                      EntryArrays ent, uint32_t* cellCount, uint32_t* cellStart, uint32_t* tiles,
                      uint32_t* scratchTotal);
-void launchEntryGather(hipStream_t s, const DevGrid& G, DevState* st, uint32_t cap, const uint32_t* nGather,
+void launchEntryGather(hipStream_t s, const DevScene& S, const DevGrid& G, DevState* st, uint32_t cap, const uint32_t* nGather,
                        EntryArrays ent, bool count);
 void launchCamComposite(hipStream_t s, uint32_t npx, PixelArrays px, EntryArrays ent, float invSpp, float4* fb);
 // Batched camera gather: primary rays of every slot of the batch; the layer

@@ -196,7 +196,7 @@ struct QueueCursor {
             const uint32_t leader = (uint32_t)__ffsll((long long)need) - 1u;
             uint32_t base = 0;
             if (lane == leader) base = atomicAdd(next, 64u);
-            base = __shfl(base, (int)leader, 64);
+            base = __builtin_amdgcn_readlane(base, leader);
             if (base >= end) {
                 empty = true;
                 return false;
@@ -719,23 +719,27 @@ __global__ __launch_bounds__(256) void k_cell_payload(const DevState* st, uint32
 //
 //   k_cam_init      primary ray of every pixel (the reference's jitter);
 //   k_cam_trace     persistent lanes walk each pixel's layers (closest-hit
-//                   queries only) and append one entry per layer: the gather
-//                   point and normal, the layer's weight w and colour factor
-//                   k, in layer order within the pixel;
+//                   queries only) and append the hit of every layer, in layer
+//                   order within the pixel.  Where a layer's ray starts does
+//                   not depend on what the hits weigh, so the walk reads no
+//                   shading record and evaluates no alpha;
 //   k_entry_key     entry -> place in its pixel's layer list, and a
 //                   counting sort of the gather entries by photon-grid cell;
 //   k_entry_gather  one irradiance gather per entry, neighbouring lanes on
-//                   neighbouring points (shared photon rows, similar loops);
-//                   w * (E * k) goes to the entry's place in the layer list;
-//   k_cam_composite per pixel, C = C + w * (E * k) over the layers in order,
-//                   then the reference's framebuffer update.
+//                   neighbouring points (shared photon rows, similar loops),
+//                   with the hit's normal, colour factor k and alpha; E * k
+//                   and alpha * opacity go to the entry's place in the layer
+//                   list;
+//   k_cam_composite per pixel over the layers in order, w = tr * alpha *
+//                   opacity, C = C + w * (E * k), then the reference's
+//                   framebuffer update.
 //
 // Every value is computed by the same expressions as in the reference's
 // single loop, and the per-pixel sums run in layer order, so the image is
 // bit-identical.  If the entry buffer fills, a pixel stops before the layer
 // that did not fit and resumes from there in the next round.
 enum : uint32_t { kPixActive = 0u, kPixFinished = 1u, kPixFlushed = 2u };
-constexpr uint32_t kEntryNoGather = 0x80000000u;
+constexpr uint32_t kEntryMesh = 0x80000000u;
 
 __global__ __launch_bounds__(256) void k_cam_init(DevCamera cam, const DevState* st, uint32_t pass, int decorrelate,
                                                   PixelArrays px) {
@@ -749,7 +753,7 @@ __global__ __launch_bounds__(256) void k_cam_init(DevCamera cam, const DevState*
     F3 o, d;
     primaryRay(cam, (float)(i % cam.W), (float)(i / cam.W), jx, jy, o, d);
     px.ot[i] = f4(o, 1.0f);
-    px.dl[i] = f4(d, u2f(0u));
+    px.dl[i] = f4(d, 0.0f);
     px.cs[i] = make_float4(0.0f, 0.0f, 0.0f, u2f(kPixActive));
     px.cnt[i] = 0u;
 }
@@ -829,16 +833,15 @@ struct CameraJob {
     // has claimed and not used when it ends is marked as holes (leaveHoles).
     uint32_t entClaim;
     uint32_t entNext = 0, entEnd = 0;
-    uint32_t layers = 0;
-    uint32_t pixel = 0, r = 0, layer = 0;
-    float tr = 1.0f;
+    uint32_t layers = 0;  // of the wave
+    uint32_t pixel = 0, r = 0;  // r: entries of the pixel this round
     Work w{};
 
     __device__ __forceinline__ bool drained() const { return exhausted; }
 
     __device__ __forceinline__ void leaveHoles() const {
         for (uint32_t e = entNext + laneId(); e < min(entEnd, cap); e += 64u)
-            ent.qb[e] = make_float4(0.0f, 0.0f, u2f(kNoSlotOfEntry), 0.0f);
+            ent.qs[e] = make_uint2(kNoSlotOfEntry, 0u);
     }
 
     // Draws pixels for the idle lanes until each has one or the slots run out
@@ -863,7 +866,7 @@ struct CameraJob {
                 const uint32_t leader = (uint32_t)__ffsll((long long)need) - 1u;
                 uint32_t base = 0;
                 if (lane == leader) base = lo + atomicAdd(cursor + region, kWalkUnit);
-                base = __shfl(base, (int)leader, 64);
+                base = __builtin_amdgcn_readlane(base, leader);
                 if (base >= hi) {
                     // Used up (it stays so): the next region, done after all.
                     if (++emptyRegions == kTraceRegions) exhausted = true;
@@ -872,7 +875,7 @@ struct CameraJob {
                 }
                 chunkNext = base;
                 chunkEnd = min(base + kWalkUnit, hi);
-                if (*reinterpret_cast<volatile const uint32_t*>(&st->overflow) != 0u) {
+                if (__builtin_amdgcn_readfirstlane(*reinterpret_cast<volatile const uint32_t*>(&st->overflow)) != 0u) {
                     exhausted = true;
                     break;
                 }
@@ -883,11 +886,8 @@ struct CameraJob {
                 if (slot < chunkEnd && map.locate(slot, p) && f2u(px.cs[p].w) == kPixActive) {
                     pixel = p;
                     got = true;
-                    const float4 a = px.ot[p], b = px.dl[p];
-                    o = mk3(a.x, a.y, a.z);
-                    tr = a.w;
-                    d = mk3(b.x, b.y, b.z);
-                    layer = f2u(b.w);
+                    o = ld3(px.ot[p]);
+                    d = ld3(px.dl[p]);
                     r = 0;
                 }
             }
@@ -899,37 +899,7 @@ struct CameraJob {
     __device__ __forceinline__ bool finish(bool done, const JobHit& h, const Work& wl, F3& o, F3& d) {
         const uint32_t lane = laneId();
         const bool want = done && h.inst != kInvalid;
-        bool terminal = true, gather = false;
-        F3 q = mk3(0, 0, 0), n = mk3(0, 0, 0), k = mk3(0, 0, 0), nextO = o;
-        float wgt = 0.0f, nextTr = tr;
-        if (want) {
-            const DevInstance& I = top.inst[h.inst];
-            if (I.type == kGeoCloud) {
-                const SurfelShade sh = S.shade[h.prim];
-                n = mk3(sh.nsx, sh.nsy, sh.nsz);
-                if (dot(n, -d) < 0.0f) n = -n;
-                q = h.pos;
-                gather = true;
-                k = (sh.alpha_r * mk3(sh.ar, sh.ag, sh.ab)) * kInvPi;
-                const float ae = sh.opacity * jobAlpha(S, h);
-                wgt = tr * ae;
-                nextTr = tr * (1.0f - ae);
-                nextO = h.pos + d * 1e-4f;
-                terminal = false;
-            } else {
-                const DevMaterial m = S.mats[I.material];
-                const F3 base = mk3(m.r, m.g, m.b);
-                wgt = tr;
-                if (m.power > 0.0f) {
-                    k = vmin(base * m.power, mk3(1.0f, 1.0f, 1.0f));
-                } else {
-                    q = h.pos;
-                    n = hitNormal(S, h);
-                    gather = true;
-                    k = base * kInvPi;
-                }
-            }
-        }
+        const bool mesh = want && top.inst[h.inst].type == kGeoMesh;
         // Append of the entries, in lane order: from the wave's claimed
         // range, then from a new one.
         const unsigned long long m = __ballot(want);
@@ -943,38 +913,38 @@ struct CameraJob {
                 const uint32_t leader = (uint32_t)__ffsll((long long)m) - 1u, claim = max(entClaim, count - taken);
                 uint32_t base = 0;
                 if (lane == leader) base = atomicAdd(&st->entries, claim);
-                base = __builtin_amdgcn_readfirstlane(__shfl(base, (int)leader, 64));
+                base = __builtin_amdgcn_readlane(base, leader);
                 if (mine >= taken) e = base + (mine - taken);
                 entNext = base + (count - taken);
                 entEnd = base + claim;
             }
         }
-        bool full = false, more = false;
+        const bool full = want && e >= cap;
+        bool more = false;
+        layers += (uint32_t)__popcll(__ballot(done && !full));
         if (done) {
-            if (want && e >= cap) {
+            if (full) {
                 // No room: stop before this layer, resume next round.
-                px.ot[pixel] = f4(o, tr);
-                px.dl[pixel] = f4(d, u2f(layer));
+                float* ot = reinterpret_cast<float*>(px.ot + pixel);
+                ot[0] = o.x;
+                ot[1] = o.y;
+                ot[2] = o.z;
                 st->overflow = 1u;
                 px.cnt[pixel] = r;
-                full = true;
             } else {
-                ++layers;
                 if (kCount) addWork(w, wl);
                 if (want) {
-                    ent.qa[e] = f4(q, n.x);
-                    ent.qb[e] = make_float4(n.y, n.z, u2f(pixel), u2f(r | (gather ? 0u : kEntryNoGather)));
-                    ent.comp[e] = f4(k, wgt);
+                    ent.qa[e] = f4(h.pos, mesh ? u2f(h.inst) : h.r2);
+                    ent.qb[e] = f4(d, u2f(h.prim));
+                    ent.qs[e] = make_uint2(pixel, r | (mesh ? kEntryMesh : 0u));
                     ++r;
-                    ++layer;
                 }
-                if (terminal) {
+                more = want && !mesh;
+                if (more) {
+                    o = h.pos + d * 1e-4f;
+                } else {
                     px.cnt[pixel] = r;
                     px.cs[pixel].w = u2f(kPixFinished);
-                } else {
-                    o = nextO;
-                    tr = nextTr;
-                    more = true;
                 }
             }
         }
@@ -995,13 +965,16 @@ __device__ __forceinline__ void camTrace(const DevScene& S, const Top& top, DevS
     job.entClaim = share < 64u ? 0u : share;
     traceWave<kCount>(S, top, stk, job);
     job.leaveHoles();
-    const uint32_t ws = waveSum(job.layers);
-    if (laneId() == 0 && ws) atomicAdd(&st->gatherQ, (unsigned long long)ws);
+    if (laneId() == 0 && job.layers) atomicAdd(&st->gatherQ, (unsigned long long)job.layers);
     if (kCount) flushWork(job.w, st, kWorkGather);
 }
 
+// 5 waves per SIMD (96 VGPRs without spills since the walk shades nothing, and
+// kWalkLdsEntries of its stack in LDS): 57.6 -> 50.6 ms against 4 with
+// independent samples, 35.7 -> 33.4 ms shared (16 passes of 800x800, 1M
+// surfels); 6 waves spill 11 registers and run the same.
 template <bool kCount, typename Map, bool kTopLds>
-__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_cam_trace(
+__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(5))) void k_cam_trace(
     DevScene S, DevState* st, Map map, PixelArrays px, EntryArrays ent, uint32_t cap, uint32_t* cursor,
     uint2* spill, uint32_t inLds) {
     extern __shared__ uint2 s_stack[];
@@ -1042,36 +1015,40 @@ constexpr uint32_t kNoCell = 0xFFFFFFFFu;
 
 // Place of every entry in its slot's layer-ordered list; grid cell and
 // per-cell count of the gather entries (the cell of worldToCellClamped,
-// KernelHelpers.h:920-934).  An entry that gathers nothing (an emitter) has
-// its contribution w * k written here (the gather's E is one).  Neighbouring
-// entries come from neighbouring lanes of the layer walk, so a wave holds
-// few distinct cells: one atomic per distinct cell of the wave.
-// The entry kernels stride over the entries with a bounded grid: the count
-// is known only on the device and the capacity is far above it.  The loop is
-// uniform over the block, so whole waves take part in the run detection.
-__global__ __launch_bounds__(256) void k_entry_key(GridParams g, const DevState* st, uint32_t cap, PixelArrays px,
-                                                   EntryArrays ent, uint32_t* cellCount) {
+// KernelHelpers.h:920-934).  An emitter gathers nothing: its contribution is
+// written here.  Neighbouring entries come from neighbouring lanes of the
+// layer walk, so a wave holds few distinct cells: one atomic per distinct cell
+// of the wave.  The entry kernels stride over the entries with a bounded grid:
+// the count is known only on the device and the capacity is far above it.  The
+// loop is uniform over the block, so whole waves take part in the run
+// detection.
+__global__ __launch_bounds__(256) void k_entry_key(DevScene S, GridParams g, const DevState* st, uint32_t cap,
+                                                   PixelArrays px, EntryArrays ent, uint32_t* cellCount) {
     const uint32_t n = min(st->entries, cap);
     for (uint32_t i0 = blockIdx.x * blockDim.x; i0 < n; i0 += gridDim.x * blockDim.x) {
         const uint32_t i = i0 + threadIdx.x;
         uint32_t c = kNoCell;
         if (i < n) {
-            const float4 b = ent.qb[i];
-            const uint32_t tag = f2u(b.w), slot = f2u(b.z);
-            const uint32_t pos = slot == kNoSlotOfEntry ? 0u : px.off[slot] + (tag & ~kEntryNoGather);
-            ent.pos[i] = pos;
-            if (slot == kNoSlotOfEntry) {
-                // claimed and not used by its wave
-            } else if (tag & kEntryNoGather) {
-                const float4 k = ent.comp[i];
-                ent.contrib[pos] = f4(k.w * mk3(k.x, k.y, k.z), 0.0f);
-            } else {
+            const uint2 s = ent.qs[i];
+            if (s.x != kNoSlotOfEntry) {  // else claimed and not used by its wave
+                const uint32_t pos = px.off[s.x] + (s.y & ~kEntryMesh);
+                ent.pos[i] = pos;
                 const float4 a = ent.qa[i];
-                const F3 f = divv(mk3(a.x, a.y, a.z) - mk3(g.ox, g.oy, g.oz), mk3(g.cell, g.cell, g.cell));
-                const int x = min(max((int)floorf(f.x), 0), g.rx - 1);
-                const int y = min(max((int)floorf(f.y), 0), g.ry - 1);
-                const int z = min(max((int)floorf(f.z), 0), g.rz - 1);
-                c = (uint32_t)((z * g.ry + y) * g.rx + x);
+                bool gather = true;
+                if (s.y & kEntryMesh) {
+                    const DevMaterial m = S.mats[S.inst[f2u(a.w)].material];
+                    if (m.power > 0.0f) {
+                        ent.contrib[pos] = f4(vmin(mk3(m.r, m.g, m.b) * m.power, mk3(1.0f, 1.0f, 1.0f)), 1.0f);
+                        gather = false;
+                    }
+                }
+                if (gather) {
+                    const F3 f = divv(mk3(a.x, a.y, a.z) - mk3(g.ox, g.oy, g.oz), mk3(g.cell, g.cell, g.cell));
+                    const int x = min(max((int)floorf(f.x), 0), g.rx - 1);
+                    const int y = min(max((int)floorf(f.y), 0), g.ry - 1);
+                    const int z = min(max((int)floorf(f.z), 0), g.rz - 1);
+                    c = (uint32_t)((z * g.ry + y) * g.rx + x);
+                }
             }
             ent.cell[i] = c;
         }
@@ -1097,9 +1074,10 @@ __global__ __launch_bounds__(256) void k_entry_scatter(const DevState* st, uint3
     }
 }
 
-// One irradiance gather per entry in cell order; the entry's contribution
-// w * (E * k) goes to its place in the slot's layer list (the products the
-// reference's loop forms, PrimalKernels.cpp:583-585, :620, :626-628).
+// One irradiance gather per entry in cell order, and what the hit makes of it:
+// the radiance E * k and alpha * opacity (a mesh: 1) go to the entry's place in
+// the slot's layer list (the products the reference's loop forms,
+// PrimalKernels.cpp:583-585, :620, :626-628).
 //
 // Bound by vector instructions (issued in 80-89 % of the cycles with shared
 // seeds, 60-64 % with independent samples), then by the latency of the rows'
@@ -1107,9 +1085,10 @@ __global__ __launch_bounds__(256) void k_entry_scatter(const DevState* st, uint3
 // 8.8 ms and 18.1 -> 14.0 ms for the 102 M gathers of the 1M-surfel step: row
 // bounds without IEEE divisions and square roots (GridRows; -1.0, -1.8 ms),
 // photons two at a time instead of four (-1.6 ms), the fifth wave (-0.6 ms).
+// The hit's alpha and shading (taken over from the layer walk) add 0.5 ms.
 template <bool kCount>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k_entry_gather(DevGrid G, DevState* st, const uint32_t* nGather,
-                                                      EntryArrays ent) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k_entry_gather(
+    DevScene S, DevGrid G, DevState* st, const uint32_t* nGather, EntryArrays ent) {
     // One lane per entry (a one-shot grid over the capacity): gathers vary
     // in cost, and fresh waves take the place of finished ones, which a
     // strided loop would not.
@@ -1118,18 +1097,32 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
     Work w{};
     if (i < n) {
         const uint32_t e = ent.sorted[i];
-        const float4 a = ent.qa[e], b = ent.qb[e], c = ent.comp[e];
-        const uint32_t pos = ent.pos[e];
-        const F3 E = gatherIrradiance<kCount, true>(G, mk3(a.x, a.y, a.z), mk3(a.w, b.x, b.y), w);
-        const F3 Lo = E * mk3(c.x, c.y, c.z);
-        ent.contrib[pos] = f4(c.w * Lo, 0.0f);
+        const float4 a = ent.qa[e], b = ent.qb[e];
+        const uint32_t pos = ent.pos[e], prim = f2u(b.w);
+        F3 nrm, k;
+        float ae = 1.0f;
+        if (ent.qs[e].y & kEntryMesh) {
+            const JobHit h{ld3(a), f2u(a.w), prim, 0.0f};
+            nrm = hitNormal(S, h);
+            const DevMaterial m = S.mats[S.inst[h.inst].material];
+            k = mk3(m.r, m.g, m.b) * kInvPi;
+        } else {
+            const SurfelShade sh = S.shade[prim];
+            nrm = mk3(sh.nsx, sh.nsy, sh.nsz);
+            if (dot(nrm, -ld3(b)) < 0.0f) nrm = -nrm;
+            k = (sh.alpha_r * mk3(sh.ar, sh.ag, sh.ab)) * kInvPi;
+            ae = sh.opacity * hitAlpha(1.0f - a.w, S.geo[prim].e4b);
+        }
+        const F3 E = gatherIrradiance<kCount, true>(G, ld3(a), nrm, w);
+        ent.contrib[pos] = f4(E * k, ae);
     }
     if (kCount) flushWork(w, st, kWorkGather);
 }
 
 // fb == nullptr (batches): a finished pixel keeps its colour in cs and the
 // framebuffer update is left to k_batch_resolve.  nDev: device-side count.
-// C = C + w * (E * k) over the pixel's layers in order.
+// C = C + w * (E * k) over the pixel's layers in order, w = tr * alpha *
+// opacity; a pixel that goes on in another round keeps its tr.
 __global__ __launch_bounds__(256) void k_cam_composite(uint32_t npx, const uint32_t* nDev, PixelArrays px,
                                                        EntryArrays ent, float invSpp, float4* fb) {
     const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1139,7 +1132,13 @@ __global__ __launch_bounds__(256) void k_cam_composite(uint32_t npx, const uint3
     if (status == kPixFlushed) return;
     F3 C = mk3(cs.x, cs.y, cs.z);
     const uint32_t first = px.off[p], cnt = px.cnt[p];
-    for (uint32_t j = 0; j < cnt; ++j) C = C + ld3(ent.contrib[first + j]);
+    float tr = px.ot[p].w;
+    for (uint32_t j = 0; j < cnt; ++j) {
+        const float4 c = ent.contrib[first + j];
+        const float w = tr * c.w;
+        C = C + w * ld3(c);
+        tr = tr * (1.0f - c.w);
+    }
     // The next round's slot scan must see zero for every pixel it did not
     // touch, finished ones included.
     px.cnt[p] = 0u;
@@ -1151,6 +1150,7 @@ __global__ __launch_bounds__(256) void k_cam_composite(uint32_t npx, const uint3
         px.cs[p] = make_float4(C.x, C.y, C.z, u2f(kPixFlushed));
     } else {
         px.cs[p] = make_float4(C.x, C.y, C.z, u2f(kPixActive));
+        px.ot[p].w = tr;
     }
 }
 
@@ -1170,7 +1170,7 @@ __global__ __launch_bounds__(256) void k_batch_init(BatchDesc b, PixelArrays px)
     F3 o, d;
     primaryRay(b.cams[s.view], (float)pxx, (float)pxy, jx, jy, o, d);
     px.ot[slot] = f4(o, 1.0f);
-    px.dl[slot] = f4(d, u2f(0u));
+    px.dl[slot] = f4(d, 0.0f);
     px.cs[slot] = make_float4(0.0f, 0.0f, 0.0f, u2f(kPixActive));
     px.cnt[slot] = 0u;
 }
@@ -2040,23 +2040,23 @@ void launchBatchResolve(hipStream_t s, BatchDesc b, uint32_t maxResolve, PixelAr
     if (maxResolve) k_batch_resolve<<<blocks(maxResolve, 256), 256, 0, s>>>(b, px, fb);
 }
 
-void launchEntrySort(hipStream_t s, const GridParams& g, DevState* st, uint32_t cap, PixelArrays px,
+void launchEntrySort(hipStream_t s, const DevScene& S, const GridParams& g, DevState* st, uint32_t cap, PixelArrays px,
                      EntryArrays ent, uint32_t* cellCount, uint32_t* cellStart, uint32_t* tiles,
                      uint32_t* scratchTotal) {
     if (!cap) return;
     const uint32_t gb = min(blocks(cap, 256), kEntryBlocks);
-    k_entry_key<<<gb, 256, 0, s>>>(g, st, cap, px, ent, cellCount);
+    k_entry_key<<<gb, 256, 0, s>>>(S, g, st, cap, px, ent, cellCount);
     launchExclusiveScan(s, cellCount, cellStart, g.total, tiles, scratchTotal);
     k_entry_scatter<<<gb, 256, 0, s>>>(st, cap, cellStart, cellCount, ent);
 }
 
-void launchEntryGather(hipStream_t s, const DevGrid& G, DevState* st, uint32_t cap, const uint32_t* nGather,
+void launchEntryGather(hipStream_t s, const DevScene& S, const DevGrid& G, DevState* st, uint32_t cap, const uint32_t* nGather,
                        EntryArrays ent, bool count) {
     if (!cap) return;
     if (count)
-        k_entry_gather<true><<<blocks(cap, 256), 256, 0, s>>>(G, st, nGather, ent);
+        k_entry_gather<true><<<blocks(cap, 256), 256, 0, s>>>(S, G, st, nGather, ent);
     else
-        k_entry_gather<false><<<blocks(cap, 256), 256, 0, s>>>(G, st, nGather, ent);
+        k_entry_gather<false><<<blocks(cap, 256), 256, 0, s>>>(S, G, st, nGather, ent);
 }
 
 void launchCamComposite(hipStream_t s, uint32_t npx, PixelArrays px, EntryArrays ent, float invSpp, float4* fb) {

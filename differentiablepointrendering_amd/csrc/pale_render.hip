@@ -376,7 +376,7 @@ struct pale_handle {
     pale_batch_tuning tune{};
     hipGraphExec_t bGraph = nullptr;
     std::vector<uint8_t> bGraphKey;
-    DevMem pxOt, pxDl, pxCs, pxCnt, pxOff, pxTiles, entQa, entQb, entComp, entContrib, entPos, entCell, entSorted,
+    DevMem pxOt, pxDl, pxCs, pxCnt, pxOff, pxTiles, entQa, entQb, entQs, entContrib, entPos, entCell, entSorted,
         entStart, flagHost;
     // Device state and seed table.
     DevMem state, seedTable, cursors;
@@ -777,7 +777,7 @@ struct pale_handle {
     // stay.  They are allocated again by the next view.
     std::vector<DevMem*> viewBuffers() {
         std::vector<DevMem*> v = {&pxOt,    &pxDl,    &pxCs,    &pxCnt,  &pxOff, &pxTiles, &entQa,  &entQb,
-                                  &entComp, &entContrib, &entPos, &entCell, &entSorted, &viewFb, &viewLdr, &pend0,
+                                  &entQs, &entContrib, &entPos, &entCell, &entSorted, &viewFb, &viewLdr, &pend0,
                                   &pend1,   &pend2,   &pend3,   &pend4,  &evCell, &evSorted, &evFlags, &dloss,
                                   &bTiles,  &bSegs,   &bRuns,   &bHdr,   &bCams, &bSegFirst, &viewsFb, &viewsLdr};
         for (int k = 0; k < 6; ++k) {
@@ -853,7 +853,7 @@ struct pale_handle {
         if (want != entryCap) {
             a(entQa, (size_t)want * 16);
             a(entQb, (size_t)want * 16);
-            a(entComp, (size_t)want * 16);
+            a(entQs, (size_t)want * 8);
             a(entContrib, (size_t)want * 16);
             a(entPos, (size_t)want * 4);
             a(entCell, (size_t)want * 4);
@@ -877,7 +877,7 @@ struct pale_handle {
                            pxOff.as<uint32_t>()};
     }
     EntryArrays enta() const {
-        return EntryArrays{entQa.as<float4>(),    entQb.as<float4>(),    entComp.as<float4>(),
+        return EntryArrays{entQa.as<float4>(),    entQb.as<float4>(),    entQs.as<uint2>(),
                            entContrib.as<float4>(), entPos.as<uint32_t>(), entCell.as<uint32_t>(),
                            entSorted.as<uint32_t>()};
     }
@@ -901,11 +901,11 @@ struct pale_handle {
             tEnd(tt);
             const size_t ts = tBegin(kTCamSort);
             launchExclusiveScan(stream, px.cnt, px.off, npx, pxTiles.as<uint32_t>(), gridTotal.as<uint32_t>());
-            launchEntrySort(stream, grid, st, entryCap, px, ent, cellCount.as<uint32_t>(), entStart.as<uint32_t>(),
+            launchEntrySort(stream, scene, grid, st, entryCap, px, ent, cellCount.as<uint32_t>(), entStart.as<uint32_t>(),
                             gridTiles.as<uint32_t>(), gridTotal.as<uint32_t>());
             tEnd(ts);
             const size_t tk = tBegin(kTGather);
-            launchEntryGather(stream, G, st, entryCap, entStart.as<uint32_t>() + grid.total, ent, countWork);
+            launchEntryGather(stream, scene, G, st, entryCap, entStart.as<uint32_t>() + grid.total, ent, countWork);
             tEnd(tk);
             const size_t tc = tBegin(kTCamSort);
             launchCamComposite(stream, npx, px, ent, invSpp, fbp);
@@ -1092,11 +1092,11 @@ struct pale_handle {
         if (timed) tEnd(tt);
         const size_t ts = timed ? tBegin(kTCamSort) : 0;
         launchExclusiveScan(stream, px.cnt, px.off, maxSlots, pxTiles.as<uint32_t>(), gridTotal.as<uint32_t>());
-        launchEntrySort(stream, grid, st(), entryCap, px, ent, cellCount.as<uint32_t>(), entStart.as<uint32_t>(),
+        launchEntrySort(stream, scene, grid, st(), entryCap, px, ent, cellCount.as<uint32_t>(), entStart.as<uint32_t>(),
                         gridTiles.as<uint32_t>(), gridTotal.as<uint32_t>());
         if (timed) tEnd(ts);
         const size_t tk = timed ? tBegin(kTGather) : 0;
-        launchEntryGather(stream, devGrid(), st(), entryCap, entStart.as<uint32_t>() + grid.total, ent, count);
+        launchEntryGather(stream, scene, devGrid(), st(), entryCap, entStart.as<uint32_t>() + grid.total, ent, count);
         if (timed) tEnd(tk);
         const size_t tc = timed ? tBegin(kTCamSort) : 0;
         launchCamCompositeBatch(stream, maxSlots, bHdr.as<BatchHeader>(), px, ent);

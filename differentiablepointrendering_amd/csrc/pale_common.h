@@ -150,6 +150,18 @@ struct alignas(16) WideNode {
     uint32_t left, right, pad0, pad1;
 };
 
+// Two levels of the cloud's tree in one record (128 B), for the traversal that
+// does not count work: slots 0 and 1 hold the boxes of the left child's two
+// children, 2 and 3 the right child's; a child that is a leaf takes the first
+// slot of its pair, and the second repeats its box with no reference.  Plane k
+// of every slot is one 16-byte word.  A quad node has its node's index and
+// refers to quad nodes by it.
+struct alignas(16) QuadNode {
+    float mnx[4], mxx[4], mny[4], mxy[4], mnz[4], mxz[4];
+    uint32_t ref[4];  // kInvalid: no node
+    uint32_t pad[4];
+};
+
 PALE_HD uint32_t leafRef(uint32_t first, uint32_t count) { return kLeafBit | (first << 2) | (count - 1u); }
 PALE_HD uint32_t leafFirst(uint32_t ref) { return (ref & ~kLeafBit) >> 2; }
 PALE_HD uint32_t leafCount(uint32_t ref) { return (ref & 3u) + 1u; }

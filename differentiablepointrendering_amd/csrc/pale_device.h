@@ -21,6 +21,7 @@ struct DevScene {
     const SurfelGeo* geo;
     const SurfelShade* shade;
     const WideNode* nodes;
+    const QuadNode* quads;  // of the cloud's nodes
     const TriGeo* tris;
     const DevInstance* inst;
     const TlasNode* tlas;
@@ -53,7 +54,6 @@ struct Hit {
     F3 pos;
     float t;
     float alpha;
-    float r2;       // a surfel: squared radius in its support
     uint32_t inst;  // kInvalid: miss
     uint32_t prim;
 };
@@ -120,6 +120,16 @@ struct LaneStack {
             ++sp;
         }
     }
+    // The cloud traversal holds at most three entries per two levels of the
+    // tree, which the stack is made for.
+    __device__ __forceinline__ void pushBounded(uint32_t& sp, uint32_t ref, float t) const {
+        const uint2 v = make_uint2(ref, __float_as_uint(t));
+        if (sp < inLds)
+            base[sp * kStackStride] = v;
+        else
+            spill[sp - inLds] = v;
+        ++sp;
+    }
     // The LDS read is unconditional and a relaxed atomic load, so that it
     // stays an LDS instruction: two plain loads would be merged into one
     // generic (flat) load of a selected address, which goes through the
@@ -138,7 +148,6 @@ struct LocalHit {
     F3 pos;
     float t;
     float alpha;
-    float r2;
     uint32_t prim;
 };
 
@@ -225,7 +234,6 @@ __device__ bool traverseCloud(const DevScene& S, const DevInstance& I, F3 o, F3 
     out.t = best;
     out.prim = bestIdx;
     out.pos = bestX;
-    out.r2 = bestR2;
     out.alpha = pow_r(1.0f - bestR2, S.geo[bestIdx].e4b);
     return true;
 }
@@ -236,6 +244,21 @@ __device__ bool traverseCloud(const DevScene& S, const DevInstance& I, F3 o, F3 
 // camera walk into scratch spills; as a call the walk has none, and the
 // walk, photon and adjoint traces run 2-10 % faster).
 __device__ __attribute__((noinline)) float hitAlpha(float oneMinusR2, float e4b) { return pow_r(oneMinusR2, e4b); }
+
+// Squared radius of the point x of a surfel's plane in its support, as the
+// surfel test forms it.
+__device__ __forceinline__ float surfelR2(const SurfelGeo& g, F3 x) {
+    const F3 r = x - mk3(g.px, g.py, g.pz);
+    const float uu = dot(mk3(g.tux, g.tuy, g.tuz), r) / g.su;
+    const float vv = dot(mk3(g.tvx, g.tvy, g.tvz), r) / g.sv;
+    return uu * uu + vv * vv;
+}
+
+// alpha of a surfel at its hit point (object space): a function of the two, so
+// the traversal carries neither alpha nor radius.
+__device__ __forceinline__ float surfelAlpha(const SurfelGeo& g, F3 x) {
+    return hitAlpha(1.0f - surfelR2(g, x), g.e4b);
+}
 
 // Traversal of the cloud without the counters and without a stack round trip
 // for the nearer child: the reference pushes the farther child, then the
@@ -248,7 +271,7 @@ constexpr uint32_t kRefDone = kInvalid;  // the traversal has ended (no leaf ref
 
 struct CloudLane {
     F3 o, d, inv;                    // object-space ray
-    float best, bestR2;              // closest hit so far: distance, squared radius in its support
+    float best;                      // closest hit so far
     uint32_t bestIdx;                // its surfel (kInvalid: none)
     uint32_t ref;                    // node or leaf to visit, kRefDone at the end
     uint32_t sp, base;               // stack height; the height below this traversal
@@ -261,7 +284,6 @@ __device__ __forceinline__ bool cloudBegin(const DevInstance& I, F3 o, F3 d, uin
     c.d = d;
     c.inv = safeInvDir(d);
     c.best = __builtin_huge_valf();
-    c.bestR2 = 0.0f;
     c.bestIdx = kInvalid;
     c.sp = c.base = sp;
     c.ref = I.rootRef;
@@ -280,31 +302,67 @@ __device__ __forceinline__ void cloudPop(const LaneStack& st, CloudLane& c) {
     }
 }
 
-// A node's box against the ray: slab() with clampLo 1e-6, its three
-// rejections as one comparison (max(tmin, 0) > min(tmax, limit) holds exactly
-// when one of them does, also with NaN in tmin, tmax or limit: the limit is
-// positive, and fmin / fmax pass a NaN operand over).
-__device__ __forceinline__ bool nodeSlab(F3 o, F3 inv, float mnx, float mny, float mnz, float mxx, float mxy,
-                                         float mxz, float limit, float& tEntry) {
-    const float t0x = (mnx - o.x) * inv.x, t0y = (mny - o.y) * inv.y, t0z = (mnz - o.z) * inv.z;
-    const float t1x = (mxx - o.x) * inv.x, t1y = (mxy - o.y) * inv.y, t1z = (mxz - o.z) * inv.z;
-    const float tmin = fmaxf(fmaxf(fminf(t0x, t1x), fminf(t0y, t1y)), fminf(t0z, t1z));
-    const float tmax = fminf(fminf(fmaxf(t0x, t1x), fmaxf(t0y, t1y)), fmaxf(t0z, t1z));
-    tEntry = fmaxf(tmin, 1e-6f);
-    return !(fmaxf(tmin, 0.0f) > fminf(tmax, limit));
-}
-
+// One step: the two levels below a node at once.
+//
+// The binary tree's step tests the children's boxes, goes on to the nearer (ties
+// to the left) and later, if it is still in range, to the farther, each of which
+// tests its own children then.  A grandchild's box lies in its parent's, and
+// every operation of the slab test is monotone, also as rounded, so a
+// grandchild that passes implies that its parent passes, with an entry not
+// after its own; and a test passed earlier is only undone by a closer hit, which
+// the stored entry shows at the pop.  Testing the four grandchildren now and
+// keeping them in the order (nearer child's nearer, its farther, farther child's
+// nearer, its farther) therefore visits the same leaves in the same order.  The
+// children's entries, which that order needs, come from the grandchildren's
+// planes (a child's box is their union; k_quad_nodes checks it).
+//
+// slab() with clampLo 1e-6; its three rejections are one comparison: max(tmin,
+// 0) > min(tmax, limit) holds exactly when one of them does, also with NaN in
+// tmin, tmax or limit (the limit is positive, fmin and fmax pass a NaN over).
 __device__ __forceinline__ void cloudNode(const DevScene& S, const LaneStack& st, CloudLane& c) {
-    const float4* nd4 = reinterpret_cast<const float4*>(S.nodes + c.ref);
-    const float4 a = nd4[0], b = nd4[1], e = nd4[2];
-    const uint2 refs = reinterpret_cast<const uint2*>(S.nodes + c.ref)[6];  // left, right (not the padding)
-    float tl, tr;
-    const bool hl = nodeSlab(c.o, c.inv, a.x, a.y, a.z, a.w, b.x, b.y, c.best, tl);
-    const bool hr = nodeSlab(c.o, c.inv, b.z, b.w, e.x, e.y, e.z, e.w, c.best, tr);
-    const bool left = hl && (!hr || tl <= tr);
-    c.ref = left ? refs.x : refs.y;
-    if (hl && hr) st.push(c.sp, left ? refs.y : refs.x, left ? tr : tl);
-    if (!hl && !hr) cloudPop(st, c);
+    const float4* q = reinterpret_cast<const float4*>(S.quads + c.ref);
+    const float4 nx = q[0], xx = q[1], ny = q[2], xy = q[3], nz = q[4], xz = q[5];
+    const uint4 refs = reinterpret_cast<const uint4*>(S.quads + c.ref)[6];
+    const float mn[3][4] = {{nx.x, nx.y, nx.z, nx.w}, {ny.x, ny.y, ny.z, ny.w}, {nz.x, nz.y, nz.z, nz.w}};
+    const float mx[3][4] = {{xx.x, xx.y, xx.z, xx.w}, {xy.x, xy.y, xy.z, xy.w}, {xz.x, xz.y, xz.z, xz.w}};
+    const float o[3] = {c.o.x, c.o.y, c.o.z}, inv[3] = {c.inv.x, c.inv.y, c.inv.z};
+    float lo[3][4], hi[3][4];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float t0 = (mn[a][k] - o[a]) * inv[a], t1 = (mx[a][k] - o[a]) * inv[a];
+            lo[a][k] = fminf(t0, t1);
+            hi[a][k] = fmaxf(t0, t1);
+        }
+    }
+    float t[4];
+    bool h[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const float tmin = fmaxf(fmaxf(lo[0][k], lo[1][k]), lo[2][k]);
+        const float tmax = fminf(fminf(hi[0][k], hi[1][k]), hi[2][k]);
+        t[k] = fmaxf(tmin, 1e-6f);
+        h[k] = !(fmaxf(tmin, 0.0f) > fminf(tmax, c.best));
+    }
+    h[1] = h[1] && refs.y != kInvalid;
+    h[3] = h[3] && refs.w != kInvalid;
+    const float tl = fmaxf(fmaxf(fmaxf(fminf(lo[0][0], lo[0][1]), fminf(lo[1][0], lo[1][1])), fminf(lo[2][0], lo[2][1])), 1e-6f);
+    const float tr = fmaxf(fmaxf(fmaxf(fminf(lo[0][2], lo[0][3]), fminf(lo[1][2], lo[1][3])), fminf(lo[2][2], lo[2][3])), 1e-6f);
+    // Order: within the pairs, then the pairs.
+    const bool sl = !(t[0] <= t[1]), sr = !(t[2] <= t[3]), sp = !(tl <= tr);
+    const uint32_t la = sl ? refs.y : refs.x, lb = sl ? refs.x : refs.y, ra = sr ? refs.w : refs.z, rb = sr ? refs.z : refs.w;
+    const float lta = sl ? t[1] : t[0], ltb = sl ? t[0] : t[1], rta = sr ? t[3] : t[2], rtb = sr ? t[2] : t[3];
+    const bool hla = sl ? h[1] : h[0], hlb = sl ? h[0] : h[1], hra = sr ? h[3] : h[2], hrb = sr ? h[2] : h[3];
+    const uint32_t r0 = sp ? ra : la, r1 = sp ? rb : lb, r2 = sp ? la : ra, r3 = sp ? lb : rb;
+    const float t1 = sp ? rtb : ltb, t2 = sp ? lta : rta, t3 = sp ? ltb : rtb;
+    const bool h0 = sp ? hra : hla, h1 = sp ? hrb : hlb, h2 = sp ? hla : hra, h3 = sp ? hlb : hrb;
+    const bool any1 = h0 || h1, any2 = any1 || h2;
+    if (h3 && any2) st.pushBounded(c.sp, r3, t3);
+    if (h2 && any1) st.pushBounded(c.sp, r2, t2);
+    if (h1 && h0) st.pushBounded(c.sp, r1, t1);
+    c.ref = h0 ? r0 : (h1 ? r1 : (h2 ? r2 : r3));
+    if (!any2 && !h3) cloudPop(st, c);
 }
 
 __device__ __forceinline__ void cloudLeaf(const DevScene& S, const LaneStack& st, CloudLane& c) {
@@ -338,7 +396,6 @@ __device__ __forceinline__ void cloudLeaf(const DevScene& S, const LaneStack& st
         if (r2 >= 1.0f) continue;
         c.best = t;
         c.bestIdx = first + k;
-        c.bestR2 = r2;
     }
     cloudPop(st, c);
 }
@@ -347,18 +404,23 @@ __device__ __forceinline__ void cloudLeaf(const DevScene& S, const LaneStack& st
 // a leaf take one test each on all 64 lanes, four neighbouring lanes (a quad)
 // per leaf.  A step of four tests one after the other costs the wave the same
 // for one lane at a leaf as for 64, and few are there at a time (the walk:
-// 7.5 leaves and 48 nodes per query).  A test of a pair reads its lane's ray
-// through the LDS crossbar; the quad then takes its four results in leaf
-// order against the lane's best, so the outcome is the sequential loop's,
-// ties and NaN included.  Every lane of the wave calls it; returns whether
-// this lane's leaf was tested.
+// 7.5 leaves and 48 nodes per query).  A pair reads its lane's ray through the
+// LDS crossbar; the quad's smallest accepted distance, the first of equal
+// ones, is what the loop in leaf order ends with.  Every lane of the wave
+// calls it; returns whether this lane's leaf was tested.
+//
+// The support test r2 < 1 needs the IEEE divisions of r2 only where it is
+// close: lhs = (a s_v)^2 + (b s_u)^2 and rhs = (s_u s_v)^2 of u = a / s_u, v =
+// b / s_v carry a dozen roundings, under 1e-6 of the value, as does r2, so
+// outside a band of 4e-6 around rhs (and with rhs far from underflow, lhs
+// finite) they decide it.
 __device__ __forceinline__ int laneGet(int v, uint32_t from) { return __builtin_amdgcn_ds_bpermute((int)(from << 2), v); }
 __device__ __forceinline__ float laneGetF(float v, uint32_t from) {
     return __int_as_float(laneGet(__float_as_int(v), from));
 }
-template <int kK>
-__device__ __forceinline__ float quadGet(float v) {  // the value of lane kK of the quad
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), kK * 0x55, 0xf, 0xf, true));
+template <int kCtrl>
+__device__ __forceinline__ float quadGet(float v) {  // of the lane that the quad permutation names
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), kCtrl, 0xf, 0xf, true));
 }
 constexpr uint32_t kLeafLanes = 16;
 
@@ -376,8 +438,8 @@ __device__ __forceinline__ bool cloudLeafRound(const DevScene& S, CloudLane& c, 
     const uint32_t ref = (uint32_t)laneGet((int)c.ref, from);
     const F3 o = mk3(laneGetF(c.o.x, from), laneGetF(c.o.y, from), laneGetF(c.o.z, from));
     const F3 d = mk3(laneGetF(c.d.x, from), laneGetF(c.d.y, from), laneGetF(c.d.z, from));
-    float best = laneGetF(c.best, from);
-    float t = 0.0f, r2 = 0.0f;
+    const float best = laneGetF(c.best, from);
+    float t = 0.0f;
     bool ok = false;
     if (r < n && k < leafCount(ref)) {
         const float4* g = reinterpret_cast<const float4*>(S.geo + (leafFirst(ref) + k));
@@ -387,27 +449,44 @@ __device__ __forceinline__ bool cloudLeafRound(const DevScene& S, CloudLane& c, 
         t = dot(pn, p - o) / nd;
         const F3 x = o + d * t;
         const F3 q = x - p;
-        const float uu = dot(mk3(g2.x, g2.y, g2.z), q) / g0.w;
-        const float vv = dot(mk3(g3.x, g3.y, g3.z), q) / g1.w;
-        r2 = uu * uu + vv * vv;
-        ok = !(fabsf(nd) < 1e-6f) && !(t <= 1e-5f) && !(r2 >= 1.0f);
+        const float a = dot(mk3(g2.x, g2.y, g2.z), q), b = dot(mk3(g3.x, g3.y, g3.z), q);
+        const float as = a * g1.w, bs = b * g0.w, ss = g0.w * g1.w;
+        const float lhs = as * as + bs * bs, rhs = ss * ss;
+        bool inside = lhs < rhs * (1.0f - 4e-6f);
+        if (!(inside || lhs > rhs * (1.0f + 4e-6f)) || !(rhs > 1e-30f) || !(lhs < 1e30f)) {
+            const float uu = a / g0.w, vv = b / g1.w;
+            inside = !(uu * uu + vv * vv >= 1.0f);
+        }
+        ok = inside && !(fabsf(nd) < 1e-6f) && !(t <= 1e-5f) && !(t >= best);
     }
-    const uint32_t oks = (uint32_t)(__builtin_amdgcn_ballot_w64(ok) >> (lane & 60u));
-    uint32_t win = 4u;
-    const float t0 = quadGet<0>(t), t1 = quadGet<1>(t), t2 = quadGet<2>(t), t3 = quadGet<3>(t);
-    if ((oks & 1u) && !(t0 >= best)) { best = t0; win = 0u; }
-    if ((oks & 2u) && !(t1 >= best)) { best = t1; win = 1u; }
-    if ((oks & 4u) && !(t2 >= best)) { best = t2; win = 2u; }
-    if ((oks & 8u) && !(t3 >= best)) { win = 3u; }
-    // The lane's result from its quad.
-    const uint32_t w = (uint32_t)laneGet((int)win, (below << 2) & 63u);
-    const uint32_t src = ((below << 2) + (w & 3u)) & 63u;
-    const float nt = laneGetF(t, src), nr2 = laneGetF(r2, src);
+    unsigned long long wins;
+    float nt;
+    if (__builtin_amdgcn_ballot_w64(ok && !(t < best)) == 0ull) {
+        float q = ok ? t : __builtin_huge_valf();
+        q = fminf(q, quadGet<0xB1>(q));
+        q = fminf(q, quadGet<0x4E>(q));
+        wins = __builtin_amdgcn_ballot_w64(ok && t == q);
+        nt = laneGetF(q, (below << 2) & 63u);
+    } else {
+        // A NaN distance (a degenerate surfel or ray) was accepted: the tests
+        // one after the other, each against the best before it.
+        const unsigned long long oks = __builtin_amdgcn_ballot_w64(ok);
+        const uint32_t mine = (uint32_t)(oks >> (lane & 60u));
+        const float t0 = quadGet<0x00>(t), t1 = quadGet<0x55>(t), t2 = quadGet<0xAA>(t), t3 = quadGet<0xFF>(t);
+        float now = best;
+        uint32_t win = 4u;
+        if ((mine & 1u) && !(t0 >= now)) { now = t0; win = 0u; }
+        if ((mine & 2u) && !(t1 >= now)) { now = t1; win = 1u; }
+        if ((mine & 4u) && !(t2 >= now)) { now = t2; win = 2u; }
+        if ((mine & 8u) && !(t3 >= now)) { now = t3; win = 3u; }
+        wins = __builtin_amdgcn_ballot_w64(win == k);
+        nt = laneGetF(now, (below << 2) & 63u);
+    }
     const bool tested = leaf && below < kLeafLanes;
-    if (tested && w < 4u) {
+    const uint32_t won = (uint32_t)(wins >> ((below << 2) & 63u)) & 15u;
+    if (tested && won) {
         c.best = nt;
-        c.bestIdx = leafFirst(c.ref) + w;
-        c.bestR2 = nr2;
+        c.bestIdx = leafFirst(c.ref) + (uint32_t)__ffs((int)won) - 1u;
     }
     return tested;
 }
@@ -426,8 +505,7 @@ __device__ bool traverseCloudFast(const DevScene& S, const DevInstance& I, F3 o,
     out.t = c.best;
     out.prim = c.bestIdx;
     out.pos = c.o + c.d * c.best;
-    out.r2 = c.bestR2;
-    out.alpha = hitAlpha(1.0f - c.bestR2, S.geo[c.bestIdx].e4b);
+    out.alpha = surfelAlpha(S.geo[c.bestIdx], out.pos);
     return true;
 }
 
@@ -518,7 +596,6 @@ __device__ bool traverseMesh(const DevScene& S, const DevInstance& I, F3 o, F3 d
     out.prim = bestTri;
     out.pos = toWorldPoint(I.o2w, o + d * best);
     out.alpha = 0.0f;
-    out.r2 = 0.0f;
     return true;
 }
 
@@ -622,7 +699,6 @@ __device__ bool intersectSceneTop(const DevScene& S, const Top& top, F3 o, F3 d,
                 h.inst = ii;
                 h.prim = lh.prim;
                 h.alpha = lh.alpha;
-                h.r2 = lh.r2;
             }
         }
     }
@@ -639,21 +715,24 @@ __device__ bool intersectScene(const DevScene& S, F3 o, F3 d, const LaneStack& s
 // the job, takes its next ray and starts again while the others still
 // traverse.
 //
-// What bounds the traversal is its vector instructions: with one query per
-// lane run to the wave's longest, and each iteration stepping the lanes at a
-// leaf and the lanes at a node, the SIMDs issued a vector instruction in
-// 70-80 % of their cycles with 16 % (photon trace), 21 % (adjoint trace), 23 %
-// and 49 % (camera walk, independent and shared samples) of its lanes
-// enabled; 1M clustered surfels, 50 nodes and 7.5 leaves per query.  So a wave
-// takes one kind of step at a time, for the lanes that are at that kind: a
-// leaf round (cloudLeafRound, the cost of one and a half node steps) once
-// kLeafMin lanes wait at a leaf or fewer than kNodeMin are left at nodes, and
-// the ends and starts of queries once 1 / kEndShare of the lanes that were
-// traversing have ended.  Camera walk of 16 passes at 800x800: 41.6 -> 36.9 ms
-// shared, 87.5 -> 56.5 ms independent; photon trace 10.1 -> 6.1 ms, adjoint
-// trace 31.2 -> 23.2 ms independent, 19.3 -> 19.4 ms shared.  kLeafMin 6, 8,
-// 10, 16 (walk, independent): 61.6, 58.7, 57.7, 64.3 ms; kEndShare 1 and 3: 80
-// and 59.3 ms; kNodeMin 1: 57.2 ms.
+// With one query per lane run to the wave's longest, and each iteration
+// stepping the lanes at a leaf and the lanes at a node, the traversals were bound
+// by vector instructions: issued in 70-80 % of a SIMD's cycles, with 16 % (photon
+// trace), 21 % (adjoint trace), 23 % and 49 % (camera walk, independent and
+// shared samples) of their lanes enabled; 1M clustered surfels, 50 nodes of the
+// binary tree and 7.5 leaves per query.  So a wave takes one kind of step at a
+// time, for the lanes that are at that kind: a leaf round (cloudLeafRound, 100
+// vector instructions; a node step has 170) once kLeafMin lanes or 1 /
+// kLeafShare of those that traverse wait at a leaf, and the ends and starts of
+// queries once 1 / kEndShare of the lanes that were traversing have ended.
+// Camera walk of 16 passes at 800x800, shared and independent: 41.6 and 87.5 ms
+// before; 36.9 and 56.5 so; 33.4 and 50.6 with the walk's hits shaded elsewhere
+// and 5 waves per SIMD; 30.6 and 49.0 with quad nodes.  Photon trace 10.1 -> 6.1
+// -> 5.1 ms, adjoint trace 31.2 -> 23.2 -> 19.4 ms (independent).  Of the walk's
+// cycles with waves on a CU, vector instructions now take 90 % and L1 accesses
+// 88 %; a sixth of its time passes after the last pixel is drawn, while the
+// longest pixels end.  kLeafMin 6, 8, 10, 16: 5 % slower to 2 % slower; kEndShare
+// 1 and 3: 40 % and 5 % slower.
 //
 // Job: bool finish(bool done, const JobHit&, const Work&, F3& o, F3& d) takes
 // the hits of the lanes with done set (and the work of their queries in
@@ -665,15 +744,9 @@ __device__ bool intersectScene(const DevScene& S, F3 o, F3 d, const LaneStack& s
 struct JobHit {
     F3 pos;
     uint32_t inst, prim;  // inst kInvalid: miss
-    float r2;             // squared radius in the surfel's support
 };
 
-// alpha of a job's hit on the cloud
-__device__ __forceinline__ float jobAlpha(const DevScene& S, const JobHit& h) {
-    return hitAlpha(1.0f - h.r2, S.geo[h.prim].e4b);
-}
-
-constexpr uint32_t kLeafMin = 12, kNodeMin = 12, kEndShare = 2;
+constexpr uint32_t kLeafMin = 12, kLeafShare = 2, kEndShare = 2;
 
 template <bool kCount, typename Top, typename Job>
 __device__ __forceinline__ void traceWave(const DevScene& S, const Top& top, const LaneStack& st, Job& job) {
@@ -695,7 +768,6 @@ __device__ __forceinline__ void traceWave(const DevScene& S, const Top& top, con
                 h.inst = intersectSceneTop<kCount>(S, top, o, d, st, q, w) ? q.inst : kInvalid;
                 h.prim = q.prim;
                 h.pos = q.pos;
-                h.r2 = q.r2;
             }
         }
     }
@@ -720,7 +792,6 @@ __device__ __forceinline__ void traceWave(const DevScene& S, const Top& top, con
                         h.pos = x;
                         h.inst = inst;
                         h.prim = c.bestIdx;
-                        h.r2 = c.bestR2;
                     }
                 }
                 c.sp = c.base;
@@ -797,7 +868,7 @@ __device__ __forceinline__ void traceWave(const DevScene& S, const Top& top, con
             const uint32_t running = (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(run));
             if (running <= stay) break;
             const uint32_t leaves = (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(leaf));
-            if (leaves > 0u && (leaves >= kLeafMin || running - leaves < kNodeMin)) {
+            if (leaves >= kLeafMin || leaves * kLeafShare >= running) {
                 if (cloudLeafRound(S, c, leaf)) cloudPop(st, c);
             } else {
                 if (run && !leaf) cloudNode(S, st, c);

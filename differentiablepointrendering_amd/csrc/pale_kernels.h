@@ -126,8 +126,8 @@ struct BatchDesc {
 };
 
 // Camera-gather entries of one round, one per layer, in append order: the hit
-// as the walk found it.  qa = hit point + squared radius in the surfel's
-// support (a mesh: its instance, bits), qb = ray direction + primitive (bits),
+// as the walk found it.  qa = hit point + instance (bits), qb = ray direction +
+// primitive (bits),
 // qs = slot, layer of the round (top bit: a mesh).  pos[i] = place of entry i
 // in its slot's layer-ordered list (slot offset + layer); contrib holds at
 // that place each entry's radiance E * k and alpha * opacity, so a slot's
@@ -206,6 +206,9 @@ void launchSeedNext(hipStream_t s, DevState* st, const uint32_t* table, uint32_t
 void launchBeginView(hipStream_t s, DevState* st, uint32_t number);
 void launchEmit(hipStream_t s, const DevScene& S, DevState* st, uint32_t photons, float invEmitted,
                 RayQueue staged, uint8_t* flags);
+// Lanes of the largest photon or adjoint trace launch over `rays` rays, with
+// inLds stack entries per lane in LDS (for the spill area of the others).
+uint32_t queueTraceLanes(const DevScene& S, uint32_t rays, uint32_t inLds);
 void launchPhotonTrace(hipStream_t s, const DevScene& S, DevState* st, uint32_t maxRays, RayQueue in,
                        RayQueue staged, uint8_t* extFlags, PhotonArrays dep, uint8_t* depFlags, TraceParams tp,
                        Reservoir rs, uint32_t* tiles, bool count);
@@ -297,6 +300,9 @@ struct DevPointArrays {
 // Surfel records from device parameter arrays, and their raw copy (16 floats
 // per surfel: p, t_u, t_v, s_u, s_v, albedo, opacity, beta).
 void launchApplyPoints(hipStream_t s, SurfelGeo* geo, SurfelShade* shade, float* raw, DevPointArrays a, uint32_t n);
+
+// Quad nodes first .. first + count - 1 from the wide nodes of the same index.
+void launchQuadNodes(hipStream_t s, const WideNode* nodes, QuadNode* quads, uint32_t first, uint32_t count);
 
 // Device build of the surfel BVH (pale_bvh.hip).  boxes / refBox: 6 floats
 // (min xyz, max xyz) per surfel / per reference node; acc: 6 order-

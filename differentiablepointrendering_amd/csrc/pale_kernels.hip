@@ -297,7 +297,7 @@ struct PhotonJob {
             } else {
                 const float u = rng.nextFloat();
                 const SurfelShade sh = S.shade[h.prim];
-                const float hAlpha = jobAlpha(S, h);
+                const float hAlpha = surfelAlpha(S.geo[h.prim], h.pos);
                 if (u < tp.qNull) {
                     const float att = 1.0f - hAlpha * sh.opacity;
                     const float wn = att / tp.qNull;
@@ -934,7 +934,7 @@ struct CameraJob {
             } else {
                 if (kCount) addWork(w, wl);
                 if (want) {
-                    ent.qa[e] = f4(h.pos, mesh ? u2f(h.inst) : h.r2);
+                    ent.qa[e] = f4(h.pos, u2f(h.inst));
                     ent.qb[e] = f4(d, u2f(h.prim));
                     ent.qs[e] = make_uint2(pixel, r | (mesh ? kEntryMesh : 0u));
                     ++r;
@@ -1102,7 +1102,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
         F3 nrm, k;
         float ae = 1.0f;
         if (ent.qs[e].y & kEntryMesh) {
-            const JobHit h{ld3(a), f2u(a.w), prim, 0.0f};
+            const JobHit h{ld3(a), f2u(a.w), prim};
             nrm = hitNormal(S, h);
             const DevMaterial m = S.mats[S.inst[h.inst].material];
             k = mk3(m.r, m.g, m.b) * kInvPi;
@@ -1111,7 +1111,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
             nrm = mk3(sh.nsx, sh.nsy, sh.nsz);
             if (dot(nrm, -ld3(b)) < 0.0f) nrm = -nrm;
             k = (sh.alpha_r * mk3(sh.ar, sh.ag, sh.ab)) * kInvPi;
-            ae = sh.opacity * hitAlpha(1.0f - a.w, S.geo[prim].e4b);
+            ae = sh.opacity * surfelAlpha(S.geo[prim], ld3(a));
         }
         const F3 E = gatherIrradiance<kCount, true>(G, ld3(a), nrm, w);
         ent.contrib[pos] = f4(E * k, ae);
@@ -1365,7 +1365,7 @@ struct AdjointJob {
         if (h.inst != kInvalid) {
             const DevInstance& I = S.inst[h.inst];
             const bool cloud = I.type == kGeoCloud;
-            const float hAlpha = cloud ? jobAlpha(S, h) : 0.0f;
+            const float hAlpha = cloud ? surfelAlpha(S.geo[h.prim], h.pos) : 0.0f;
             F3 on, ng = mk3(0, 0, 0), dir;
             float pdf;
             SurfelShade sh{};
@@ -1816,6 +1816,57 @@ __global__ __launch_bounds__(256) void k_gather_points(DevGrid G, uint32_t n, co
     out[3 * i + 2] = E.z;
 }
 
+// A node's quad node.  The children's own boxes are not stored: the traversal
+// takes their entries from the union of their children's, so a node is written
+// two levels deep only where those unions are the children's boxes (always,
+// unless a box has NaN or no extent); otherwise its two children take a slot
+// each.
+__global__ __launch_bounds__(256) void k_quad_nodes(const WideNode* nodes, QuadNode* quads, uint32_t first, uint32_t n) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const WideNode w = nodes[first + i];
+    struct Box {
+        float b[6];  // min xyz, max xyz
+    };
+    const Box child[2] = {{{w.lminx, w.lminy, w.lminz, w.lmaxx, w.lmaxy, w.lmaxz}},
+                          {{w.rminx, w.rminy, w.rminz, w.rmaxx, w.rmaxy, w.rmaxz}}};
+    const uint32_t ref[2] = {w.left, w.right};
+    Box box[4];
+    uint32_t refs[4];
+    bool whole = true;
+    for (int c = 0; c < 2; ++c) {
+        box[2 * c] = box[2 * c + 1] = child[c];
+        refs[2 * c] = ref[c];
+        refs[2 * c + 1] = kInvalid;
+        if (ref[c] & kLeafBit) continue;
+        const WideNode g = nodes[ref[c]];
+        const Box l = {{g.lminx, g.lminy, g.lminz, g.lmaxx, g.lmaxy, g.lmaxz}};
+        const Box r = {{g.rminx, g.rminy, g.rminz, g.rmaxx, g.rmaxy, g.rmaxz}};
+        for (int a = 0; a < 6; ++a) {
+            const float u = a < 3 ? fminf(l.b[a], r.b[a]) : fmaxf(l.b[a], r.b[a]);
+            whole = whole && u == child[c].b[a] && l.b[a] == l.b[a] && r.b[a] == r.b[a];
+            if (a < 3) whole = whole && l.b[a] <= l.b[a + 3] && r.b[a] <= r.b[a + 3];
+        }
+        box[2 * c] = l;
+        box[2 * c + 1] = r;
+        refs[2 * c] = g.left;
+        refs[2 * c + 1] = g.right;
+    }
+    QuadNode q;
+    for (int k = 0; k < 4; ++k) {
+        const Box& b = whole ? box[k] : child[k >> 1];
+        q.mnx[k] = b.b[0];
+        q.mny[k] = b.b[1];
+        q.mnz[k] = b.b[2];
+        q.mxx[k] = b.b[3];
+        q.mxy[k] = b.b[4];
+        q.mxz[k] = b.b[5];
+        q.ref[k] = whole ? refs[k] : ((k & 1) ? kInvalid : ref[k >> 1]);
+        q.pad[k] = 0u;
+    }
+    quads[first + i] = q;
+}
+
 // ------------------------------------------------------------ launchers --
 static inline uint32_t blocks(uint32_t n, uint32_t b) { return (n + b - 1) / b; }
 // Grid of the light per-item kernels (keys and scatters of the entry and
@@ -1865,6 +1916,21 @@ static uint32_t traceGrid(const void* kernel, size_t lds) {
 template <bool kCount, typename Map, bool kTopLds>
 static uint32_t camTraceGrid(size_t lds) {
     return traceGrid(reinterpret_cast<const void*>(&k_cam_trace<kCount, Map, kTopLds>), lds);
+}
+
+uint32_t queueTraceLanes(const DevScene& S, uint32_t rays, uint32_t inLds) {
+    const size_t lds = (size_t)min(S.stackDepth, inLds) * sizeof(uint2) * kTraceBlock;
+    uint32_t grid = 0;
+    const auto add = [&](auto k) { grid = std::max(grid, traceGrid(reinterpret_cast<const void*>(k), lds)); };
+    add(&k_photon_trace<false, false>);
+    add(&k_photon_trace<false, true>);
+    add(&k_photon_trace<true, false>);
+    add(&k_photon_trace<true, true>);
+    add(&k_adj_trace<false, false>);
+    add(&k_adj_trace<false, true>);
+    add(&k_adj_trace<true, false>);
+    add(&k_adj_trace<true, true>);
+    return min(grid, blocks(rays, kTraceBlock)) * kTraceBlock;
 }
 
 void launchPhotonTrace(hipStream_t s, const DevScene& S, DevState* st, uint32_t maxRays, RayQueue in,
@@ -2126,6 +2192,10 @@ void launchTraceRays(hipStream_t s, const DevScene& S, uint32_t n, const float* 
 
 void launchGatherPoints(hipStream_t s, const DevGrid& G, uint32_t n, const float* q, const float* nrm, float* out) {
     if (n) k_gather_points<<<blocks(n, 256), 256, 0, s>>>(G, n, q, nrm, out);
+}
+
+void launchQuadNodes(hipStream_t s, const WideNode* nodes, QuadNode* quads, uint32_t first, uint32_t count) {
+    if (count) k_quad_nodes<<<blocks(count, 256), 256, 0, s>>>(nodes, quads, first, count);
 }
 
 void launchSetOpacity(hipStream_t s, SurfelShade* shade, const float* opacity, uint32_t n) {

@@ -308,7 +308,7 @@ struct pale_handle {
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
 
-    DevMem geo, shade, nodes, tris, inst, tlas, mats, lights, emTris;
+    DevMem geo, shade, nodes, quads, tris, inst, tlas, mats, lights, emTris;
     DevScene scene{};
 
     // Photon map (persistent between forward and backward passes, as the
@@ -333,13 +333,13 @@ struct pale_handle {
     uint32_t walkLds() const { return tune.walk_lds_entries ? tune.walk_lds_entries : kWalkLdsEntries; }
     // The photon and adjoint traces keep kTraceLdsEntries stack entries per
     // lane in LDS and the rest in traceSpill: 16 KB of LDS per workgroup
-    // instead of the whole stack's (23 KB at 1M surfels), so that LDS allows
+    // instead of the whole stack's (31 KB at 1M surfels), so that LDS allows
     // the 4 waves per SIMD their registers allow.
     static constexpr uint32_t kTraceLdsEntries = 16;
     DevMem traceSpill;
     size_t traceSpillBytes(uint32_t rays) const {
         if (img.stackDepth <= kTraceLdsEntries || !rays) return 0;
-        const size_t lanes = (size_t)((rays + kTraceBlock - 1) / kTraceBlock) * kTraceBlock;
+        const size_t lanes = queueTraceLanes(scene, rays, kTraceLdsEntries);
         return (size_t)(img.stackDepth - kTraceLdsEntries) * lanes * sizeof(uint2);
     }
     // t with the split stack when the spill area (sized with the queues)
@@ -554,6 +554,9 @@ struct pale_handle {
         scene.geo = geo.as<SurfelGeo>();
         scene.shade = shade.as<SurfelShade>();
         scene.nodes = nodes.as<WideNode>();
+        quads.reserve((size_t)img.wideCount * sizeof(QuadNode));
+        launchQuadNodes(stream, nodes.as<WideNode>(), quads.as<QuadNode>(), img.meshWide, img.wideCount - img.meshWide);
+        scene.quads = quads.as<QuadNode>();
         scene.tris = tris.as<TriGeo>();
         scene.inst = inst.as<DevInstance>();
         scene.tlas = tlas.as<TlasNode>();

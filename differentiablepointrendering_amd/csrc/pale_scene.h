@@ -198,7 +198,8 @@ struct DeviceImage {
     std::vector<DevMaterial> materials;
     std::vector<DevLight> lights;
     std::vector<DevEmTri> emTris;
-    uint32_t stackDepth = 0;  // LDS stack entries one lane needs
+    uint32_t stackDepth = 0;  // stack entries one lane needs
+    uint32_t wideCount = 0;   // wide nodes of all trees, the cloud's from meshWide on
     // With BuildProducts::cloudOnDevice: surfGeo / surfShade are sized but
     // not filled, and only nodes[0, meshWide) (the meshes' wide nodes) are;
     // the device holds the rest.

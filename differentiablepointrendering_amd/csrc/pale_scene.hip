@@ -629,6 +629,7 @@ void makeDeviceImage(const BuildProducts& bp, const std::vector<HostMesh>& meshe
     for (uint32_t i = 0; i < cloudRange.count; ++i)
         if (compact[cloudRange.first + i] != kInvalid) meshWide = std::min(meshWide, compact[cloudRange.first + i]);
     img.meshWide = meshWide;
+    img.wideCount = next;
     img.nodes.resize(bp.cloudOnDevice ? meshWide : next);
     auto refOf = [&](const Range& r, uint32_t local) -> uint32_t {
         const RefNode& n = bp.blas[r.first + local];
@@ -682,8 +683,9 @@ void makeDeviceImage(const BuildProducts& bp, const std::vector<HostMesh>& meshe
     }
     for (const HostEmTri& e : bp.emTris) img.emTris.push_back(DevEmTri{e.tri, e.cdf});
     // Near-far depth-first traversal keeps at most one pending sibling per
-    // level: depth + 1 entries per BLAS, tlasDepth + 1 below it.
-    img.stackDepth = (bp.tlasMaxDepth + 1) + (bp.blasMaxDepth + 1);
+    // level, or three per two levels of quad nodes; tlasDepth + 1 entries below
+    // a BLAS's.
+    img.stackDepth = (bp.tlasMaxDepth + 1) + std::max(bp.blasMaxDepth + 1, 3 * ((bp.blasMaxDepth + 1) / 2));
 }
 
 }  // namespace pale

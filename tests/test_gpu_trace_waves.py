@@ -137,3 +137,28 @@ def test_gather_rows_against_all_photons(radius, offset):
     n = rng.normal(size=q.shape)
     n = (n / np.linalg.norm(n, axis=1, keepdims=True)).astype(np.float32)
     assert np.array_equal(gpu.gather_irradiance(q, n), orc.gather(q, n))
+
+
+@pytest.mark.parametrize("n", [6, 9, 17, 33, 37, 70, 515, 4099, 70_001])
+def test_quad_nodes_over_tree_shapes(n):
+    """Trees whose levels pair up in every way (odd and even depths, leaves
+    beside subtrees) and both builds: closest hits, ties by leaf order, and the
+    photon map through the two-level steps equal the oracle's binary walk."""
+    pts = scene.uniform_surfels(n, seed=n, scale_lo=0.02 if n > 4000 else 0.1, scale_hi=0.05 if n > 4000 else 0.3)[0]
+    # coincident surfels: exact ties in distance go to the leaf visited first
+    for k in pts:
+        pts[k][1::5] = pts[k][0::5][:len(pts[k][1::5])]
+    spec = scene.SceneSpec([scene.light_quad()], [scene.default_camera(32, 24)], pts,
+                           dict(photons=3000, bounces=3, forward_passes=1, gather_passes=2, adjoint_bounces=3,
+                                adjoint_passes=1, gather_radius=0.1, spp_decorrelate=1))
+    gpu, orc = _pair(spec, {})
+    rng = np.random.default_rng(3)
+    o = rng.uniform(-1.2, 1.2, size=(4000, 3)).astype(np.float32)
+    d = rng.normal(size=(4000, 3)).astype(np.float32)
+    d[::7, 0] = 0.0  # axis-parallel rays
+    d[::11, 1:] = 0.0
+    d = (d / np.maximum(np.linalg.norm(d, axis=1, keepdims=True), 1e-6)).astype(np.float32)
+    a, b = gpu.trace_rays(o, d), orc.trace(o, d)
+    for k in ("instance", "primitive", "t", "position"):
+        assert np.array_equal(a[k], b[k]), k
+    _check(gpu, orc)

@@ -21,7 +21,7 @@ constexpr uint32_t kTraceRegions = 8;
 struct DevState {
     uint32_t cursor;       // next entry of the seed table
     uint32_t number;       // seed of the current launch
-    uint32_t live;         // current bounce runs (queue not empty)
+    uint32_t ticket;       // next tile of the running compaction
     uint32_t qCount;       // rays in the current queue
     uint32_t photonCount;  // photon deposits so far (attempted = stored)
     uint32_t extTotal;     // survivors of the last bounce
@@ -48,6 +48,18 @@ struct RayQueue {
     float4* o;
     float4* d;
     float4* T;
+};
+
+// Closest hits of a queue's rays: point + instance (bits, kInvalid: a miss),
+// primitive.
+struct HitArrays {
+    float4* pos;
+    uint32_t* prim;
+};
+
+// One word per tile of kTile items of a compaction (cleared before it).
+struct TileStates {
+    unsigned long long* state;
 };
 
 // Photon deposits: position + power.x, direction + power.y, power.z.
@@ -202,32 +214,28 @@ struct GridParams {
 void launchFill(hipStream_t s, uint32_t* p, uint32_t n, uint32_t v);
 void launchFillF(hipStream_t s, float* p, uint32_t n, float v);
 void launchIota(hipStream_t s, uint32_t* p, uint32_t n);  // p[i] = i
-void launchSeedNext(hipStream_t s, DevState* st, const uint32_t* table, uint32_t tableLen, int bounce);
+// Between the launches of the photon stage (k_photon_next): bounce >= 0,
+// kNextDraw or kNextEnd; rays: most items of the next compaction; resvCap: the
+// photon capacity if the map can fill, else 0.
+constexpr int kNextDraw = -1, kNextEnd = -2;
+void launchPhotonNext(hipStream_t s, DevState* st, const uint32_t* table, uint32_t tableLen, int bounce,
+                      uint32_t resvCap, TileStates ts, uint32_t rays);
 void launchBeginView(hipStream_t s, DevState* st, uint32_t number);
-void launchEmit(hipStream_t s, const DevScene& S, DevState* st, uint32_t photons, float invEmitted,
-                RayQueue staged, uint8_t* flags);
+void launchEmit(hipStream_t s, const DevScene& S, DevState* st, uint32_t photons, float invEmitted, RayQueue out,
+                uint32_t outCap, TileStates ts);
 // Lanes of the largest photon or adjoint trace launch over `rays` rays, with
 // inLds stack entries per lane in LDS (for the spill area of the others).
 uint32_t queueTraceLanes(const DevScene& S, uint32_t rays, uint32_t inLds);
-void launchPhotonTrace(hipStream_t s, const DevScene& S, DevState* st, uint32_t maxRays, RayQueue in,
-                       RayQueue staged, uint8_t* extFlags, PhotonArrays dep, uint8_t* depFlags, TraceParams tp,
-                       Reservoir rs, uint32_t* tiles, bool count);
-// After the bounce's deposits are compacted: deposits past capacity that the
-// reservoir accepted overwrite their slots, the highest attempt winning.
-void launchReservoirWrite(hipStream_t s, DevState* st, uint32_t maxRays, Reservoir rs, PhotonArrays dep,
-                          PhotonArrays raw);
-// Stable compaction of flagged items i < *count (items >= *count are ignored).
-void launchCompactRays(hipStream_t s, const uint8_t* flags, const uint32_t* count, uint32_t maxItems,
-                       uint32_t* tiles, uint32_t* total, RayQueue src, RayQueue dst, uint32_t dstCap);
-void launchCompactPhotons(hipStream_t s, const uint8_t* flags, const uint32_t* count, uint32_t maxItems,
-                          uint32_t* tiles, uint32_t* total, const uint32_t* base, PhotonArrays src,
-                          PhotonArrays dst, uint32_t dstCap);
-// Stable compaction of one bounce's events, appended to the event pool
-// (DevState::evPool items; this bounce's count goes to DevState::evTotal).
-void launchCompactEvents(hipStream_t s, const uint8_t* flags, const uint32_t* count, uint32_t maxItems,
-                         uint32_t* tiles, DevState* st, EventArrays src, EventArrays pool, uint32_t poolCap);
-void launchFinishPhotonBounce(hipStream_t s, DevState* st, uint32_t cap);
-void launchSetQueue(hipStream_t s, DevState* st, const uint32_t* src);
+// Closest hits of the queue's rays (at most maxRays).
+void launchQueueTrace(hipStream_t s, const DevScene& S, DevState* st, uint32_t maxRays, RayQueue in, HitArrays hits,
+                      TraceParams tp, bool adjoint, bool count);
+// Deposits of a bounce into the map (rs.cap photons) and its survivors into
+// out.  Where the map can fill (rs.attempt), deposits past capacity that the
+// reservoir accepts overwrite their slots, the highest attempt winning (staged,
+// depFlags and tiles are used only then).
+void launchPhotonShade(hipStream_t s, const DevScene& S, DevState* st, uint32_t maxRays, RayQueue in, HitArrays hits,
+                       RayQueue out, uint32_t outCap, PhotonArrays map, PhotonArrays staged, TraceParams tp,
+                       Reservoir rs, uint8_t* depFlags, uint32_t* tiles, TileStates ts);
 // Photon grid (counting sort by cell, stable in deposit order); the sorted
 // powers are divided by the area of the gather's disc.
 void launchBuildGrid(hipStream_t s, const GridParams& g, DevState* st, uint32_t photonCap, PhotonArrays raw,
@@ -265,16 +273,21 @@ void launchCamCompositeBatch(hipStream_t s, uint32_t maxSlots, const BatchHeader
 void launchBatchResolve(hipStream_t s, BatchDesc b, uint32_t maxResolve, PixelArrays px, float4* fb);
 void launchPostprocess(hipStream_t s, const float4* fb, float4* ldr, uint32_t n);
 // Batched adjoint: primary rays of every slot of the batch (queue index =
-// slot, T.w = segment); first queue index of every segment present.
+// slot, T.w = segment) and the first queue index of every segment.
 void launchAdjRaygenBatch(hipStream_t s, BatchDesc b, uint32_t maxTiles, const float* dloss, RayQueue q,
-                          PendingArrays pend, DevState* st);
-void launchSegFirst(hipStream_t s, const DevState* st, uint32_t maxRays, RayQueue q, uint32_t* segFirst,
-                    uint32_t* segEnd, uint32_t nSegs, uint4* groups, uint32_t nGroups, const uint32_t* groupSegs);
+                          PendingArrays pend, DevState* st, uint32_t* segFirst);
 void launchAdjRaygen(hipStream_t s, const DevCamera& cam, const float* dloss, RayQueue q, PendingArrays pend,
                      DevState* st, uint32_t seed);
-void launchAdjTrace(hipStream_t s, const DevScene& S, DevState* st, uint32_t maxRays, uint32_t bounce, RayQueue in,
-                    RayQueue staged, uint8_t* extFlags, EventArrays ev, uint8_t* evFlags, PendingArrays pend,
-                    TraceParams tp, bool count);
+// Before every bounce of the adjoint (bounce 0: the queue is raygen's) and
+// after the last (kNextEnd), see k_adj_next; nSegs 0: no batch.
+void launchAdjNext(hipStream_t s, DevState* st, int bounce, uint32_t poolCap, TileStates ts, uint32_t rays,
+                   uint32_t* segFirst, uint32_t* segEnd, uint32_t* segNext, uint32_t nSegs, uint4* groups,
+                   uint32_t nGroups, const uint32_t* groupSegs);
+// A bounce's events, appended to the event pool (DevState::evPool items; the
+// bounce's count goes to DevState::evTotal), and its survivors into out.
+void launchAdjShade(hipStream_t s, const DevScene& S, DevState* st, uint32_t maxRays, uint32_t bounce, RayQueue in,
+                    HitArrays hits, RayQueue out, uint32_t outCap, EventArrays pool, uint32_t poolCap,
+                    PendingArrays pend, TraceParams tp, uint32_t* segNext, TileStates ts);
 // Transport of the pooled events (in cell order after launchEventSort).
 void launchEventSort(hipStream_t s, const GridParams& g, DevState* st, uint32_t poolCap, EventArrays ev,
                      uint32_t* cell, uint32_t* sorted, uint32_t* cellCount, uint32_t* cellStart, uint32_t* tiles,

@@ -119,20 +119,99 @@ __global__ void k_iota(uint32_t* p, uint32_t n) {
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = i;
 }
 
-// Seed schedule of submitPhotonMappingKernel (SyclBridge.cpp:83-143): one
-// draw per emitter launch, per executed bounce and per camera.  `bounce` < 0
-// always draws; a bounce draws only if its queue is not empty.
-__global__ void k_seed_next(DevState* st, const uint32_t* table, uint32_t len, int bounce) {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
+// Between the launches of the photon stage.  Seed schedule of
+// submitPhotonMappingKernel (SyclBridge.cpp:83-143): one draw per emitter
+// launch, per executed bounce and per camera.  bounce kNextDraw always draws
+// (an emitter launch, a camera); a bounce takes over the queue that the launch
+// before it wrote and draws only if it is not empty; kNextEnd only adds the
+// last bounce's deposits (photonCount counts deposit attempts, the reference's
+// counter T; only the first `cap` are stored).  The next bounce may pass a
+// reservoir's capacity if the deposits so far plus one per queued photon do.
+// The tile states of the next compaction are cleared.
+__global__ __launch_bounds__(256) void k_photon_next(DevState* st, const uint32_t* table, uint32_t len, int bounce,
+                                                     uint32_t resvCap, TileStates ts, uint32_t tiles) {
+    for (uint32_t k = threadIdx.x; k < tiles; k += blockDim.x) ts.state[k] = 0ull;
+    if (threadIdx.x != 0) return;
+    const uint32_t deposits = st->photonCount + st->depTotal;
+    st->photonCount = deposits;
+    st->depTotal = 0;
     st->traceNext = 0;
-    if (bounce >= 0 && st->qCount == 0) {
-        st->live = 0;
-        return;
+    st->ticket = 0;
+    if (bounce == kNextEnd) return;
+    if (bounce >= 0) {
+        const uint32_t q = st->extTotal;
+        st->qCount = q;
+        st->resv = (resvCap && q && (uint64_t)deposits + (uint64_t)q > (uint64_t)resvCap) ? 1u : 0u;
+        if (q == 0) return;
     }
     const uint32_t c = st->cursor;
     st->number = c < len ? table[c] : 0u;
     st->cursor = c + 1;
-    st->live = 1;
+}
+
+// Between the bounces of the adjoint: the queue and the events that the bounce
+// before wrote are taken over, the tile states cleared.  In a batch (nSegs > 0)
+// also where each segment's rays start and end in the queue (it stays in
+// segment order: raygen writes it so, compaction is stable; segFirst has the
+// first of every segment present, kInvalid for the others, whose first and end
+// become 0), the places of the views' groups for the trace's interleaved order
+// (K segments x the most rays of one), and segNext cleared for the bounce.
+__global__ __launch_bounds__(256) void k_adj_next(DevState* st, int bounce, uint32_t poolCap, TileStates ts,
+                                                  uint32_t tiles, uint32_t* segFirst, uint32_t* segEnd,
+                                                  uint32_t* segNext, uint32_t nSegs, uint4* groups, uint32_t nGroups,
+                                                  const uint32_t* groupSegs) {
+    for (uint32_t k = threadIdx.x; k < tiles; k += blockDim.x) ts.state[k] = 0ull;
+    __shared__ uint32_t sQueue;
+    if (threadIdx.x == 0) {
+        const uint32_t n = st->evPool + st->evTotal;
+        st->evPool = n < poolCap ? n : poolCap;
+        st->evTotal = 0;
+        st->traceNext = 0;
+        st->ticket = 0;
+        if (bounce > 0) st->qCount = st->extTotal;
+        sQueue = st->qCount;
+    }
+    if (!nSegs || bounce == kNextEnd) return;
+    __syncthreads();
+    if (threadIdx.x < 64u) {
+        uint32_t after = sQueue;  // where the segment after this chunk starts
+        for (uint32_t base = (nSegs - 1u) & ~63u;; base -= 64u) {
+            const uint32_t s = base + threadIdx.x;
+            const uint32_t first = s < nSegs ? segFirst[s] : kInvalid;
+            uint32_t m = first;  // the smallest first of this and later segments (they ascend)
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const uint32_t v = __shfl_down(m, o, 64);
+                if (threadIdx.x + (uint32_t)o < 64u) m = min(m, v);
+            }
+            const uint32_t next = __shfl_down(m, 1, 64);
+            const uint32_t end = min(threadIdx.x < 63u ? next : kInvalid, after);
+            if (s < nSegs) {
+                segFirst[s] = first == kInvalid ? 0u : first;
+                segEnd[s] = first == kInvalid ? 0u : end;
+            }
+            after = min(after, (uint32_t)__shfl(m, 0, 64));
+            if (base == 0u) break;
+        }
+    }
+    __syncthreads();
+    for (uint32_t s = threadIdx.x; s < nSegs; s += blockDim.x) segNext[s] = kInvalid;
+    for (uint32_t g = threadIdx.x; g < nGroups; g += blockDim.x) {
+        const uint4 gr = groups[g];
+        uint32_t most = 0;
+        for (uint32_t k = 0; k < gr.y; ++k) {
+            const uint32_t s = groupSegs[gr.x + k];
+            most = max(most, segEnd[s] - segFirst[s]);
+        }
+        groups[g].w = most;
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    uint32_t place = 0;
+    for (uint32_t g = 0; g < nGroups; ++g) {
+        groups[g].z = place;
+        place += groups[g].y * groups[g].w;
+    }
 }
 
 // Start of a served view: its passes draw from `number` (+ pass); the
@@ -149,31 +228,90 @@ __global__ void k_begin_view(DevState* st, uint32_t number) {
     }
 }
 
-// photonCount counts deposit attempts (the reference's counter T); only the
-// first `cap` are stored.
-__global__ void k_finish_photon_bounce(DevState* st, uint32_t cap) {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    (void)cap;
-    if (st->live) {
-        st->qCount = st->extTotal;
-        st->photonCount += st->depTotal;
-    } else {
-        st->qCount = 0;
-    }
+// ------------------------------------------------------- compaction --
+// Offsets of a launch's items in the compacted outputs, in one pass: the
+// workgroups take tiles of kTile items in ticket order, publish their tile's
+// counts, add up those of the tiles before until one has published its prefix,
+// and publish their own (decoupled look-back, Merrill and Garland 2016).  A
+// tile's ticket is drawn by a running workgroup, and a workgroup waits only for
+// earlier tickets after it has published its own counts, so every wait ends.
+// The writers of the outputs then go on with them in registers: with staged
+// outputs, flags, a count, a scan and a scatter launch per output a bounce took
+// 9 launches (adjoint: 12) instead of 3 and moved every ray, deposit and event
+// twice more.  Per bounce at 640,000 rays those took about 260 us of an adjoint
+// bounce; k_adj_shade takes 126 us with the shading in it.
+//
+// A tile's state is one word, so that its parts are seen together: 2 bits of
+// what it holds, 31 bits for each of two counts.
+__device__ __forceinline__ uint32_t tileTicket(DevState* st) {
+    __shared__ uint32_t t;
+    if (threadIdx.x == 0) t = atomicAdd(&st->ticket, 1u);
+    __syncthreads();
+    return t;
 }
+constexpr uint64_t kTileCounts = 1ull << 62, kTilePrefix = 2ull << 62, kTileValue = (1ull << 62) - 1ull;
 
-// Events of one bounce were appended to the pool.
-__global__ void k_event_pool_add(DevState* st, uint32_t cap) {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    const uint32_t n = st->evPool + st->evTotal;
-    st->evPool = n < cap ? n : cap;
-}
-
-__global__ void k_set_queue(DevState* st, const uint32_t* src) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        st->qCount = *src;
-        st->traceNext = 0;
+struct TileOffset {
+    uint32_t a, b;        // this thread's places
+    uint32_t endA, endB;  // the counts up to and with this tile
+};
+// Every thread of the workgroup calls it.
+__device__ __forceinline__ TileOffset tileOffsets(TileStates ts, uint32_t tile, bool a, bool b) {
+    __shared__ uint32_t waveA[kTile / 64], waveB[kTile / 64];
+    __shared__ uint64_t sBase, sSum;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const unsigned long long ma = __ballot(a), mb = __ballot(b);
+    if (lane == 0) {
+        waveA[wave] = (uint32_t)__popcll(ma);
+        waveB[wave] = (uint32_t)__popcll(mb);
     }
+    __syncthreads();
+    if (wave == 0) {
+        uint64_t v = lane < kTile / 64 ? ((uint64_t)waveA[lane] << 31) | waveB[lane] : 0ull;
+        const uint64_t own = v;
+#pragma unroll
+        for (int o = 1; o < (int)(kTile / 64); o <<= 1) {
+            const uint64_t y = __shfl_up(v, o, 64);
+            if (lane >= (uint32_t)o) v += y;
+        }
+        const uint64_t sum = __shfl(v, kTile / 64 - 1, 64);
+        if (lane < kTile / 64) {
+            waveA[lane] = (uint32_t)((v - own) >> 31);
+            waveB[lane] = (uint32_t)((v - own) & 0x7FFFFFFFull);
+        }
+        uint64_t before = 0;
+        if (tile > 0u) {
+            if (lane == 0) __hip_atomic_store(ts.state + tile, kTileCounts | sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            int64_t at = (int64_t)tile - 1;
+            while (true) {
+                const int64_t t = at - (int64_t)lane;
+                const uint64_t w = t >= 0 ? __hip_atomic_load(ts.state + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : kTilePrefix;
+                const unsigned long long prefix = __ballot((w & kTilePrefix) != 0ull), none = __ballot((w >> 62) == 0ull);
+                const uint32_t p = prefix ? (uint32_t)__ffsll((long long)prefix) - 1u : 64u;
+                if (none && (uint32_t)__ffsll((long long)none) - 1u < p) {
+                    __builtin_amdgcn_s_sleep(2);
+                    continue;
+                }
+                uint64_t c = lane <= p ? (w & kTileValue) : 0ull;
+#pragma unroll
+                for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
+                before += c;
+                if (p < 64u) break;
+                at -= 64;
+            }
+        }
+        if (lane == 0) {
+            __hip_atomic_store(ts.state + tile, kTilePrefix | (before + sum), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            sBase = before;
+            sSum = sum;
+        }
+    }
+    __syncthreads();
+    const uint64_t base = sBase, end = sBase + sSum;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    return TileOffset{(uint32_t)(base >> 31) + waveA[wave] + (uint32_t)__popcll(ma & below),
+                      (uint32_t)(base & 0x7FFFFFFFull) + waveB[wave] + (uint32_t)__popcll(mb & below),
+                      (uint32_t)(end >> 31), (uint32_t)(end & 0x7FFFFFFFull)};
 }
 
 // ------------------------------------------------------- queue traces --
@@ -214,42 +352,73 @@ struct QueueCursor {
 
 // ---------------------------------------------------------- emission --
 // launchRayGenEmitterKernel (PrimalKernels.cpp:13-62)
-__global__ __launch_bounds__(256) void k_emit(DevScene S, const DevState* st, uint32_t P, float invEmitted,
-                                              RayQueue out, uint8_t* flags) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= P) return;
-    Rng rng(perItemSeed(st->number, i));
+__global__ __launch_bounds__(kTile) void k_emit(DevScene S, DevState* st, uint32_t P, float invEmitted, RayQueue out,
+                                                uint32_t outCap, TileStates ts) {
+    const uint32_t tile = tileTicket(st);
+    if (tile * kTile >= P) {
+        if (P == 0u) st->extTotal = 0u;
+        return;
+    }
+    const uint32_t i = tile * kTile + threadIdx.x;
     F3 pos, dir, power;
-    const bool ok = sampleLight(S, rng, pos, dir, power);
-    flags[i] = ok ? 1 : 0;
-    if (!ok) return;
-    const F3 T = (power * (float)S.nLights) * invEmitted;
-    out.o[i] = f4(pos, u2f(kInvalid));
-    out.d[i] = f4(dir, u2f(0u));
-    out.T[i] = f4(T, 0.0f);
+    bool ok = false;
+    if (i < P) {
+        Rng rng(perItemSeed(st->number, i));
+        ok = sampleLight(S, rng, pos, dir, power);
+    }
+    const TileOffset at = tileOffsets(ts, tile, ok, false);
+    if (ok && at.a < outCap) {
+        const F3 T = (power * (float)S.nLights) * invEmitted;
+        out.o[at.a] = f4(pos, u2f(kInvalid));
+        out.d[at.a] = f4(dir, u2f(0u));
+        out.T[at.a] = f4(T, 0.0f);
+    }
+    if (threadIdx.x == 0 && tile == (P - 1u) / kTile) st->extTotal = min(at.endA, outCap);
 }
 
 // ---------------------------------------------------- photon bounce --
-// launchIntersectKernel (PrimalKernels.cpp:65-321) for one queue: the hit of
-// ray i, its deposit and the ray that goes on.
-template <bool kCount>
-struct PhotonJob {
+// Closest hits of a queue's rays, on a persistent grid.
+struct QueueHits {
+    float4* pos;     // hit point, instance (bits; kInvalid: miss)
+    uint32_t* prim;  // primitive
+    __device__ __forceinline__ JobHit load(uint32_t i) const {
+        const float4 p = pos[i];
+        return JobHit{ld3(p), f2u(p.w), prim[i]};
+    }
+};
+
+template <bool kCount, bool kGroups>
+struct QueueJob {
     static constexpr bool kGoesOn = false;
-    const DevScene& S;
-    const RayQueue &in, &out;
-    const PhotonArrays& dep;
+    const RayQueue& in;
+    const HitArrays& hits;
     const TraceParams& tp;
-    const Reservoir& rs;
-    uint8_t *extFlags, *depFlags;
-    uint32_t number;  // seed of the launch
-    bool resv;
-    QueueCursor queue;
+    QueueCursor queue;  // of queue indices, or of places of the view groups
     uint32_t i = 0;
     Work w{};
 
     __device__ __forceinline__ bool drained() const { return queue.empty; }
     __device__ __forceinline__ bool fetch(bool idle, F3& o, F3& d) {
-        if (!queue.take(idle, i)) return false;
+        uint32_t t;
+        if (!queue.take(idle, t)) return false;
+        i = t;
+        if (kGroups && tp.groups) {
+            // Place t -> (view group, segment, rank) -> queue index.
+            uint32_t lo = 0, hi = tp.nGroups;  // last group whose first place <= t
+            while (hi - lo > 1u) {
+                const uint32_t mid = (lo + hi) >> 1;
+                if (tp.groups[mid].z <= t)
+                    lo = mid;
+                else
+                    hi = mid;
+            }
+            const uint4 gr = tp.groups[lo];
+            const uint32_t local = t - gr.z;
+            if (t < gr.z || local >= gr.y * gr.w) return false;
+            const uint32_t s = tp.groupSegs[gr.x + local % gr.y], r = local / gr.y;
+            if (r >= tp.segEnd[s] - tp.segFirst[s]) return false;
+            i = tp.segFirst[s] + r;
+        }
         o = ld3(in.o[i]);
         d = ld3(in.d[i]);
         return true;
@@ -257,8 +426,75 @@ struct PhotonJob {
     __device__ __forceinline__ bool finish(bool done, const JobHit& h, const Work& wl, F3&, F3&) {
         if (!done) return false;
         if (kCount) addWork(w, wl);
-        uint8_t ef = 0, df = 0;
-        Rng rng(perItemSeed(number, i));
+        hits.pos[i] = f4(h.pos, u2f(h.inst));
+        hits.prim[i] = h.prim;
+        return false;
+    }
+};
+
+// What a hit makes of a photon or an adjoint ray is left to the shade kernels,
+// one full wave after the other: at the end of the traversal it ran on half
+// empty waves, its registers spilled and kept the trace at 4 waves per SIMD.
+// The trace waits for its nodes: 5 waves (87 VGPRs, no spill) against 4 take
+// 4 % off the rays of 1M surfels and nothing off those of 100k.  Together with
+// the compaction in the shade kernels: backward pass of 800x800 rays on 1M
+// surfels 26.0 -> 21.2 ms, step of a 4k scene 2.05 -> 1.82 ms.
+template <bool kCount, bool kTopLds, bool kAdjoint>
+__device__ __forceinline__ void queueTrace(const DevScene& S, DevState* st, const RayQueue& in, const HitArrays& hits,
+                                           const TraceParams& tp) {
+    extern __shared__ uint2 s_stack[];
+    __shared__ TopLds sTop;
+    if (kTopLds) loadTopLds(S, sTop);
+    const LaneStack stk = walkStack(s_stack, S.stackDepth, tp.spill, tp.inLds);
+    const uint32_t n = st->qCount;
+    uint32_t end = n;
+    if (kAdjoint && tp.groups) {
+        const uint4 last = tp.nGroups ? tp.groups[tp.nGroups - 1u] : make_uint4(0u, 0u, 0u, 0u);
+        end = last.z + last.y * last.w;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        atomicAdd(kAdjoint ? &st->adjointQ : &st->photonQ, (unsigned long long)n);
+    QueueJob<kCount, kAdjoint> job{in, hits, tp, QueueCursor(&st->traceNext, end)};
+    if (kTopLds)
+        traceWave<kCount>(S, sTop, stk, job);
+    else
+        traceWave<kCount>(S, TopGlobal{S.tlas, S.inst}, stk, job);
+    if (kCount) flushWork(job.w, st, kAdjoint ? kWorkAdjoint : kWorkPhoton);
+}
+
+template <bool kCount, bool kTopLds>
+__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(5))) void k_photon_trace(
+    DevScene S, DevState* st, RayQueue in, HitArrays hits, TraceParams tp) {
+    queueTrace<kCount, kTopLds, false>(S, st, in, hits, tp);
+}
+template <bool kCount, bool kTopLds>
+__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(5))) void k_adj_trace(
+    DevScene S, DevState* st, RayQueue in, HitArrays hits, TraceParams tp) {
+    queueTrace<kCount, kTopLds, true>(S, st, in, hits, tp);
+}
+
+// launchIntersectKernel (PrimalKernels.cpp:65-321) for one queue: what the hit
+// of ray i deposits and the ray that goes on, written in queue order.
+__global__ __launch_bounds__(kTile) void k_photon_shade(DevScene S, DevState* st, RayQueue in, HitArrays hitArrays,
+                                                        RayQueue out, uint32_t outCap, PhotonArrays map,
+                                                        PhotonArrays staged, TraceParams tp, Reservoir rs,
+                                                        TileStates ts) {
+    const uint32_t n = st->qCount;
+    const uint32_t tile = tileTicket(st);
+    if (tile * kTile >= n) {
+        if (n == 0u && tile == 0u && threadIdx.x == 0) st->extTotal = st->depTotal = 0u;
+        return;
+    }
+    const QueueHits hits{hitArrays.pos, hitArrays.prim};
+    const uint32_t i = tile * kTile + threadIdx.x;
+    const bool resv = st->resv != 0u;
+    bool ef = false, df = false;
+    F3 no = mk3(0, 0, 0), nT = mk3(0, 0, 0), ndir = mk3(0, 0, 0);
+    float4 depPos, depDir;
+    float depZ = 0.0f;
+    uint32_t bounce = 0;
+    if (i < n) {
+        Rng rng(perItemSeed(st->number, i));
         // depositPhotonSurface past capacity (KernelHelpers.h:1705-1718): the
         // attempt index comes from the probe pass; accept with probability
         // cap / (attempt + 1), then pick the slot (two draws of this item).
@@ -272,21 +508,27 @@ struct PhotonJob {
                 if (u < accept) sl = rng.nextUint() % rs.cap;
             }
             rs.slot[i] = sl;
+            if (sl != kNoSlot) {
+                staged.posPow[i] = depPos;
+                staged.dirPow[i] = depDir;
+                staged.powZ[i] = depZ;
+            }
         };
         if (resv) rs.slot[i] = kNoSlot;
-        const float4 o4 = in.o[i], d4 = in.d[i], T4 = in.T[i];
-        const F3 d = ld3(d4), T = ld3(T4);
-        const uint32_t bounce = f2u(d4.w);
+        const float4 d4 = in.d[i];
+        const F3 d = ld3(d4), T = ld3(in.T[i]);
+        bounce = f2u(d4.w);
+        const JobHit h = hits.load(i);
         if (h.inst != kInvalid) {
             const DevInstance& I = S.inst[h.inst];
-            F3 no = mk3(0, 0, 0), nT = mk3(0, 0, 0), ndir = d;
+            ndir = d;
             bool spawn = false;
             if (I.type == kGeoMesh) {
                 const F3 ng = hitNormal(S, h);
-                df = 1;
-                dep.posPow[i] = f4(h.pos, T.x);
-                dep.dirPow[i] = f4(d, T.y);
-                dep.powZ[i] = T.z;
+                df = true;
+                depPos = f4(h.pos, T.x);
+                depDir = f4(d, T.y);
+                depZ = T.z;
                 reservoirDraws();
                 const DevMaterial m = S.mats[I.material];
                 float pdf;
@@ -310,10 +552,10 @@ struct PhotonJob {
                     const int sign = sc >= 0.0f ? 1 : -1;
                     const F3 on = (float)sign * nc;
                     const F3 flux = divs(T, tp.qReflect);
-                    df = 1;
-                    dep.posPow[i] = f4(h.pos, flux.x);
-                    dep.dirPow[i] = f4(d, flux.y);
-                    dep.powZ[i] = flux.z;
+                    df = true;
+                    depPos = f4(h.pos, flux.x);
+                    depDir = f4(d, flux.y);
+                    depZ = flux.z;
                     reservoirDraws();
                     float pdf;
                     sampleUniformHemi(rng, on, ndir, pdf);
@@ -340,64 +582,44 @@ struct PhotonJob {
                     spawn = true;
                 }
             }
-            if (spawn && russianRoulette(rng, bounce + 1, nT, tp.rrStart)) {
-                ef = 1;
-                out.o[i] = f4(no, o4.w);
-                out.d[i] = f4(ndir, u2f(bounce + 1));
-                out.T[i] = f4(nT, 0.0f);
-            }
+            ef = spawn && russianRoulette(rng, bounce + 1, nT, tp.rrStart);
         }
-        extFlags[i] = ef;
-        depFlags[i] = df;
-        return false;
     }
-};
-
-template <bool kCount, bool kTopLds>
-__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_photon_trace(
-    DevScene S, DevState* st, RayQueue in, RayQueue out, uint8_t* extFlags, PhotonArrays dep, uint8_t* depFlags,
-    TraceParams tp, Reservoir rs) {
-    extern __shared__ uint2 s_stack[];
-    __shared__ TopLds sTop;
-    if (kTopLds) loadTopLds(S, sTop);
-    const LaneStack stk = walkStack(s_stack, S.stackDepth, tp.spill, tp.inLds);
-    const uint32_t n = st->live ? st->qCount : 0u;
-    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&st->photonQ, (unsigned long long)n);
-    PhotonJob<kCount> job{S,  in,       out,      dep,        tp,          rs, extFlags, depFlags, st->number,
-                          st->resv != 0u, QueueCursor(&st->traceNext, n)};
-    if (kTopLds)
-        traceWave<kCount>(S, sTop, stk, job);
-    else
-        traceWave<kCount>(S, TopGlobal{S.tlas, S.inst}, stk, job);
-    if (kCount) flushWork(job.w, st, kWorkPhoton);
+    const TileOffset at = tileOffsets(ts, tile, ef, df);
+    if (ef && at.a < outCap) {
+        out.o[at.a] = f4(no, in.o[i].w);
+        out.d[at.a] = f4(ndir, u2f(bounce + 1));
+        out.T[at.a] = f4(nT, 0.0f);
+    }
+    if (df) {
+        const uint32_t j = st->photonCount + at.b;
+        if (j < rs.cap) {
+            map.posPow[j] = depPos;
+            map.dirPow[j] = depDir;
+            map.powZ[j] = depZ;
+        }
+    }
+    if (threadIdx.x == 0 && tile == (n - 1u) / kTile) {
+        st->extTotal = min(at.endA, outCap);
+        st->depTotal = at.endB;
+    }
 }
 
-// Reservoir mode of one bounce: on when the deposits so far plus one per
-// queued photon could pass the capacity.
-__global__ void k_resv_check(DevState* st, uint32_t cap) {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    st->resv = (st->live && (uint64_t)st->photonCount + (uint64_t)st->qCount > (uint64_t)cap) ? 1u : 0u;
-}
-
-// Probe pass of a reservoir bounce: which items deposit (the same hit and
-// the same first draw as k_photon_trace), so that every deposit learns its
-// attempt index in queue order before its random stream is used.
-__global__ __launch_bounds__(kTraceBlock) void k_photon_probe(DevScene S, DevState* st, RayQueue in,
-                                                              uint8_t* depFlags, TraceParams tp) {
+// Which items of a reservoir bounce deposit (the hit and the first draw of
+// k_photon_shade), so that every deposit learns its attempt index in queue order
+// before its random stream is used.
+__global__ __launch_bounds__(256) void k_photon_probe(DevScene S, const DevState* st, HitArrays hitArrays,
+                                                      uint8_t* depFlags, TraceParams tp) {
     if (!st->resv) return;
-    extern __shared__ uint2 s_stack[];
-    const LaneStack stk = laneStack(s_stack, S.stackDepth);
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t n = st->live ? st->qCount : 0u;
-    if (i >= n) return;
-    Rng rng(perItemSeed(st->number, i));
-    Work w{};
-    Hit h;
+    if (i >= st->qCount) return;
+    const JobHit h = QueueHits{hitArrays.pos, hitArrays.prim}.load(i);
     uint8_t df = 0;
-    if (intersectScene<false>(S, ld3(in.o[i]), ld3(in.d[i]), stk, h, w)) {
+    if (h.inst != kInvalid) {
         if (S.inst[h.inst].type == kGeoMesh) {
             df = 1;
         } else {
+            Rng rng(perItemSeed(st->number, i));
             const float u = rng.nextFloat();
             df = (u >= tp.qNull && u < tp.qNull + tp.qReflect) ? 1 : 0;
         }
@@ -409,7 +631,7 @@ __global__ __launch_bounds__(kTraceBlock) void k_photon_probe(DevScene S, DevSta
 __global__ __launch_bounds__(kScanThreads) void k_resv_rank(const uint8_t* flags, const DevState* st,
                                                             const uint32_t* tiles, uint32_t* attempt) {
     if (!st->resv) return;
-    const uint32_t n = st->live ? st->qCount : 0u;
+    const uint32_t n = st->qCount;
     const uint32_t first = blockIdx.x * kTile + threadIdx.x * kTileSpan;
     uint8_t f[kTileSpan];
     uint32_t s = 0;
@@ -428,7 +650,7 @@ __global__ __launch_bounds__(kScanThreads) void k_resv_rank(const uint8_t* flags
 
 __global__ __launch_bounds__(256) void k_resv_claim(const DevState* st, Reservoir rs) {
     if (!st->resv) return;
-    const uint32_t n = st->live ? st->qCount : 0u;
+    const uint32_t n = st->qCount;
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const uint32_t sl = rs.slot[i];
@@ -438,7 +660,7 @@ __global__ __launch_bounds__(256) void k_resv_claim(const DevState* st, Reservoi
 __global__ __launch_bounds__(256) void k_resv_write(const DevState* st, Reservoir rs, PhotonArrays dep,
                                                     PhotonArrays raw) {
     if (!st->resv) return;
-    const uint32_t n = st->live ? st->qCount : 0u;
+    const uint32_t n = st->qCount;
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const uint32_t sl = rs.slot[i];
@@ -448,7 +670,7 @@ __global__ __launch_bounds__(256) void k_resv_write(const DevState* st, Reservoi
     raw.powZ[sl] = dep.powZ[i];
 }
 
-// -------------------------------------------------- stable compaction --
+// --------------------------------------------------------- tile scans --
 __global__ __launch_bounds__(kScanThreads) void k_tile_count(const uint8_t* flags, const uint32_t* count,
                                                              uint32_t maxItems, uint32_t* tiles) {
     const uint32_t n = loadCount(count, maxItems);
@@ -498,69 +720,6 @@ __global__ __launch_bounds__(1024) void k_tile_scan(uint32_t* tiles, const uint3
         __syncthreads();
     }
     if (threadIdx.x == 0) *total = carry < cap ? carry : cap;
-}
-
-template <typename Copy>
-__device__ __forceinline__ void scatterTile(const uint8_t* flags, uint32_t n, const uint32_t* tiles, uint32_t base,
-                                            uint32_t cap, Copy copy) {
-    const uint32_t first = blockIdx.x * kTile + threadIdx.x * kTileSpan;
-    uint8_t f[kTileSpan];
-    uint32_t s = 0;
-#pragma unroll
-    for (uint32_t k = 0; k < kTileSpan; ++k) {
-        f[k] = (first + k < n) ? flags[first + k] : 0;
-        s += f[k];
-    }
-    uint32_t total;
-    uint32_t off = blockExclusiveScan(s, total) + tiles[blockIdx.x] + base;
-#pragma unroll
-    for (uint32_t k = 0; k < kTileSpan; ++k) {
-        if (f[k]) {
-            if (off < cap) copy(first + k, off);
-            ++off;
-        }
-    }
-}
-
-__global__ __launch_bounds__(kScanThreads) void k_scatter_rays(const uint8_t* flags, const uint32_t* count,
-                                                               uint32_t maxItems, const uint32_t* tiles,
-                                                               RayQueue src, RayQueue dst, uint32_t cap) {
-    const uint32_t n = loadCount(count, maxItems);
-    scatterTile(flags, n, tiles, 0u, cap, [&](uint32_t i, uint32_t j) {
-        dst.o[j] = src.o[i];
-        dst.d[j] = src.d[i];
-        dst.T[j] = src.T[i];
-    });
-}
-
-__global__ __launch_bounds__(kScanThreads) void k_scatter_photons(const uint8_t* flags, const uint32_t* count,
-                                                                  uint32_t maxItems, const uint32_t* tiles,
-                                                                  const uint32_t* base, PhotonArrays src,
-                                                                  PhotonArrays dst, uint32_t cap) {
-    const uint32_t n = loadCount(count, maxItems);
-    scatterTile(flags, n, tiles, *base, cap, [&](uint32_t i, uint32_t j) {
-        dst.posPow[j] = src.posPow[i];
-        dst.dirPow[j] = src.dirPow[i];
-        dst.powZ[j] = src.powZ[i];
-    });
-}
-
-__global__ __launch_bounds__(kScanThreads) void k_scatter_events(const uint8_t* flags, const uint32_t* count,
-                                                                 uint32_t maxItems, const uint32_t* tiles,
-                                                                 const uint32_t* base, EventArrays src,
-                                                                 EventArrays dst, uint32_t cap) {
-    const uint32_t n = loadCount(count, maxItems);
-    const bool rays = src.e4 != nullptr;
-    scatterTile(flags, n, tiles, *base, cap, [&](uint32_t i, uint32_t j) {
-        dst.e0[j] = src.e0[i];
-        dst.e1[j] = src.e1[i];
-        dst.e2[j] = src.e2[i];
-        dst.e3[j] = src.e3[i];
-        if (rays) {
-            dst.e4[j] = src.e4[i];
-            dst.e5[j] = src.e5[i];
-        }
-    });
 }
 
 // ------------------------------------------------------ photon grid --
@@ -1224,10 +1383,7 @@ __global__ __launch_bounds__(256) void k_adj_raygen(DevCamera cam, const float* 
                                                     PendingArrays pend, DevState* st, uint32_t seed) {
     const uint32_t npx = cam.W * cam.H;
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i == 0) {
-        st->qCount = npx;
-        st->traceNext = 0;
-    }
+    if (i == 0) st->qCount = npx;
     if (i >= npx) return;
     Rng rng(perItemSeed((uint64_t)seed, i));
     const float jx = rng.nextFloat() - 0.5f;
@@ -1243,12 +1399,9 @@ __global__ __launch_bounds__(256) void k_adj_raygen(DevCamera cam, const float* 
 // Adjoint primary rays of a batch: one thread per tile pixel, the jitter and
 // ray of k_adj_raygen for the pixel of its view; queue index = slot.
 __global__ __launch_bounds__(256) void k_adj_raygen_batch(BatchDesc b, const float* dloss, RayQueue q,
-                                                          PendingArrays pend, DevState* st) {
+                                                          PendingArrays pend, DevState* st, uint32_t* segFirst) {
     const uint32_t t = blockIdx.x * 4u + (threadIdx.x >> 6);
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        st->qCount = b.hdr->nSlots;
-        st->traceNext = 0;
-    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) st->qCount = b.hdr->nSlots;
     if (t >= b.hdr->nTiles) return;
     uint32_t seg, pxx, pxy;
     const BatchSeg* sp;
@@ -1260,6 +1413,7 @@ __global__ __launch_bounds__(256) void k_adj_raygen_batch(BatchDesc b, const flo
     const float jy = rng.nextFloat() - 0.5f;
     F3 o, d;
     primaryRay(b.cams[s.view], (float)pxx, (float)pxy, jx, jy, o, d);
+    if (pixel == 0u) segFirst[seg] = slot;
     const size_t src = 3 * ((size_t)s.pixOffset + pixel);
     q.o[slot] = f4(o, u2f(slot));
     q.d[slot] = f4(d, u2f(0u));
@@ -1267,98 +1421,37 @@ __global__ __launch_bounds__(256) void k_adj_raygen_batch(BatchDesc b, const flo
     pend.p0[slot] = make_float4(0.0f, 0.0f, 0.0f, u2f(kNone));
 }
 
-// First and end queue index of every segment present in a batch's queue
-// (the queue stays in slot order: raygen writes slot order, compaction is
-// stable); absent segments keep first = end = 0 from k_seg_clear.
-__global__ __launch_bounds__(256) void k_seg_clear(uint32_t* segFirst, uint32_t* segEnd, uint32_t nSegs) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < nSegs) segFirst[i] = segEnd[i] = 0u;
-}
-
-__global__ __launch_bounds__(256) void k_seg_first(const DevState* st, RayQueue q, uint32_t* segFirst,
-                                                   uint32_t* segEnd) {
-    const uint32_t n = st->qCount;
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t seg = f2u(q.T[i].w);
-    if (i == 0 || f2u(q.T[i - 1].w) != seg) segFirst[seg] = i;
-    if (i + 1 == n || f2u(q.T[i + 1].w) != seg) segEnd[seg] = i + 1;
-}
-
-// Lanes of each view group: K segments x the most rays of one of them.
-__global__ __launch_bounds__(64) void k_group_lanes(const uint32_t* segFirst, const uint32_t* segEnd, uint4* groups,
-                                                    uint32_t nGroups, const uint32_t* groupSegs) {
-    if (threadIdx.x != 0) return;
-    uint32_t base = 0;
-    for (uint32_t g = 0; g < nGroups; ++g) {
-        uint4 gr = groups[g];
-        uint32_t most = 0;
-        for (uint32_t k = 0; k < gr.y; ++k) {
-            const uint32_t s = groupSegs[gr.x + k];
-            most = max(most, segEnd[s] - segFirst[s]);
-        }
-        gr.z = base;
-        gr.w = most;
-        groups[g] = gr;
-        base += gr.y * most;
-    }
-}
-
 // launchAdjointIntersectKernel (AdjointKernels.cpp:87-386) for one queue: the
-// hit of ray i, the pending event it completes, the event it makes and the
-// ray that goes on.
-template <bool kCount>
-struct AdjointJob {
-    static constexpr bool kGoesOn = false;
-    const DevScene& S;
-    const RayQueue &in, &out;
-    const EventArrays& ev;
-    const PendingArrays& pend;
-    const TraceParams& tp;
-    uint8_t *extFlags, *evFlags;
-    uint32_t bounceIndex, pendCap;
-    QueueCursor queue;  // of queue indices, or of lanes of the view groups
-    uint32_t i = 0;
-    Work w{};
-
-    __device__ __forceinline__ bool drained() const { return queue.empty; }
-    __device__ __forceinline__ bool fetch(bool idle, F3& o, F3& d) {
-        uint32_t t;
-        if (!queue.take(idle, t)) return false;
-        i = t;
-        if (tp.groups) {
-            // Place t -> (view group, segment, rank) -> queue index.
-            uint32_t lo = 0, hi = tp.nGroups;  // last group whose first place <= t
-            while (hi - lo > 1u) {
-                const uint32_t mid = (lo + hi) >> 1;
-                if (tp.groups[mid].z <= t)
-                    lo = mid;
-                else
-                    hi = mid;
-            }
-            const uint4 gr = tp.groups[lo];
-            const uint32_t local = t - gr.z;
-            if (t < gr.z || local >= gr.y * gr.w) return false;
-            const uint32_t s = tp.groupSegs[gr.x + local % gr.y], r = local / gr.y;
-            if (r >= tp.segEnd[s] - tp.segFirst[s]) return false;
-            i = tp.segFirst[s] + r;
-        }
-        o = ld3(in.o[i]);
-        d = ld3(in.d[i]);
-        return true;
+// pending event that the hit of ray i completes, the event it makes and the ray
+// that goes on, written in queue order; segNext gets the first place of every
+// segment that goes on (a batch).
+__global__ __launch_bounds__(kTile) void k_adj_shade(DevScene S, DevState* st, uint32_t bounceIndex, RayQueue in,
+                                                     HitArrays hitArrays, RayQueue out, uint32_t outCap,
+                                                     EventArrays pool, uint32_t poolCap, PendingArrays pend,
+                                                     uint32_t pendCap, TraceParams tp, uint32_t* segNext,
+                                                     TileStates ts) {
+    const uint32_t n = st->qCount;
+    const uint32_t tile = tileTicket(st);
+    if (tile * kTile >= n) {
+        if (n == 0u && tile == 0u && threadIdx.x == 0) st->extTotal = st->evTotal = 0u;
+        return;
     }
-    __device__ __forceinline__ bool finish(bool done, const JobHit& h, const Work& wl, F3&, F3&) {
-        if (!done) return false;
-        if (kCount) addWork(w, wl);
-        uint8_t ef = 0, vf = 0;
+    const QueueHits hits{hitArrays.pos, hitArrays.prim};
+    const uint32_t i = tile * kTile + threadIdx.x;
+    bool ef = false, vf = false;
+    F3 no = mk3(0, 0, 0), nT = mk3(0, 0, 0), ndir = mk3(0, 0, 0);
+    float4 e0, e1, e2, e3, e4, e5;
+    uint32_t seg = 0, path = 0, bounce = 0;
+    if (i < n) {
         const float4 o4 = in.o[i], d4 = in.d[i], T4 = in.T[i];
-        const uint32_t seg = f2u(T4.w);
+        const JobHit h = hits.load(i);
+        seg = f2u(T4.w);
         const uint32_t rank = tp.segFirst ? i - tp.segFirst[seg] : i;
         const float invS = tp.segs ? tp.segs[seg].invSpp : tp.invSpp;
         Rng rng(perItemSeed((uint64_t)(tp.segs ? tp.segs[seg].seed : tp.seed), rank));
         const F3 o = ld3(o4), d = ld3(d4), T = ld3(T4);
-        const uint32_t path = f2u(o4.w);
-        const uint32_t bounce = f2u(d4.w);
+        path = f2u(o4.w);
+        bounce = f2u(d4.w);
         const uint32_t dpx = !tp.debug ? 0u
                              : tp.segs ? tp.segs[seg].pixOffset + (path - tp.segs[seg].slotBase)
                                        : tp.debugBase + path;
@@ -1392,40 +1485,38 @@ struct AdjointJob {
                     const uint2 p2 = pend.p2[path];
                     const F3 Tp = ld3(p1) * (reflectDone ? tp.qReflect : tp.qNull);
                     const float endCos = fmaxf(0.0f, dot(dir, on));
-                    ev.e0[i] = f4(h.pos, u2f(kind));
+                    e0 = f4(h.pos, u2f(kind));
                     if (reflectDone) {
-                        ev.e1[i] = f4(on, u2f(h.prim));
-                        ev.e2[i] = f4(Tp, hAlpha);
-                        ev.e3[i] = make_float4(u2f(S.inst[p2.y].material), pdf, endCos, invS);
+                        e1 = f4(on, u2f(h.prim));
+                        e2 = f4(Tp, hAlpha);
+                        e3 = make_float4(u2f(S.inst[p2.y].material), pdf, endCos, invS);
                         if (tp.fullGradients || tp.debug) {  // this ray hit the endpoint surfel
-                            ev.e4[i] = f4(o, 0.0f);
-                            ev.e5[i] = f4(d, u2f(dpx));
+                            e4 = f4(o, 0.0f);
+                            e5 = f4(d, u2f(dpx));
                         }
                     } else {
-                        ev.e1[i] = f4(on, u2f(p2.x));
-                        ev.e2[i] = f4(Tp, p1.w);
-                        ev.e3[i] = make_float4(u2f(cloud ? kGeoCloud : kGeoMesh), u2f(cloud ? h.prim : I.material),
-                                               endCos, invS);
+                        e1 = f4(on, u2f(p2.x));
+                        e2 = f4(Tp, p1.w);
+                        e3 = make_float4(u2f(cloud ? kGeoCloud : kGeoMesh), u2f(cloud ? h.prim : I.material), endCos,
+                                         invS);
                         if (tp.fullGradients) {  // the ray that crossed the pending surfel
-                            ev.e4[i] = pend.p3[path];
-                            float4 e5 = pend.p4[path];
+                            e4 = pend.p3[path];
+                            e5 = pend.p4[path];
                             e5.w = u2f(dpx);
-                            ev.e5[i] = e5;
                         } else if (tp.debug) {
-                            ev.e5[i] = make_float4(0.0f, 0.0f, 0.0f, u2f(dpx));
+                            e5 = make_float4(0.0f, 0.0f, 0.0f, u2f(dpx));
                         }
                     }
-                    vf = 1;
+                    vf = true;
                     pend.p0[path] = make_float4(0.0f, 0.0f, 0.0f, u2f(kNone));
                 }
             }
-            F3 no, nT;
             bool spawn = false;
             uint32_t newKind = kNone;
             F3 pT = mk3(0, 0, 0);
             float pAlpha = 0.0f;
             uint2 pIds = make_uint2(kInvalid, kInvalid);
-            F3 ndir = dir;
+            ndir = dir;
             bool projection = false;
             if (!cloud) {
                 const DevMaterial m = S.mats[I.material];
@@ -1483,50 +1574,52 @@ struct AdjointJob {
                     }
                 }
                 if (projection && path < pendCap) {
-                    ev.e0[i] = f4(h.pos, u2f(kProjection));
-                    ev.e1[i] = f4(on, u2f(h.prim));
-                    ev.e2[i] = f4(divs(T, tp.qReflect), hAlpha);
-                    ev.e3[i] = make_float4(0.0f, 0.0f, 0.0f, invS);
+                    e0 = f4(h.pos, u2f(kProjection));
+                    e1 = f4(on, u2f(h.prim));
+                    e2 = f4(divs(T, tp.qReflect), hAlpha);
+                    e3 = make_float4(0.0f, 0.0f, 0.0f, invS);
                     if (tp.fullGradients || tp.debug) {
-                        ev.e4[i] = f4(o, 0.0f);
-                        ev.e5[i] = f4(d, u2f(dpx));
+                        e4 = f4(o, 0.0f);
+                        e5 = f4(d, u2f(dpx));
                     }
-                    vf = 1;
+                    vf = true;
                 }
-                ef = 1;
-                out.o[i] = f4(no, o4.w);
-                out.d[i] = f4(ndir, u2f(bounce + 1));
-                out.T[i] = f4(nT, T4.w);
+                ef = true;
             }
         }
-        extFlags[i] = ef;
-        evFlags[i] = vf;
-        return false;
     }
-};
-
-template <bool kCount, bool kTopLds>
-__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_adj_trace(
-    DevScene S, DevState* st, uint32_t bounceIndex, RayQueue in, RayQueue out, uint8_t* extFlags, EventArrays ev,
-    uint8_t* evFlags, PendingArrays pend, uint32_t pendCap, TraceParams tp) {
-    extern __shared__ uint2 s_stack[];
-    __shared__ TopLds sTop;
-    if (kTopLds) loadTopLds(S, sTop);
-    const LaneStack stk = walkStack(s_stack, S.stackDepth, tp.spill, tp.inLds);
-    const uint32_t n = st->qCount;
-    uint32_t end = n;
-    if (tp.groups) {
-        const uint4 last = tp.nGroups ? tp.groups[tp.nGroups - 1u] : make_uint4(0u, 0u, 0u, 0u);
-        end = last.z + last.y * last.w;
+    const TileOffset at = tileOffsets(ts, tile, ef, vf);
+    if (vf) {
+        const uint32_t j = st->evPool + at.b;
+        if (j < poolCap) {
+            pool.e0[j] = e0;
+            pool.e1[j] = e1;
+            pool.e2[j] = e2;
+            pool.e3[j] = e3;
+            if (pool.e4) {
+                pool.e4[j] = e4;
+                pool.e5[j] = e5;
+            }
+        }
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&st->adjointQ, (unsigned long long)n);
-    AdjointJob<kCount> job{S,  in,       out,     ev,          pend,    tp,
-                           extFlags, evFlags, bounceIndex, pendCap, QueueCursor(&st->traceNext, end)};
-    if (kTopLds)
-        traceWave<kCount>(S, sTop, stk, job);
-    else
-        traceWave<kCount>(S, TopGlobal{S.tlas, S.inst}, stk, job);
-    if (kCount) flushWork(job.w, st, kWorkAdjoint);
+    if (ef && at.a < outCap) {
+        out.o[at.a] = f4(no, u2f(path));
+        out.d[at.a] = f4(ndir, u2f(bounce + 1));
+        out.T[at.a] = f4(nT, u2f(seg));
+    }
+    if (segNext) {
+        // The wave's first ray of each segment; the value read first spares
+        // the atomic of the waves behind the segment's start.
+        const uint32_t lane = laneId();
+        const unsigned long long m = __ballot(ef), before = m & ((1ull << lane) - 1ull);
+        const uint32_t prev = before ? 63u - (uint32_t)__clzll((long long)before) : lane;
+        const uint32_t prevSeg = __shfl(seg, (int)prev, 64);
+        if (ef && (!before || prevSeg != seg) && at.a < segNext[seg]) atomicMin(segNext + seg, at.a);
+    }
+    if (threadIdx.x == 0 && tile == (n - 1u) / kTile) {
+        st->extTotal = min(at.endA, outCap);
+        st->evTotal = at.endB;
+    }
 }
 
 // Counting sort of the pooled events by the photon-grid cell of their
@@ -1884,13 +1977,15 @@ void launchFillF(hipStream_t s, float* p, uint32_t n, float v) {
 void launchIota(hipStream_t s, uint32_t* p, uint32_t n) {
     if (n) k_iota<<<min(blocks(n, 256), 65535u), 256, 0, s>>>(p, n);
 }
-void launchSeedNext(hipStream_t s, DevState* st, const uint32_t* table, uint32_t len, int bounce) {
-    k_seed_next<<<1, 64, 0, s>>>(st, table, len, bounce);
+static inline uint32_t tilesOf(uint32_t rays) { return blocks(rays, kTile); }
+void launchPhotonNext(hipStream_t s, DevState* st, const uint32_t* table, uint32_t len, int bounce, uint32_t resvCap,
+                      TileStates ts, uint32_t rays) {
+    k_photon_next<<<1, 256, 0, s>>>(st, table, len, bounce, resvCap, ts, tilesOf(rays));
 }
 void launchBeginView(hipStream_t s, DevState* st, uint32_t number) { k_begin_view<<<1, 64, 0, s>>>(st, number); }
-void launchEmit(hipStream_t s, const DevScene& S, DevState* st, uint32_t P, float invEmitted, RayQueue staged,
-                uint8_t* flags) {
-    if (P) k_emit<<<blocks(P, 256), 256, 0, s>>>(S, st, P, invEmitted, staged, flags);
+void launchEmit(hipStream_t s, const DevScene& S, DevState* st, uint32_t P, float invEmitted, RayQueue out,
+                uint32_t outCap, TileStates ts) {
+    k_emit<<<tilesOf(max(P, 1u)), kTile, 0, s>>>(S, st, P, invEmitted, out, outCap, ts);
 }
 // Persistent grid of a trace kernel: as many workgroups as fit on the device.
 // Renderers on several host threads share the cache.
@@ -1933,64 +2028,40 @@ uint32_t queueTraceLanes(const DevScene& S, uint32_t rays, uint32_t inLds) {
     return min(grid, blocks(rays, kTraceBlock)) * kTraceBlock;
 }
 
-void launchPhotonTrace(hipStream_t s, const DevScene& S, DevState* st, uint32_t maxRays, RayQueue in,
-                       RayQueue staged, uint8_t* extFlags, PhotonArrays dep, uint8_t* depFlags, TraceParams tp,
-                       Reservoir rs, uint32_t* tiles, bool count) {
+void launchQueueTrace(hipStream_t s, const DevScene& S, DevState* st, uint32_t maxRays, RayQueue in, HitArrays hits,
+                      TraceParams tp, bool adjoint, bool count) {
     if (!maxRays) return;
-    const dim3 g(blocks(maxRays, kTraceBlock));
+    using Kernel = void (*)(DevScene, DevState*, RayQueue, HitArrays, TraceParams);
+    static constexpr Kernel kernels[2][2][2] = {
+        {{&k_photon_trace<false, false>, &k_photon_trace<false, true>},
+         {&k_photon_trace<true, false>, &k_photon_trace<true, true>}},
+        {{&k_adj_trace<false, false>, &k_adj_trace<false, true>}, {&k_adj_trace<true, false>, &k_adj_trace<true, true>}}};
+    const size_t lds = tp.spill ? (size_t)tp.inLds * sizeof(uint2) * kTraceBlock : stackBytes(S);
+    const Kernel k = kernels[adjoint][count][topFitsLds(S)];
+    const uint32_t g = min(traceGrid(reinterpret_cast<const void*>(k), lds), blocks(maxRays, kTraceBlock));
+    k<<<g, kTraceBlock, lds, s>>>(S, st, in, hits, tp);
+}
+
+void launchPhotonShade(hipStream_t s, const DevScene& S, DevState* st, uint32_t maxRays, RayQueue in, HitArrays hits,
+                       RayQueue out, uint32_t outCap, PhotonArrays map, PhotonArrays staged, TraceParams tp,
+                       Reservoir rs, uint8_t* depFlags, uint32_t* tiles, TileStates ts) {
+    if (!maxRays) return;
     if (rs.attempt) {
-        // The map can fill during this render: probe, rank, then trace.
-        k_resv_check<<<1, 64, 0, s>>>(st, rs.cap);
-        k_photon_probe<<<g, kTraceBlock, stackBytes(S), s>>>(S, st, in, depFlags, tp);
+        // The map can fill during this render: which deposit, their ranks.
         const uint32_t* qCount =
             reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(st) + offsetof(DevState, qCount));
         const uint32_t nt = blocks(maxRays, kTile);
+        k_photon_probe<<<blocks(maxRays, 256), 256, 0, s>>>(S, st, hits, depFlags, tp);
         k_tile_count<<<nt, kScanThreads, 0, s>>>(depFlags, qCount, maxRays, tiles);
         k_tile_scan<<<1, 1024, 0, s>>>(tiles, qCount, 0u, maxRays, tiles + nt, 0xFFFFFFFFu);
         k_resv_rank<<<nt, kScanThreads, 0, s>>>(depFlags, st, tiles, rs.attempt);
     }
-    const size_t lds = tp.spill ? (size_t)tp.inLds * sizeof(uint2) * kTraceBlock : stackBytes(S);
-    const bool top = topFitsLds(S);
-    const auto k = count ? (top ? &k_photon_trace<true, true> : &k_photon_trace<true, false>)
-                         : (top ? &k_photon_trace<false, true> : &k_photon_trace<false, false>);
-    const uint32_t pg = min(traceGrid(reinterpret_cast<const void*>(k), lds), blocks(maxRays, kTraceBlock));
-    k<<<pg, kTraceBlock, lds, s>>>(S, st, in, staged, extFlags, dep, depFlags, tp, rs);
+    k_photon_shade<<<tilesOf(maxRays), kTile, 0, s>>>(S, st, in, hits, out, outCap, map, staged, tp, rs, ts);
+    if (rs.attempt) {
+        k_resv_claim<<<blocks(maxRays, 256), 256, 0, s>>>(st, rs);
+        k_resv_write<<<blocks(maxRays, 256), 256, 0, s>>>(st, rs, staged, map);
+    }
 }
-void launchReservoirWrite(hipStream_t s, DevState* st, uint32_t maxRays, Reservoir rs, PhotonArrays dep,
-                          PhotonArrays raw) {
-    if (!maxRays || !rs.attempt) return;
-    k_resv_claim<<<blocks(maxRays, 256), 256, 0, s>>>(st, rs);
-    k_resv_write<<<blocks(maxRays, 256), 256, 0, s>>>(st, rs, dep, raw);
-}
-void launchCompactRays(hipStream_t s, const uint8_t* flags, const uint32_t* count, uint32_t maxItems,
-                       uint32_t* tiles, uint32_t* total, RayQueue src, RayQueue dst, uint32_t dstCap) {
-    const uint32_t nt = blocks(maxItems, kTile);
-    k_tile_count<<<nt, kScanThreads, 0, s>>>(flags, count, maxItems, tiles);
-    k_tile_scan<<<1, 1024, 0, s>>>(tiles, count, 0u, maxItems, total, dstCap);
-    k_scatter_rays<<<nt, kScanThreads, 0, s>>>(flags, count, maxItems, tiles, src, dst, dstCap);
-}
-void launchCompactPhotons(hipStream_t s, const uint8_t* flags, const uint32_t* count, uint32_t maxItems,
-                          uint32_t* tiles, uint32_t* total, const uint32_t* base, PhotonArrays src,
-                          PhotonArrays dst, uint32_t dstCap) {
-    const uint32_t nt = blocks(maxItems, kTile);
-    k_tile_count<<<nt, kScanThreads, 0, s>>>(flags, count, maxItems, tiles);
-    k_tile_scan<<<1, 1024, 0, s>>>(tiles, count, 0u, maxItems, total, 0xFFFFFFFFu);
-    k_scatter_photons<<<nt, kScanThreads, 0, s>>>(flags, count, maxItems, tiles, base, src, dst, dstCap);
-}
-void launchCompactEvents(hipStream_t s, const uint8_t* flags, const uint32_t* count, uint32_t maxItems,
-                         uint32_t* tiles, DevState* st, EventArrays src, EventArrays pool, uint32_t poolCap) {
-    const uint32_t nt = blocks(maxItems, kTile);
-    uint32_t* total = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(st) + offsetof(DevState, evTotal));
-    const uint32_t* base = reinterpret_cast<const uint32_t*>(reinterpret_cast<char*>(st) + offsetof(DevState, evPool));
-    k_tile_count<<<nt, kScanThreads, 0, s>>>(flags, count, maxItems, tiles);
-    k_tile_scan<<<1, 1024, 0, s>>>(tiles, count, 0u, maxItems, total, 0xFFFFFFFFu);
-    k_scatter_events<<<nt, kScanThreads, 0, s>>>(flags, count, maxItems, tiles, base, src, pool, poolCap);
-    k_event_pool_add<<<1, 64, 0, s>>>(st, poolCap);
-}
-void launchFinishPhotonBounce(hipStream_t s, DevState* st, uint32_t cap) {
-    k_finish_photon_bounce<<<1, 64, 0, s>>>(st, cap);
-}
-void launchSetQueue(hipStream_t s, DevState* st, const uint32_t* src) { k_set_queue<<<1, 64, 0, s>>>(st, src); }
 
 void launchBuildGrid(hipStream_t s, const GridParams& g, DevState* st, uint32_t cap, PhotonArrays raw,
                      PhotonArrays sorted, uint32_t* cellId, uint32_t* sortedIdx, uint32_t* cellCount,
@@ -2133,31 +2204,26 @@ void launchPostprocess(hipStream_t s, const float4* fb, float4* ldr, uint32_t n)
     if (n) k_post<<<blocks(n, 256), 256, 0, s>>>(fb, ldr, n);
 }
 void launchAdjRaygenBatch(hipStream_t s, BatchDesc b, uint32_t maxTiles, const float* dloss, RayQueue q,
-                          PendingArrays pend, DevState* st) {
-    k_adj_raygen_batch<<<blocks(max(maxTiles, 1u), 4), 256, 0, s>>>(b, dloss, q, pend, st);
+                          PendingArrays pend, DevState* st, uint32_t* segFirst) {
+    k_adj_raygen_batch<<<blocks(max(maxTiles, 1u), 4), 256, 0, s>>>(b, dloss, q, pend, st, segFirst);
 }
-void launchSegFirst(hipStream_t s, const DevState* st, uint32_t maxRays, RayQueue q, uint32_t* segFirst,
-                    uint32_t* segEnd, uint32_t nSegs, uint4* groups, uint32_t nGroups, const uint32_t* groupSegs) {
-    if (!maxRays) return;
-    k_seg_clear<<<blocks(max(nSegs, 1u), 256), 256, 0, s>>>(segFirst, segEnd, nSegs);
-    k_seg_first<<<blocks(maxRays, 256), 256, 0, s>>>(st, q, segFirst, segEnd);
-    k_group_lanes<<<1, 64, 0, s>>>(segFirst, segEnd, groups, nGroups, groupSegs);
+void launchAdjNext(hipStream_t s, DevState* st, int bounce, uint32_t poolCap, TileStates ts, uint32_t rays,
+                   uint32_t* segFirst, uint32_t* segEnd, uint32_t* segNext, uint32_t nSegs, uint4* groups,
+                   uint32_t nGroups, const uint32_t* groupSegs) {
+    k_adj_next<<<1, 256, 0, s>>>(st, bounce, poolCap, ts, tilesOf(rays), segFirst, segEnd, segNext, nSegs, groups,
+                                 nGroups, groupSegs);
+}
+void launchAdjShade(hipStream_t s, const DevScene& S, DevState* st, uint32_t maxRays, uint32_t bounce, RayQueue in,
+                    HitArrays hits, RayQueue out, uint32_t outCap, EventArrays pool, uint32_t poolCap,
+                    PendingArrays pend, TraceParams tp, uint32_t* segNext, TileStates ts) {
+    if (maxRays)
+        k_adj_shade<<<tilesOf(maxRays), kTile, 0, s>>>(S, st, bounce, in, hits, out, outCap, pool, poolCap, pend,
+                                                       maxRays, tp, segNext, ts);
 }
 void launchAdjRaygen(hipStream_t s, const DevCamera& cam, const float* dloss, RayQueue q, PendingArrays pend,
                      DevState* st, uint32_t seed) {
     const uint32_t npx = cam.W * cam.H;
     k_adj_raygen<<<blocks(npx > 0 ? npx : 1, 256), 256, 0, s>>>(cam, dloss, q, pend, st, seed);
-}
-void launchAdjTrace(hipStream_t s, const DevScene& S, DevState* st, uint32_t maxRays, uint32_t bounce, RayQueue in,
-                    RayQueue staged, uint8_t* extFlags, EventArrays ev, uint8_t* evFlags, PendingArrays pend,
-                    TraceParams tp, bool count) {
-    if (!maxRays) return;
-    const size_t lds = tp.spill ? (size_t)tp.inLds * sizeof(uint2) * kTraceBlock : stackBytes(S);
-    const bool top = topFitsLds(S);
-    const auto k = count ? (top ? &k_adj_trace<true, true> : &k_adj_trace<true, false>)
-                         : (top ? &k_adj_trace<false, true> : &k_adj_trace<false, false>);
-    const uint32_t g = min(traceGrid(reinterpret_cast<const void*>(k), lds), blocks(maxRays, kTraceBlock));
-    k<<<g, kTraceBlock, lds, s>>>(S, st, bounce, in, staged, extFlags, ev, evFlags, pend, maxRays, tp);
 }
 void launchEventSort(hipStream_t s, const GridParams& g, DevState* st, uint32_t poolCap, EventArrays ev,
                      uint32_t* cell, uint32_t* sorted, uint32_t* cellCount, uint32_t* cellStart, uint32_t* tiles,

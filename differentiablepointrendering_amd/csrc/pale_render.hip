@@ -267,11 +267,11 @@ class DeviceCloudBuild final : public CloudBuild {
 // only a symbol: its device address comes from hipGetSymbolAddress, resolved
 // once per device (noAllocScratch) and kept in the handle.
 constexpr uint32_t kNoAllocMaxPixels = 65536;  // 256 x 256
-// Per pixel: 9 queue arrays (16 B), 2 flag bytes, pending 16 + 16 + 8 B,
-// 4 staging + 4 pool event arrays (16 B), 4 B of transport order; plus the
-// compaction tiles.
+// Per pixel: 6 queue arrays (16 B), hits 16 + 4 B, pending 16 + 16 + 8 B, 4
+// event arrays (16 B), 4 B of transport order; plus the compaction's tiles.
 constexpr size_t kNoAllocScratchBytes =
-    (size_t)kNoAllocMaxPixels * (9 * 16 + 1 + 1 + 16 + 16 + 8 + 4 * 16 + 4 * 16 + 4) + 512;
+    (size_t)kNoAllocMaxPixels * (6 * 16 + 16 + 4 + 16 + 16 + 8 + 4 * 16 + 4) +
+    ((kNoAllocMaxPixels / kTile + 1) * 8 + 255) / 256 * 256;
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
 namespace {
@@ -327,15 +327,16 @@ struct pale_handle {
 
     // Ray queues and staging.
     uint32_t queueCap = 0;
-    DevMem qA[3], qB[3], stg[3], extFlags, depStg[3], depFlags, tiles, counts;
+    DevMem qA[3], qB[3], hitPos, hitPrim, tileState;
+    DevMem depStg[3], depFlags, tiles;  // only where the photon map can fill
     DevMem walkSpill;  // layer-walk stack entries beyond the LDS part (deep BVHs)
     uint2* walkSpillPtr() const { return walkSpill.p ? walkSpill.as<uint2>() : nullptr; }
     uint32_t walkLds() const { return tune.walk_lds_entries ? tune.walk_lds_entries : kWalkLdsEntries; }
     // The photon and adjoint traces keep kTraceLdsEntries stack entries per
-    // lane in LDS and the rest in traceSpill: 16 KB of LDS per workgroup
+    // lane in LDS and the rest in traceSpill: 12 KB of LDS per workgroup
     // instead of the whole stack's (31 KB at 1M surfels), so that LDS allows
-    // the 4 waves per SIMD their registers allow.
-    static constexpr uint32_t kTraceLdsEntries = 16;
+    // the 5 waves per SIMD their registers allow (8 or 16 entries: within 2 %).
+    static constexpr uint32_t kTraceLdsEntries = 12;
     DevMem traceSpill;
     size_t traceSpillBytes(uint32_t rays) const {
         if (img.stackDepth <= kTraceLdsEntries || !rays) return 0;
@@ -360,7 +361,7 @@ struct pale_handle {
     }
     // Adjoint.
     uint32_t adjCap = 0, poolCap = 0;
-    DevMem pend0, pend1, pend2, pend3, pend4, evStg[6], evCmp[6], evCell, evSorted, evFlags, dloss, gradOpacity,
+    DevMem pend0, pend1, pend2, pend3, pend4, evCmp[6], evCell, evSorted, dloss, gradOpacity,
         gradFull;
     // Host gradient outputs: the split arrays on the device, then pinned.
     DevMem gradStage, gradHost;
@@ -372,7 +373,7 @@ struct pale_handle {
     float4* outLdr = nullptr;
     // Batched views (pale_render_views): descriptors of the current batch,
     // the framebuffers of all views, the captured graph of a batch's rounds.
-    DevMem bTiles, bSegs, bRuns, bHdr, bCams, bSegFirst, bSegEnd, bGroups, bGroupSegs, viewsFb, viewsLdr;
+    DevMem bTiles, bSegs, bRuns, bHdr, bCams, bSegFirst[2], bSegEnd, bGroups, bGroupSegs, viewsFb, viewsLdr;
     pale_batch_tuning tune{};
     hipGraphExec_t bGraph = nullptr;
     std::vector<uint8_t> bGraphKey;
@@ -595,7 +596,6 @@ struct pale_handle {
     // PathTracer::setScene (PathTracer.cpp:22-53): queue capacity, photon map
     // and grid (configured once, on the first call).
     void setScene() {
-        ensureQueues(nextPow2(std::max(S.photons, 1u)));
         if (!gridConfigured) {
             // allocatePhotonMap (PathTracer.cpp:123-157): photons * passes *
             // bounces, clamped to 10 GiB of 64-byte reference records.
@@ -643,7 +643,10 @@ struct pale_handle {
             HIPCHECK(hipStreamSynchronize(stream));
             gridConfigured = true;
         }
+        ensureQueues(nextPow2(std::max(S.photons, 1u)));
     }
+    HitArrays hits() const { return HitArrays{hitPos.as<float4>(), hitPrim.as<uint32_t>()}; }
+    TileStates tileStates() const { return TileStates{tileState.as<unsigned long long>()}; }
 
     // Buffer sizing runs either for real (Allocate) or as a dry run that
     // adds up the growth a request would cause (Probe: HBM admission).
@@ -681,17 +684,19 @@ struct pale_handle {
         for (int k = 0; k < 3; ++k) {
             a(qA[k], (size_t)cap * sizeof(float4));
             a(qB[k], (size_t)cap * sizeof(float4));
-            a(stg[k], (size_t)cap * sizeof(float4));
         }
-        a(extFlags, cap);
-        a(depStg[0], (size_t)cap * sizeof(float4));
-        a(depStg[1], (size_t)cap * sizeof(float4));
-        a(depStg[2], (size_t)cap * sizeof(float));
-        a(depFlags, cap);
-        a(tiles, ((size_t)cap / kTile + 4) * sizeof(uint32_t));
-        a(counts, 16 * sizeof(uint32_t));
-        a(resvAttempt, (size_t)cap * sizeof(uint32_t));
-        a(resvSlot, (size_t)cap * sizeof(uint32_t));
+        a(hitPos, (size_t)cap * sizeof(float4));
+        a(hitPrim, (size_t)cap * sizeof(uint32_t));
+        a(tileState, ((size_t)cap / kTile + 1) * sizeof(uint64_t));
+        if (reservoirOn) {
+            a(depStg[0], (size_t)cap * sizeof(float4));
+            a(depStg[1], (size_t)cap * sizeof(float4));
+            a(depStg[2], (size_t)cap * sizeof(float));
+            a(depFlags, cap);
+            a(tiles, ((size_t)cap / kTile + 4) * sizeof(uint32_t));
+            a(resvAttempt, (size_t)cap * sizeof(uint32_t));
+            a(resvSlot, (size_t)cap * sizeof(uint32_t));
+        }
         if (const size_t sb = traceSpillBytes(cap)) a(traceSpill, sb);
         if (!A::kDry) queueCap = cap;
     }
@@ -714,17 +719,13 @@ struct pale_handle {
         // one cell-sorted transport launch.
         const uint32_t pool = (uint32_t)std::min<uint64_t>((uint64_t)npx * 24u, 1u << 28);
         const int arrays = eventRays() ? 6 : 4;
-        for (int k = 0; k < arrays; ++k) {
-            a(evStg[k], (size_t)npx * sizeof(float4));
-            a(evCmp[k], (size_t)pool * sizeof(float4));
-        }
+        for (int k = 0; k < arrays; ++k) a(evCmp[k], (size_t)pool * sizeof(float4));
         if (S.full_gradients) {
             a(pend3, (size_t)npx * sizeof(float4));
             a(pend4, (size_t)npx * sizeof(float4));
         }
         a(evCell, (size_t)pool * 4);
         a(evSorted, (size_t)pool * 4);
-        a(evFlags, npx);
         if (!A::kDry) {
             poolCap = pool;
             if (eventRays()) adjFull = true;
@@ -781,10 +782,9 @@ struct pale_handle {
     std::vector<DevMem*> viewBuffers() {
         std::vector<DevMem*> v = {&pxOt,    &pxDl,    &pxCs,    &pxCnt,  &pxOff, &pxTiles, &entQa,  &entQb,
                                   &entQs, &entContrib, &entPos, &entCell, &entSorted, &viewFb, &viewLdr, &pend0,
-                                  &pend1,   &pend2,   &pend3,   &pend4,  &evCell, &evSorted, &evFlags, &dloss,
-                                  &bTiles,  &bSegs,   &bRuns,   &bHdr,   &bCams, &bSegFirst, &viewsFb, &viewsLdr};
+                                  &pend1,   &pend2,   &pend3,   &pend4,  &evCell, &evSorted, &dloss,
+                                  &bTiles,  &bSegs,   &bRuns,   &bHdr,   &bCams, &bSegFirst[0], &viewsFb, &viewsLdr};
         for (int k = 0; k < 6; ++k) {
-            v.push_back(&evStg[k]);
             v.push_back(&evCmp[k]);
         }
         return v;
@@ -934,7 +934,7 @@ struct pale_handle {
         camRounds = 0;
         if (S.batch_passes && S.gather_passes > 0 && !camIdx.empty()) {
             // Every camera draws one seed from the table where the photon
-            // stage left the cursor (k_seed_next); its passes use it
+            // stage left the cursor (k_photon_next); its passes use it
             // (+ pass when decorrelated).  All passes of all cameras run as
             // batches; each image equals the pass-by-pass one.
             DevState hs{};
@@ -969,7 +969,7 @@ struct pale_handle {
             const HostCamera& c = cams[camIdx[k]];
             const uint32_t npx = c.W * c.H;
             ensureCamera(npx);
-            launchSeedNext(stream, st, seedTable.as<uint32_t>(), tlen, -1);
+            launchPhotonNext(stream, st, seedTable.as<uint32_t>(), tlen, kNextDraw, 0u, tileStates(), 0u);
             launchFillF(stream, fb[camIdx[k]].as<float>(), npx * 4, 0.0f);
             const DevCamera dc = devCam(c);
             for (uint32_t pass = 0; pass < S.gather_passes; ++pass)
@@ -1007,41 +1007,29 @@ struct pale_handle {
         DevState* st = this->st();
         const uint32_t emitted = S.photons * S.forward_passes;
         const float invEmitted = 1.0f / (float)emitted;
-        uint32_t* emitCount = counts.as<uint32_t>();
-        launchFill(stream, emitCount, 1, P);
-        uint32_t* qCount = stField(offsetof(DevState, qCount));
-        uint32_t* extTotal = stField(offsetof(DevState, extTotal));
-        uint32_t* depTotal = stField(offsetof(DevState, depTotal));
-        uint32_t* photonCount = stField(offsetof(DevState, photonCount));
         const Reservoir rs{reservoirOn ? resvAttempt.as<uint32_t>() : nullptr, resvSlot.as<uint32_t>(),
                            resvOwner.as<uint32_t>(), photonCap};
         if (reservoirOn) launchFill(stream, resvOwner.as<uint32_t>(), photonCap, 0u);
+        const TileStates ts = tileStates();
+        const uint32_t resvCap = reservoirOn ? photonCap : 0u;
+        const uint32_t* table = seedTable.as<uint32_t>();
         DevMem* in = qA;
         DevMem* out = qB;
         for (uint32_t pass = 0; pass < S.forward_passes; ++pass) {
-            launchSeedNext(stream, st, seedTable.as<uint32_t>(), tlen, -1);
-            launchEmit(stream, scene, st, P, invEmitted, rq(stg), extFlags.as<uint8_t>());
-            launchCompactRays(stream, extFlags.as<uint8_t>(), emitCount, P, tiles.as<uint32_t>(), extTotal, rq(stg),
-                              rq(in), queueCap);
-            launchSetQueue(stream, st, extTotal);
+            launchPhotonNext(stream, st, table, tlen, kNextDraw, resvCap, ts, P);
+            launchEmit(stream, scene, st, P, invEmitted, rq(in), queueCap, ts);
             for (uint32_t b = 0; b < S.bounces; ++b) {
-                launchSeedNext(stream, st, seedTable.as<uint32_t>(), tlen, (int)b);
+                launchPhotonNext(stream, st, table, tlen, (int)b, resvCap, ts, P);
                 const size_t te = tBegin(kTPhoton);
-                launchPhotonTrace(stream, scene, st, P, rq(in), rq(stg), extFlags.as<uint8_t>(),
-                                  pa(depStg[0], depStg[1], depStg[2]), depFlags.as<uint8_t>(),
-                                  withTraceSpill(tp(), P), rs, tiles.as<uint32_t>(), countWork);
+                launchQueueTrace(stream, scene, st, P, rq(in), hits(), withTraceSpill(tp(), P), false, countWork);
                 tEnd(te);
-                launchCompactRays(stream, extFlags.as<uint8_t>(), qCount, P, tiles.as<uint32_t>(), extTotal, rq(stg),
-                                  rq(out), queueCap);
-                launchCompactPhotons(stream, depFlags.as<uint8_t>(), qCount, P, tiles.as<uint32_t>(), depTotal,
-                                     photonCount, pa(depStg[0], depStg[1], depStg[2]),
-                                     pa(rawPosPow, rawDirPow, rawPowZ), photonCap);
-                launchReservoirWrite(stream, st, P, rs, pa(depStg[0], depStg[1], depStg[2]),
-                                     pa(rawPosPow, rawDirPow, rawPowZ));
-                launchFinishPhotonBounce(stream, st, photonCap);
+                launchPhotonShade(stream, scene, st, P, rq(in), hits(), rq(out), queueCap,
+                                  pa(rawPosPow, rawDirPow, rawPowZ), pa(depStg[0], depStg[1], depStg[2]), tp(), rs,
+                                  depFlags.as<uint8_t>(), tiles.as<uint32_t>(), ts);
                 std::swap(in, out);
             }
         }
+        launchPhotonNext(stream, st, table, tlen, kNextEnd, resvCap, ts, 0u);
         // buildPhotonCellRangesAndOrdering (PrimalKernels.cpp:1007-1018)
         const size_t tg = tBegin(kTGrid);
         launchBuildGrid(stream, grid, st, photonCap, pa(rawPosPow, rawDirPow, rawPowZ),
@@ -1394,6 +1382,7 @@ struct pale_handle {
         h.events = 0;
         h.qCount = 0;
         h.evPool = 0;
+        h.evTotal = 0;
         HIPCHECK(hipMemcpyAsync(state.p, &h, sizeof(DevState), hipMemcpyHostToDevice, stream));
         HIPCHECK(hipStreamSynchronize(stream));
         dloss.reserve(std::max<size_t>(off.back(), 1) * sizeof(float));
@@ -1457,7 +1446,8 @@ struct pale_handle {
         a(bSegs, plan.maxSegs * sizeof(BatchSeg));
         a(bRuns, sizeof(BatchRun));
         a(bHdr, sizeof(BatchHeader));
-        a(bSegFirst, plan.maxSegs * sizeof(uint32_t));
+        a(bSegFirst[0], plan.maxSegs * sizeof(uint32_t));
+        a(bSegFirst[1], plan.maxSegs * sizeof(uint32_t));
         a(bSegEnd, plan.maxSegs * sizeof(uint32_t));
         a(bGroups, std::max<size_t>(nViews, 1) * sizeof(uint4));
         a(bGroupSegs, plan.maxSegs * sizeof(uint32_t));
@@ -1533,10 +1523,9 @@ struct pale_handle {
         upload(stream, bCams, dcs);
         beginBackward(plan.off, src, srcOnDevice);
         DevState* st = this->st();
-        uint32_t* qCount = stField(offsetof(DevState, qCount));
-        uint32_t* extTotal = stField(offsetof(DevState, extTotal));
         const BatchDesc bd = batchDesc();
-        TraceParams tpb = tp(1.0f, bSegs.as<BatchSeg>(), bSegFirst.as<uint32_t>());
+        const TileStates ts = tileStates();
+        TraceParams tpb = tp(1.0f, bSegs.as<BatchSeg>());
         tpb.segEnd = bSegEnd.as<uint32_t>();
         tpb.groups = bGroups.as<uint4>();
         tpb.groupSegs = bGroupSegs.as<uint32_t>();
@@ -1567,26 +1556,30 @@ struct pale_handle {
             const uint32_t nr = b.hdr.nSlots;
             DevMem* in = qA;
             DevMem* out = qB;
-            launchAdjRaygenBatch(stream, bd, b.hdr.nTiles, dloss.as<float>(), rq(in), pend, st);
+            uint32_t *segs = bSegFirst[0].as<uint32_t>(), *segsNext = bSegFirst[1].as<uint32_t>();
+            auto next = [&](int bounce) {
+                launchAdjNext(stream, st, bounce, poolCap, ts, nr, segs, bSegEnd.as<uint32_t>(), segsNext, b.hdr.nSegs,
+                              bGroups.as<uint4>(), tpb.nGroups, bGroupSegs.as<uint32_t>());
+            };
+            launchAdjRaygenBatch(stream, bd, b.hdr.nTiles, dloss.as<float>(), rq(in), pend, st, segs);
             for (uint32_t k = 0; k < S.adjoint_bounces; ++k) {
+                next((int)k);
                 if (pooledBound + nr > poolCap) {
                     flushEvents();
                     pooledBound = 0;
                 }
-                launchSegFirst(stream, st, nr, rq(in), bSegFirst.as<uint32_t>(), bSegEnd.as<uint32_t>(), b.hdr.nSegs,
-                               bGroups.as<uint4>(), tpb.nGroups, bGroupSegs.as<uint32_t>());
+                tpb.segFirst = segs;
+                const TraceParams t = withTraceSpill(tpb, nr);
                 const size_t ta = tBegin(kTAdjTrace);
-                launchAdjTrace(stream, scene, st, nr, k, rq(in), rq(stg), extFlags.as<uint8_t>(), ea(evStg),
-                               evFlags.as<uint8_t>(), pend, withTraceSpill(tpb, nr), countWork);
+                launchQueueTrace(stream, scene, st, nr, rq(in), hits(), t, true, countWork);
                 tEnd(ta);
-                launchCompactEvents(stream, evFlags.as<uint8_t>(), qCount, nr, tiles.as<uint32_t>(), st, ea(evStg),
-                                    ea(evCmp), poolCap);
+                launchAdjShade(stream, scene, st, nr, k, rq(in), hits(), rq(out), queueCap, ea(evCmp), poolCap, pend, t,
+                               segsNext, ts);
                 pooledBound += nr;
-                launchCompactRays(stream, extFlags.as<uint8_t>(), qCount, nr, tiles.as<uint32_t>(), extTotal,
-                                  rq(stg), rq(out), queueCap);
-                launchSetQueue(stream, st, extTotal);
+                std::swap(segs, segsNext);
                 std::swap(in, out);
             }
+            next(kNextEnd);
         }
         if (pooledBound) flushEvents();
         batchCount = (uint32_t)batches.size();
@@ -1616,8 +1609,7 @@ struct pale_handle {
         for (size_t k = 0; k < camList.size(); ++k) off[k + 1] = off[k] + (size_t)camList[k]->W * camList[k]->H * 3;
         beginBackward(off, src, srcOnDevice);
         DevState* st = this->st();
-        uint32_t* qCount = stField(offsetof(DevState, qCount));
-        uint32_t* extTotal = stField(offsetof(DevState, extTotal));
+        const TileStates ts = tileStates();
         const float invSpp = 1.0f / (float)samples;
         // launchAdjointTransportKernel (AdjointKernels.cpp:389-509) over the
         // pooled events of several bounces, in grid-cell order.  Gradients
@@ -1639,22 +1631,24 @@ struct pale_handle {
                 DevMem* in = qA;
                 DevMem* out = qB;
                 launchAdjRaygen(stream, dc, dloss.as<float>() + off[k], rq(in), pend, st, adjointSeed(spp));
+                auto next = [&](int bounce) {
+                    launchAdjNext(stream, st, bounce, poolCap, ts, npx, nullptr, nullptr, nullptr, 0u, nullptr, 0u, nullptr);
+                };
                 for (uint32_t b = 0; b < S.adjoint_bounces; ++b) {
+                    next((int)b);
                     if (pooledBound + npx > poolCap) flush();
-                    const size_t ta = tBegin(kTAdjTrace);
                     TraceParams tpc = tp(invSpp, nullptr, nullptr, adjointSeed(spp));
                     tpc.debugBase = (uint32_t)(off[k] / 3);
-                    launchAdjTrace(stream, scene, st, npx, b, rq(in), rq(stg), extFlags.as<uint8_t>(), ea(evStg),
-                                   evFlags.as<uint8_t>(), pend, withTraceSpill(tpc, npx), countWork);
+                    tpc = withTraceSpill(tpc, npx);
+                    const size_t ta = tBegin(kTAdjTrace);
+                    launchQueueTrace(stream, scene, st, npx, rq(in), hits(), tpc, true, countWork);
                     tEnd(ta);
-                    launchCompactEvents(stream, evFlags.as<uint8_t>(), qCount, npx, tiles.as<uint32_t>(), st,
-                                        ea(evStg), ea(evCmp), poolCap);
+                    launchAdjShade(stream, scene, st, npx, b, rq(in), hits(), rq(out), queueCap, ea(evCmp), poolCap,
+                                   pend, tpc, nullptr, ts);
                     pooledBound += npx;
-                    launchCompactRays(stream, extFlags.as<uint8_t>(), qCount, npx, tiles.as<uint32_t>(), extTotal,
-                                      rq(stg), rq(out), queueCap);
-                    launchSetQueue(stream, st, extTotal);
                     std::swap(in, out);
                 }
+                next(kNextEnd);
             }
         }
         flush();
@@ -1675,30 +1669,27 @@ struct pale_handle {
             p += (bytes + 255) & ~(size_t)255;
             return r;
         };
-        float4* q[9];
+        float4* q[7];
         for (float4*& x : q) x = reinterpret_cast<float4*>(take(M * sizeof(float4)));
-        uint8_t* ext = reinterpret_cast<uint8_t*>(take(M));
-        uint8_t* evf = reinterpret_cast<uint8_t*>(take(M));
+        const HitArrays hit{q[6], reinterpret_cast<uint32_t*>(take(M * sizeof(uint32_t)))};
+        const TileStates ts{reinterpret_cast<unsigned long long*>(take((M / kTile + 1) * sizeof(uint64_t)))};
         const PendingArrays pend{reinterpret_cast<float4*>(take(M * sizeof(float4))),
                                  reinterpret_cast<float4*>(take(M * sizeof(float4))),
                                  reinterpret_cast<uint2*>(take(M * sizeof(uint2))), nullptr, nullptr};
-        float4* e[8];
+        float4* e[4];
         for (float4*& x : e) x = reinterpret_cast<float4*>(take(M * sizeof(float4)));
-        const EventArrays evS{e[0], e[1], e[2], e[3], nullptr, nullptr};
-        const EventArrays evP{e[4], e[5], e[6], e[7], nullptr, nullptr};
+        const EventArrays evP{e[0], e[1], e[2], e[3], nullptr, nullptr};
         uint32_t* order = reinterpret_cast<uint32_t*>(take(M * sizeof(uint32_t)));
-        uint32_t* tl = reinterpret_cast<uint32_t*>(take((M / kTile + 4) * sizeof(uint32_t)));
         if ((size_t)(p - scratchBase) > kNoAllocScratchBytes)
             throw StatusError(PALE_ERR_INTERNAL, "no-allocation scratch layout exceeds the array");
-        const RayQueue A{q[0], q[1], q[2]}, B{q[3], q[4], q[5]}, stgq{q[6], q[7], q[8]};
+        const RayQueue A{q[0], q[1], q[2]}, B{q[3], q[4], q[5]};
         DevState* st = this->st();
-        uint32_t* qCount = stField(offsetof(DevState, qCount));
-        uint32_t* extTotal = stField(offsetof(DevState, extTotal));
         uint32_t* evPool = stField(offsetof(DevState, evPool));
         // Fill kernels, not hipMemsetAsync: the calls stay capturable.
         launchFillF(stream, gradDev, N, 0.0f);
-        launchFill(stream, qCount, 1, 0u);
+        launchFill(stream, stField(offsetof(DevState, qCount)), 1, 0u);
         launchFill(stream, evPool, 1, 0u);
+        launchFill(stream, stField(offsetof(DevState, evTotal)), 1, 0u);
         launchIota(stream, order, npx);
         const DevCamera dc = devCam(c);
         const float invSpp = 1.0f / (float)samples;
@@ -1708,13 +1699,16 @@ struct pale_handle {
             TraceParams t = tp(invSpp, nullptr, nullptr, adjointSeed(spp));
             t.fullGradients = 0;
             t.debug = 0;
+            auto next = [&](int bounce) {
+                launchAdjNext(stream, st, bounce, npx, ts, npx, nullptr, nullptr, nullptr, 0u, nullptr, 0u, nullptr);
+            };
+            next(0);
             for (uint32_t b = 0; b < S.adjoint_bounces; ++b) {
-                launchAdjTrace(stream, scene, st, npx, b, in, stgq, ext, evS, evf, pend, t, false);
-                launchCompactEvents(stream, evf, qCount, npx, tl, st, evS, evP, npx);
+                launchQueueTrace(stream, scene, st, npx, in, hit, t, true, false);
+                launchAdjShade(stream, scene, st, npx, b, in, hit, out, (uint32_t)M, evP, npx, pend, t, nullptr, ts);
+                next(b + 1 < S.adjoint_bounces ? (int)b + 1 : kNextEnd);
                 launchAdjTransport(stream, scene, devGrid(), st, npx, evP, order, gradDev, nullptr, nullptr, false);
                 launchFill(stream, evPool, 1, 0u);
-                launchCompactRays(stream, ext, qCount, npx, tl, extTotal, stgq, out, (uint32_t)M);
-                launchSetQueue(stream, st, extTotal);
                 std::swap(in, out);
             }
         }

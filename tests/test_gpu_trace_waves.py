@@ -162,3 +162,19 @@ def test_quad_nodes_over_tree_shapes(n):
     for k in ("instance", "primitive", "t", "position"):
         assert np.array_equal(a[k], b[k]), k
     _check(gpu, orc)
+
+
+@pytest.mark.parametrize("photons", [1, 1023, 1024, 1025, 65 * 1024 - 1, 70 * 1024 + 3])
+@pytest.mark.parametrize("capacity", [0, 900])
+def test_queue_compaction_tiles(photons, capacity):
+    """Survivors, deposits and gradient events keep queue order across the
+    tiles of the compaction: one tile, a tile's edge, more tiles than one look
+    back window, queues that run empty before the last bounce, and a photon map
+    that fills in the middle of a tile (the reservoir's draws follow)."""
+    pts = scene.uniform_surfels(3000, seed=2, scale_lo=0.03, scale_hi=0.1)[0]
+    spec = scene.SceneSpec([scene.light_quad()], [scene.default_camera(300, 230)], pts,
+                           dict(photons=photons, bounces=12, forward_passes=2, gather_passes=1, adjoint_bounces=9,
+                                adjoint_passes=2, seed=3, gather_radius=0.05, spp_decorrelate=1,
+                                photon_map_capacity=capacity))
+    gpu, orc = _pair(spec, {})
+    _check(gpu, orc, backward=photons == 70 * 1024 + 3)

@@ -15,6 +15,10 @@ constexpr uint32_t kTraceBlock = kStackStride;  // threads per traversal workgro
 // XCD under round-robin dispatch) so each XCD's L2 serves one part of the
 // image, and moves on when its region is used up.
 constexpr uint32_t kTraceRegions = 8;
+// The regions' counters are 256 bytes apart: atomics of the whole device on one
+// cache line take about 11 ns each, one after the other.
+constexpr uint32_t kCursorStride = 64;
+constexpr uint32_t kCursorWords = kTraceRegions * kCursorStride;
 
 // Device-side progress of one render call.  Counts live on the device so the
 // whole forward or backward pass runs without host round trips.
@@ -32,12 +36,13 @@ struct DevState {
     uint32_t evPool;       // adjoint events waiting for the transport
     uint32_t resv;         // this bounce may pass the photon capacity
     uint32_t bigCells;     // photon cells too large for the per-wave sort
-    uint32_t traceNext;    // next ray of the queue to trace (photon and adjoint traces)
+    uint32_t pad32;
     unsigned long long photonQ, gatherQ, adjointQ, deposits, events, pad;
     // Counting mode, per kernel class (photon, gather, adjoint): popped
     // nodes, AABB tests, primitive tests, gathers, gather cells, non-empty
     // cells, photons scanned.
     unsigned long long work[3][8];
+    uint32_t traceNext[kCursorWords];  // claims of the running photon or adjoint trace, per region
 };
 
 enum : int { kWorkPhoton = 0, kWorkGather = 1, kWorkAdjoint = 2 };

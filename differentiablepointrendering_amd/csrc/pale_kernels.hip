@@ -131,11 +131,11 @@ __global__ void k_iota(uint32_t* p, uint32_t n) {
 __global__ __launch_bounds__(256) void k_photon_next(DevState* st, const uint32_t* table, uint32_t len, int bounce,
                                                      uint32_t resvCap, TileStates ts, uint32_t tiles) {
     for (uint32_t k = threadIdx.x; k < tiles; k += blockDim.x) ts.state[k] = 0ull;
+    if (threadIdx.x < kTraceRegions) st->traceNext[threadIdx.x * kCursorStride] = 0u;
     if (threadIdx.x != 0) return;
     const uint32_t deposits = st->photonCount + st->depTotal;
     st->photonCount = deposits;
     st->depTotal = 0;
-    st->traceNext = 0;
     st->ticket = 0;
     if (bounce == kNextEnd) return;
     if (bounce >= 0) {
@@ -161,12 +161,12 @@ __global__ __launch_bounds__(256) void k_adj_next(DevState* st, int bounce, uint
                                                   uint32_t* segNext, uint32_t nSegs, uint4* groups, uint32_t nGroups,
                                                   const uint32_t* groupSegs) {
     for (uint32_t k = threadIdx.x; k < tiles; k += blockDim.x) ts.state[k] = 0ull;
+    if (threadIdx.x < kTraceRegions) st->traceNext[threadIdx.x * kCursorStride] = 0u;
     __shared__ uint32_t sQueue;
     if (threadIdx.x == 0) {
         const uint32_t n = st->evPool + st->evTotal;
         st->evPool = n < poolCap ? n : poolCap;
         st->evTotal = 0;
-        st->traceNext = 0;
         st->ticket = 0;
         if (bounce > 0) st->qCount = st->extTotal;
         sQueue = st->qCount;
@@ -315,15 +315,31 @@ __device__ __forceinline__ TileOffset tileOffsets(TileStates ts, uint32_t tile, 
 }
 
 // ------------------------------------------------------- queue traces --
-// Rays of a queue for the waves of a persistent grid: a wave claims 64
-// consecutive rays at a time and gives them to its lanes as they fall idle.
+// Rays of a queue for the waves of a persistent grid: 64 consecutive rays (a
+// unit) at a time, given to the wave's lanes as they fall idle.  A wave starts
+// with the unit at its own place in the grid; the units after those go round
+// the regions, and the waves of a region claim them from its counter.  With one
+// counter and every unit claimed from it, the claims bounded the trace: 36
+// bounces of 1M photons in a 100k-surfel room 18.4 ms, with the first units
+// given 15.7 ms, with a counter per region 15.1 ms; 6 adjoint bounces of 167k
+// rays in a 775-surfel scene 340 us against 170 us.
 struct QueueCursor {
-    uint32_t* next;             // shared by the grid, zero at the start of a launch
-    uint32_t end;               // rays to hand out
-    uint32_t at = 0, to = 0;    // the wave's claimed, untaken rays
-    bool empty = false;
+    uint32_t* next;      // claims of the region, zero at the start of a launch
+    uint32_t end;        // rays to hand out
+    uint32_t regions, region, own;  // own: units that the waves start with
+    uint32_t at, to;     // the wave's untaken rays
+    bool empty;
 
-    __device__ QueueCursor(uint32_t* n, uint32_t e) : next(n), end(e) {}
+    __device__ QueueCursor(uint32_t* n, uint32_t e) : end(e) {
+        const uint32_t waves = blockDim.x / 64u;
+        regions = min(kTraceRegions, gridDim.x);
+        region = blockIdx.x % regions;
+        next = n + region * kCursorStride;
+        own = gridDim.x * waves;
+        at = (blockIdx.x * waves + __builtin_amdgcn_readfirstlane(threadIdx.x / 64u)) * 64u;
+        to = min(at + 64u, end);
+        empty = at >= end;
+    }
     // Every lane of the wave calls it; false: no ray for this lane now (t
     // stays as it is).
     __device__ __forceinline__ bool take(bool want, uint32_t& t) {
@@ -331,16 +347,20 @@ struct QueueCursor {
         if (!need || empty) return false;
         const uint32_t lane = laneId();
         if (at >= to) {
-            const uint32_t leader = (uint32_t)__ffsll((long long)need) - 1u;
-            uint32_t base = 0;
-            if (lane == leader) base = atomicAdd(next, 64u);
-            base = __builtin_amdgcn_readlane(base, leader);
+            uint64_t base = (uint64_t)own * 64u;
+            if (base < end) {
+                const uint32_t leader = (uint32_t)__ffsll((long long)need) - 1u;
+                uint32_t claim = 0;
+                if (lane == leader) claim = atomicAdd(next, 1u);
+                claim = __builtin_amdgcn_readlane(claim, leader);
+                base += ((uint64_t)claim * regions + region) * 64u;
+            }
             if (base >= end) {
                 empty = true;
                 return false;
             }
-            at = base;
-            to = min(base + 64u, end);
+            at = (uint32_t)base;
+            to = min(at + 64u, end);
         }
         const uint32_t mine = at + (uint32_t)__popcll(need & ((1ull << lane) - 1ull));
         const bool got = want && mine < to;
@@ -454,7 +474,7 @@ __device__ __forceinline__ void queueTrace(const DevScene& S, DevState* st, cons
     }
     if (blockIdx.x == 0 && threadIdx.x == 0)
         atomicAdd(kAdjoint ? &st->adjointQ : &st->photonQ, (unsigned long long)n);
-    QueueJob<kCount, kAdjoint> job{in, hits, tp, QueueCursor(&st->traceNext, end)};
+    QueueJob<kCount, kAdjoint> job{in, hits, tp, QueueCursor(st->traceNext, end)};
     if (kTopLds)
         traceWave<kCount>(S, sTop, stk, job);
     else
@@ -983,7 +1003,8 @@ struct CameraJob {
     uint32_t* cursor;
     uint32_t tiles, region;
     uint32_t emptyRegions = 0;
-    uint32_t chunkNext = 0, chunkEnd = 0;  // the wave's claimed, untaken slots
+    uint32_t chunkNext = 0, chunkEnd = 0;  // the wave's untaken slots
+    bool begun = false;                    // the wave has taken its first unit
     bool exhausted = false;
     // Entries are claimed entClaim at a time: one claim per entry append made
     // every wave wait for an atomic on the one counter of the grid, and with
@@ -1019,13 +1040,33 @@ struct CameraJob {
             // longer, 28 % with decorrelated passes).
             if (chunkNext >= chunkEnd) {
                 // Slots [lo, hi) of the current region; cursor[region] counts
-                // the slots drawn from it this round.
+                // the slots claimed from it this round.
                 const uint32_t lo = (uint32_t)(((uint64_t)region * tiles) / kTraceRegions) * 64u;
                 const uint32_t hi = (uint32_t)(((uint64_t)(region + 1u) * tiles) / kTraceRegions) * 64u;
-                const uint32_t leader = (uint32_t)__ffsll((long long)need) - 1u;
-                uint32_t base = 0;
-                if (lane == leader) base = lo + atomicAdd(cursor + region, kWalkUnit);
-                base = __builtin_amdgcn_readlane(base, leader);
+                // The first units are the waves' own by their place in the
+                // grid; after them a region's counter is read before it is
+                // advanced, as each wave finds all regions used up once
+                // (QueueCursor has what claims cost; with the waves' first
+                // entries given as well, 16 passes of 155x130 on 1.1k surfels
+                // 580 -> 174 us, nothing at 800x800 on 1M surfels).
+                const uint32_t waves = kTraceBlock / 64u;
+                uint32_t base;
+                if (!begun) {
+                    begun = true;
+                    base = lo + ((blockIdx.x / kTraceRegions) * waves + __builtin_amdgcn_readfirstlane(threadIdx.x / 64u)) *
+                                    kWalkUnit;
+                } else {
+                    const uint32_t blocks = (gridDim.x + kTraceRegions - 1u - region) / kTraceRegions;
+                    base = lo + blocks * waves * kWalkUnit;
+                    if (base < hi)
+                        base += __builtin_amdgcn_readfirstlane(
+                            *reinterpret_cast<volatile const uint32_t*>(cursor + region * kCursorStride));
+                    if (base < hi) {
+                        const uint32_t leader = (uint32_t)__ffsll((long long)need) - 1u;
+                        if (lane == leader) base = lo + blocks * waves * kWalkUnit + atomicAdd(cursor + region * kCursorStride, kWalkUnit);
+                        base = __builtin_amdgcn_readlane(base, leader);
+                    }
+                }
                 if (base >= hi) {
                     // Used up (it stays so): the next region, done after all.
                     if (++emptyRegions == kTraceRegions) exhausted = true;
@@ -1112,16 +1153,34 @@ struct CameraJob {
     }
 };
 
+// Entries that a wave of the layer walk claims at a time: at most an eighth of
+// the buffer is claimed ahead; 0 (below 64): what it appends.  Else every wave
+// starts with kEntryOwn entries at its place in the grid.
+constexpr uint32_t kEntryOwn = 64;
+__host__ __device__ __forceinline__ uint32_t entryClaim(uint32_t cap, uint32_t waves) {
+    const uint32_t a = cap / (8u * waves), share = a < kEntryClaim ? a : kEntryClaim;
+    return share < kEntryOwn ? 0u : share;
+}
+// Start of a round of the layer walk.
+__global__ void k_walk_begin(DevState* st, uint32_t* cursor, uint32_t entries) {
+    if (threadIdx.x < kTraceRegions) cursor[threadIdx.x * kCursorStride] = 0u;
+    if (threadIdx.x == 0) {
+        st->entries = entries;
+        st->overflow = 0u;
+    }
+}
+
 template <bool kCount, typename Map, typename Top>
 __device__ __forceinline__ void camTrace(const DevScene& S, const Top& top, DevState* st, const Map& map,
                                          const PixelArrays& px, const EntryArrays& ent, uint32_t cap, uint32_t* cursor,
                                          const LaneStack& stk) {
     CameraJob<kCount, Map, Top> job{S, top, st, map, px, ent, cap, cursor, map.slots() >> 6, blockIdx.x % kTraceRegions};
-    // At most an eighth of the buffer is claimed ahead; below 64 entries a
-    // wave claims what it appends.
     const uint32_t waves = gridDim.x * (kTraceBlock / 64u);
-    const uint32_t share = min(cap / (8u * waves), kEntryClaim);
-    job.entClaim = share < 64u ? 0u : share;
+    job.entClaim = entryClaim(cap, waves);
+    if (job.entClaim) {
+        job.entNext = (blockIdx.x * (kTraceBlock / 64u) + threadIdx.x / 64u) * kEntryOwn;
+        job.entEnd = job.entNext + kEntryOwn;
+    }
     traceWave<kCount>(S, top, stk, job);
     job.leaveHoles();
     if (laneId() == 0 && job.layers) atomicAdd(&st->gatherQ, (unsigned long long)job.layers);
@@ -2112,29 +2171,29 @@ size_t walkSpillBytes(const DevScene& S, uint32_t inLds) {
     return (size_t)(S.stackDepth - inLds) * grid * kTraceBlock * sizeof(uint2);
 }
 
-void launchCamTrace(hipStream_t s, const DevScene& S, DevState* st, uint32_t npx, uint32_t width, PixelArrays px,
-                    EntryArrays ent, uint32_t cap, uint32_t* cursor, uint2* spill, uint32_t inLds, bool count) {
-    if (!npx) return;
+// A round of the layer walk over `slots` slots, on `fraction` of the lanes that
+// the device holds.
+template <typename Map>
+static void walkRound(hipStream_t s, const DevScene& S, DevState* st, const Map& map, uint32_t slots, PixelArrays px,
+                      EntryArrays ent, uint32_t cap, uint32_t* cursor, uint2* spill, uint32_t inLds, float fraction,
+                      bool count) {
     inLds = std::max(1u, inLds);
     if (S.stackDepth <= inLds) spill = nullptr;
     const size_t lds = walkLdsBytes(S, spill, inLds);
-    const ImageMap map{width, npx / width, (width + 7u) / 8u};
     const bool top = topFitsLds(S);
-    if (count) {
-        const uint32_t g = min(top ? camTraceGrid<true, ImageMap, true>(lds) : camTraceGrid<true, ImageMap, false>(lds),
-                               blocks(npx, kTraceBlock));
-        if (top)
-            k_cam_trace<true, ImageMap, true><<<g, kTraceBlock, lds, s>>>(S, st, map, px, ent, cap, cursor, spill, inLds);
-        else
-            k_cam_trace<true, ImageMap, false><<<g, kTraceBlock, lds, s>>>(S, st, map, px, ent, cap, cursor, spill, inLds);
-    } else {
-        const uint32_t g = min(top ? camTraceGrid<false, ImageMap, true>(lds) : camTraceGrid<false, ImageMap, false>(lds),
-                               blocks(npx, kTraceBlock));
-        if (top)
-            k_cam_trace<false, ImageMap, true><<<g, kTraceBlock, lds, s>>>(S, st, map, px, ent, cap, cursor, spill, inLds);
-        else
-            k_cam_trace<false, ImageMap, false><<<g, kTraceBlock, lds, s>>>(S, st, map, px, ent, cap, cursor, spill, inLds);
-    }
+    const auto k = count ? (top ? &k_cam_trace<true, Map, true> : &k_cam_trace<true, Map, false>)
+                         : (top ? &k_cam_trace<false, Map, true> : &k_cam_trace<false, Map, false>);
+    const uint32_t full = traceGrid(reinterpret_cast<const void*>(k), lds);
+    const uint32_t g = min(max(1u, (uint32_t)((float)full * fraction)), blocks(slots, kTraceBlock));
+    const uint32_t waves = g * (kTraceBlock / 64u);
+    k_walk_begin<<<1, 64, 0, s>>>(st, cursor, entryClaim(cap, waves) ? waves * kEntryOwn : 0u);
+    k<<<g, kTraceBlock, lds, s>>>(S, st, map, px, ent, cap, cursor, spill, inLds);
+}
+void launchCamTrace(hipStream_t s, const DevScene& S, DevState* st, uint32_t npx, uint32_t width, PixelArrays px,
+                    EntryArrays ent, uint32_t cap, uint32_t* cursor, uint2* spill, uint32_t inLds, bool count) {
+    if (npx)
+        walkRound(s, S, st, ImageMap{width, npx / width, (width + 7u) / 8u}, npx, px, ent, cap, cursor, spill, inLds,
+                  1.0f, count);
 }
 
 void launchBatchInit(hipStream_t s, BatchDesc b, uint32_t maxTiles, PixelArrays px) {
@@ -2144,27 +2203,9 @@ void launchBatchInit(hipStream_t s, BatchDesc b, uint32_t maxTiles, PixelArrays 
 void launchCamTraceBatch(hipStream_t s, const DevScene& S, DevState* st, BatchDesc b, uint32_t maxSlots,
                          PixelArrays px, EntryArrays ent, uint32_t cap, uint32_t* cursor, uint2* spill,
                          uint32_t inLds, float gridFraction, bool count) {
-    if (!maxSlots) return;
-    inLds = std::max(1u, inLds);
-    if (S.stackDepth <= inLds) spill = nullptr;
-    const size_t lds = walkLdsBytes(S, spill, inLds);
-    const BatchMap map{b.tiles, b.segs, b.hdr};
-    const bool top = topFitsLds(S);
-    if (count) {
-        const uint32_t full = top ? camTraceGrid<true, BatchMap, true>(lds) : camTraceGrid<true, BatchMap, false>(lds);
-        const uint32_t g = min(max(1u, (uint32_t)((float)full * gridFraction)), blocks(maxSlots, kTraceBlock));
-        if (top)
-            k_cam_trace<true, BatchMap, true><<<g, kTraceBlock, lds, s>>>(S, st, map, px, ent, cap, cursor, spill, inLds);
-        else
-            k_cam_trace<true, BatchMap, false><<<g, kTraceBlock, lds, s>>>(S, st, map, px, ent, cap, cursor, spill, inLds);
-    } else {
-        const uint32_t full = top ? camTraceGrid<false, BatchMap, true>(lds) : camTraceGrid<false, BatchMap, false>(lds);
-        const uint32_t g = min(max(1u, (uint32_t)((float)full * gridFraction)), blocks(maxSlots, kTraceBlock));
-        if (top)
-            k_cam_trace<false, BatchMap, true><<<g, kTraceBlock, lds, s>>>(S, st, map, px, ent, cap, cursor, spill, inLds);
-        else
-            k_cam_trace<false, BatchMap, false><<<g, kTraceBlock, lds, s>>>(S, st, map, px, ent, cap, cursor, spill, inLds);
-    }
+    if (maxSlots)
+        walkRound(s, S, st, BatchMap{b.tiles, b.segs, b.hdr}, maxSlots, px, ent, cap, cursor, spill, inLds, gridFraction,
+                  count);
 }
 
 void launchCamCompositeBatch(hipStream_t s, uint32_t maxSlots, const BatchHeader* hdr, PixelArrays px,

@@ -744,7 +744,7 @@ struct pale_handle {
         const uint32_t npx = W * H;
         if (!S.batch_passes) {
             sizeCamera(npx, p);
-            p(cursors, kTraceRegions * sizeof(uint32_t));
+            p(cursors, kCursorWords * sizeof(uint32_t));
             p(viewFb, (size_t)npx * sizeof(float4));
             p(viewLdr, (size_t)npx * sizeof(float4));
             if (adjoint) {
@@ -893,11 +893,8 @@ struct pale_handle {
         const PixelArrays px = pxa();
         const EntryArrays ent = enta();
         const DevGrid G = devGrid();
-        uint32_t* entries = stField(offsetof(DevState, entries));
         launchCamInit(stream, dc, st, pass, decorrelate, px);
         for (uint32_t round = 0;; ++round) {
-            launchFill(stream, entries, 2, 0u);  // entries, overflow
-            launchFill(stream, cursors.as<uint32_t>(), kTraceRegions, 0u);
             const size_t tt = tBegin(kTCamTrace);
             launchCamTrace(stream, scene, st, npx, dc.W, px, ent, entryCap, cursors.as<uint32_t>(), walkSpillPtr(),
                            walkLds(), countWork);
@@ -964,7 +961,7 @@ struct pale_handle {
         }
         DevState* st = this->st();
         const float invSpp = 1.0f / (float)S.gather_passes;
-        cursors.reserve(kTraceRegions * sizeof(uint32_t));
+        cursors.reserve(kCursorWords * sizeof(uint32_t));
         for (size_t k = 0; k < camIdx.size(); ++k) {
             const HostCamera& c = cams[camIdx[k]];
             const uint32_t npx = c.W * c.H;
@@ -1075,8 +1072,6 @@ struct pale_handle {
         const PixelArrays px = pxa();
         const EntryArrays ent = enta();
         const bool count = timed && countWork;
-        launchFill(stream, stField(offsetof(DevState, entries)), 2, 0u);  // entries, overflow
-        launchFill(stream, cursors.as<uint32_t>(), kTraceRegions, 0u);
         const size_t tt = timed ? tBegin(kTCamTrace) : 0;
         launchCamTraceBatch(stream, scene, st(), batchDesc(), maxSlots, px, ent, entryCap, cursors.as<uint32_t>(),
                             walkSpillPtr(), walkLds(), fraction, count);
@@ -1162,7 +1157,7 @@ struct pale_handle {
     void sizeForward(const ForwardPlan& plan, size_t nViews, A& a) {
         // Entries per slot: the tuning's, else the settings' per-pixel budget.
         sizeCamera(std::max(plan.maxSlots, 1u), a, tune.entries_per_slot);
-        a(cursors, kTraceRegions * sizeof(uint32_t));
+        a(cursors, kCursorWords * sizeof(uint32_t));
         a(bTiles, (size_t)std::max(plan.maxTiles, 1u) * sizeof(uint4));
         a(bSegs, plan.maxSegs * sizeof(BatchSeg));
         a(bRuns, plan.maxRuns * sizeof(BatchRun));
@@ -1363,7 +1358,7 @@ struct pale_handle {
         launchFillF(stream, viewFb.as<float>(), npx * 4, 0.0f);
         const DevCamera dc = devCam(c);
         const float invSpp = 1.0f / (float)spp;
-        cursors.reserve(kTraceRegions * sizeof(uint32_t));
+        cursors.reserve(kCursorWords * sizeof(uint32_t));
         for (uint32_t pass = 0; pass < spp; ++pass) cameraPass(dc, pass, invSpp, viewFb.as<float4>(), 1);
         launchPostprocess(stream, viewFb.as<float4>(), viewLdr.as<float4>(), npx);
         finishForward();

@@ -178,3 +178,13 @@ def test_queue_compaction_tiles(photons, capacity):
                                 photon_map_capacity=capacity))
     gpu, orc = _pair(spec, {})
     _check(gpu, orc, backward=photons == 70 * 1024 + 3)
+
+
+def test_queue_beyond_the_grid():
+    """More rays and pixels than the device holds lanes (8 waves on each of
+    1024 SIMDs at most): after the units that the waves start with come those
+    claimed region by region, the last ones ragged."""
+    spec = scene.config_scene(0, n=500, width=1031, height=691)
+    gpu, orc = _pair(spec, dict(photons=700_001, bounces=2, gather_passes=1, adjoint_passes=1, adjoint_bounces=2,
+                                gather_radius=0.02))
+    _check(gpu, orc)

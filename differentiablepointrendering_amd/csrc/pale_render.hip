@@ -318,7 +318,7 @@ struct pale_handle {
     float radius = 0.0f;
     uint32_t photonCap = 0;
     DevMem rawPosPow, rawDirPow, rawPowZ, srtPosPow, srtDirPow, srtPowZ, cellId, sortedIdx, cellCount, cellStart,
-        gridTiles, gridTotal;
+        gridScan;
     bool mapValid = false;
     // Reservoir replacement once the map is full (only when the capacity is
     // below photons * passes * bounces, the most deposits a render makes).
@@ -377,7 +377,7 @@ struct pale_handle {
     pale_batch_tuning tune{};
     hipGraphExec_t bGraph = nullptr;
     std::vector<uint8_t> bGraphKey;
-    DevMem pxOt, pxDl, pxCs, pxCnt, pxOff, pxTiles, entQa, entQb, entQs, entContrib, entPos, entCell, entSorted,
+    DevMem pxOt, pxDl, pxCs, pxCnt, pxOff, pxScan, entQa, entQb, entQs, entContrib, entPos, entCell, entSorted,
         entStart, flagHost;
     // Device state and seed table.
     DevMem state, seedTable, cursors;
@@ -637,8 +637,7 @@ struct pale_handle {
             sortedIdx.reserve(pc * sizeof(uint32_t));
             cellCount.reserve((size_t)grid.total * sizeof(uint32_t));
             cellStart.reserve(((size_t)grid.total + 1) * sizeof(uint32_t));
-            gridTiles.reserve(((size_t)grid.total / kTile + 2) * sizeof(uint32_t));
-            gridTotal.reserve(sizeof(uint32_t) * 4);
+            gridScan.reserve(scanScratchBytes(grid.total));
             launchFill(stream, cellCount.as<uint32_t>(), grid.total, 0u);
             HIPCHECK(hipStreamSynchronize(stream));
             gridConfigured = true;
@@ -780,7 +779,7 @@ struct pale_handle {
     // images, adjoint); the scene, BVH, photon map and photon-stage queues
     // stay.  They are allocated again by the next view.
     std::vector<DevMem*> viewBuffers() {
-        std::vector<DevMem*> v = {&pxOt,    &pxDl,    &pxCs,    &pxCnt,  &pxOff, &pxTiles, &entQa,  &entQb,
+        std::vector<DevMem*> v = {&pxOt,    &pxDl,    &pxCs,    &pxCnt,  &pxOff, &pxScan, &entQa,  &entQb,
                                   &entQs, &entContrib, &entPos, &entCell, &entSorted, &viewFb, &viewLdr, &pend0,
                                   &pend1,   &pend2,   &pend3,   &pend4,  &evCell, &evSorted, &dloss,
                                   &bTiles,  &bSegs,   &bRuns,   &bHdr,   &bCams, &bSegFirst[0], &viewsFb, &viewsLdr};
@@ -846,7 +845,7 @@ struct pale_handle {
             a(pxCs, (size_t)npx * 16);
             a(pxCnt, (size_t)npx * 4);
             a(pxOff, ((size_t)npx + 1) * 4);
-            a(pxTiles, ((size_t)npx / kTile + 2) * 4);
+            a(pxScan, scanScratchBytes(npx));
             if (!A::kDry) pxCap = npx;
         }
         const uint32_t budget = perPixelOverride ? perPixelOverride : S.gather_entry_budget;
@@ -900,12 +899,13 @@ struct pale_handle {
                            walkLds(), countWork);
             tEnd(tt);
             const size_t ts = tBegin(kTCamSort);
-            launchExclusiveScan(stream, px.cnt, px.off, npx, pxTiles.as<uint32_t>(), gridTotal.as<uint32_t>());
+            launchExclusiveScan(stream, px.cnt, px.off, npx, pxScan.as<unsigned long long>());
             launchEntrySort(stream, scene, grid, st, entryCap, px, ent, cellCount.as<uint32_t>(), entStart.as<uint32_t>(),
-                            gridTiles.as<uint32_t>(), gridTotal.as<uint32_t>());
+                            gridScan.as<unsigned long long>());
             tEnd(ts);
             const size_t tk = tBegin(kTGather);
-            launchEntryGather(stream, scene, G, st, entryCap, entStart.as<uint32_t>() + grid.total, ent, countWork);
+            launchEntryGather(stream, scene, G, st, entryCap,
+                              entStart.as<uint32_t>() + sortBuckets(grid, entryCap), ent, countWork);
             tEnd(tk);
             const size_t tc = tBegin(kTCamSort);
             launchCamComposite(stream, npx, px, ent, invSpp, fbp);
@@ -1031,8 +1031,7 @@ struct pale_handle {
         const size_t tg = tBegin(kTGrid);
         launchBuildGrid(stream, grid, st, photonCap, pa(rawPosPow, rawDirPow, rawPowZ),
                         pa(srtPosPow, srtDirPow, srtPowZ), cellId.as<uint32_t>(), sortedIdx.as<uint32_t>(),
-                        cellCount.as<uint32_t>(), cellStart.as<uint32_t>(), gridTiles.as<uint32_t>(),
-                        gridTotal.as<uint32_t>(), radius);
+                        cellCount.as<uint32_t>(), cellStart.as<uint32_t>(), gridScan.as<unsigned long long>(), radius);
         tEnd(tg);
         mapValid = true;
     }
@@ -1077,12 +1076,13 @@ struct pale_handle {
                             walkSpillPtr(), walkLds(), fraction, count);
         if (timed) tEnd(tt);
         const size_t ts = timed ? tBegin(kTCamSort) : 0;
-        launchExclusiveScan(stream, px.cnt, px.off, maxSlots, pxTiles.as<uint32_t>(), gridTotal.as<uint32_t>());
+        launchExclusiveScan(stream, px.cnt, px.off, maxSlots, pxScan.as<unsigned long long>());
         launchEntrySort(stream, scene, grid, st(), entryCap, px, ent, cellCount.as<uint32_t>(), entStart.as<uint32_t>(),
-                        gridTiles.as<uint32_t>(), gridTotal.as<uint32_t>());
+                        gridScan.as<unsigned long long>());
         if (timed) tEnd(ts);
         const size_t tk = timed ? tBegin(kTGather) : 0;
-        launchEntryGather(stream, scene, devGrid(), st(), entryCap, entStart.as<uint32_t>() + grid.total, ent, count);
+        launchEntryGather(stream, scene, devGrid(), st(), entryCap,
+                          entStart.as<uint32_t>() + sortBuckets(grid, entryCap), ent, count);
         if (timed) tEnd(tk);
         const size_t tc = timed ? tBegin(kTCamSort) : 0;
         launchCamCompositeBatch(stream, maxSlots, bHdr.as<BatchHeader>(), px, ent);
@@ -1115,9 +1115,8 @@ struct pale_handle {
         keyAdd(key, walkSpill.p);
         keyAdd(key, walkLds());
         keyAdd(key, entStart.p);
-        keyAdd(key, pxTiles.p);
-        keyAdd(key, gridTiles.p);
-        keyAdd(key, gridTotal.p);
+        keyAdd(key, pxScan.p);
+        keyAdd(key, gridScan.p);
         keyAdd(key, cellCount.p);
         keyAdd(key, maxTiles);
         keyAdd(key, maxSlots);
@@ -1407,8 +1406,7 @@ struct pale_handle {
         const size_t tt = tBegin(kTTransport);
         DevState* st = this->st();
         launchEventSort(stream, grid, st, poolCap, ea(evCmp), evCell.as<uint32_t>(), evSorted.as<uint32_t>(),
-                        cellCount.as<uint32_t>(), entStart.as<uint32_t>(), gridTiles.as<uint32_t>(),
-                        gridTotal.as<uint32_t>());
+                        cellCount.as<uint32_t>(), entStart.as<uint32_t>(), gridScan.as<unsigned long long>());
         launchAdjTransport(stream, scene, devGrid(), st, poolCap, ea(evCmp), evSorted.as<uint32_t>(),
                            gradOpacity.as<float>(), S.full_gradients ? gradFull.as<float>() : nullptr,
                            S.debug_images ? debugImg.as<float>() : nullptr, countWork);

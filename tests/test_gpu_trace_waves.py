@@ -188,3 +188,18 @@ def test_queue_beyond_the_grid():
     gpu, orc = _pair(spec, dict(photons=700_001, bounces=2, gather_passes=1, adjoint_passes=1, adjoint_bounces=2,
                                 gather_radius=0.02))
     _check(gpu, orc)
+
+
+@pytest.mark.parametrize("size", [(1, 1), (127, 129), (128, 128), (29, 565), (257, 255)])
+@pytest.mark.parametrize("radius", [0.3, 0.0118, 0.004])
+def test_scans_and_sort_buckets(size, radius):
+    """Scans of pixels and cells at the edges of a tile (16384 items, the last
+    vector of four cut off at every place), and sorts by whole cells (0.3) and
+    by runs of cells where the grid has more cells than the entries have places
+    (up to 125M against 65,536)."""
+    pts = scene.uniform_surfels(1500, seed=6, scale_lo=0.04, scale_hi=0.1)[0]
+    spec = scene.SceneSpec([scene.light_quad()], [scene.default_camera(*size)], pts,
+                           dict(photons=5000, bounces=3, forward_passes=1, gather_passes=1, adjoint_bounces=3,
+                                adjoint_passes=1, gather_radius=radius, spp_decorrelate=1))
+    gpu, orc = _pair(spec, {})
+    _check(gpu, orc)

@@ -617,7 +617,7 @@ __global__ __launch_bounds__(256) void k_bvh_records(const HostPoint* pts, const
                                                     SurfelGeo* geo, SurfelShade* shade) {
     const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
-    const HostPoint s = pts[ord[k]];
+    const HostPoint s = pts[ord ? ord[k] : k];
     geo[k] = surfelGeoOf(s);
     shade[k] = surfelShadeOf(s);
 }

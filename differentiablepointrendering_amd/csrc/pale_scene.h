@@ -145,6 +145,7 @@ struct BuildProducts {
     // The surfel BLAS was built on the device, which already holds the
     // surfel records and the cloud's wide nodes (after the meshes' ones).
     bool cloudOnDevice = false;
+    uint32_t cloudWide = 0;  // then: wide nodes of the cloud, the root's first
     std::vector<HostPoint> collected;  // scratch of a host build: the points in asset order
 };
 
@@ -158,8 +159,9 @@ struct BuildProducts {
 struct CloudBuild {
     virtual ~CloudBuild() = default;
     virtual HostPoint* staging(uint32_t n) = 0;
+    virtual void staged(uint32_t n) = 0;  // the first n points are written: their copy may start
     virtual bool build(const HostPoint* pts, uint32_t n, uint32_t wideBase, std::vector<RefNode>& blas,
-                       std::vector<uint32_t>& perm, uint32_t& depth) = 0;
+                       std::vector<uint32_t>& perm, uint32_t& depth, uint32_t& wide) = 0;
 };
 
 // The shape of the surfel BLAS over n surfels, which depends on n only (a
@@ -343,5 +345,21 @@ inline void parallelFor(size_t n, F&& f) {
     if (error) std::rethrow_exception(error);
 }
 
+// Points staged between two copies of them to the device.
+constexpr size_t kStageSlice = 1u << 18;
+// f(first, last) over chunks of [0, n) as parallelFor, slice by slice of
+// kStageSlice; after(last) when all before `last` are done.
+template <typename F, typename G>
+inline void parallelSlices(size_t n, F&& f, G&& after) {
+    constexpr size_t kChunk = 1u << 13;
+    for (size_t a = 0; a < n; a += kStageSlice) {
+        const size_t b = n - a < kStageSlice ? n : a + kStageSlice;
+        parallelFor((b - a + kChunk - 1) / kChunk, [&](size_t c) {
+            const size_t first = a + c * kChunk;
+            f(first, b - first < kChunk ? b : first + kChunk);
+        });
+        after(b);
+    }
+}
 
 }  // namespace pale

@@ -378,23 +378,26 @@ void buildScene(const std::vector<HostMesh>& meshes, const std::vector<AssetPoin
         bp.collected.resize(n);
         pts = bp.collected.data();
     }
-    parallelFor((asset.size() + 16383) / 16384, [&](size_t c) {
-      for (size_t i = c * 16384; i < std::min(asset.size(), (c + 1) * 16384); ++i) {
-        const AssetPoint& a = asset[i];
-        HostPoint p{};
-        p.p = a.p;
-        p.tu = normalize(a.tu);
-        p.tv = normalize(a.tv);
-        p.su = a.su;
-        p.sv = a.sv;
-        p.albedo = mk3(clampf(a.albedo.x, 0, 1), clampf(a.albedo.y, 0, 1), clampf(a.albedo.z, 0, 1));
-        p.opacity = clampf(a.opacity, 0, 1);
-        p.alpha_r = 1.0f;
-        p.alpha_t = 0.0f;
-        p.beta = a.beta;
-        p.shape = clampf(a.shape, -5.0f, 5.0f);
-        pts[i] = p;
-      }
+    const auto collect = [&](size_t first, size_t last) {
+        for (size_t i = first; i < last; ++i) {
+            const AssetPoint& a = asset[i];
+            HostPoint p{};
+            p.p = a.p;
+            p.tu = normalize(a.tu);
+            p.tv = normalize(a.tv);
+            p.su = a.su;
+            p.sv = a.sv;
+            p.albedo = mk3(clampf(a.albedo.x, 0, 1), clampf(a.albedo.y, 0, 1), clampf(a.albedo.z, 0, 1));
+            p.opacity = clampf(a.opacity, 0, 1);
+            p.alpha_r = 1.0f;
+            p.alpha_t = 0.0f;
+            p.beta = a.beta;
+            p.shape = clampf(a.shape, -5.0f, 5.0f);
+            pts[i] = p;
+        }
+    };
+    parallelSlices(n, collect, [&](size_t done) {
+        if (staged) cloud->staged((uint32_t)done);
     });
     // The "Gaussian" point-cloud instance with identity transform
     // (pale_bindings.cpp:90-101, SceneBuild.cpp:229-251).
@@ -478,7 +481,7 @@ void buildScene(const std::vector<HostMesh>& meshes, const std::vector<AssetPoin
             for (uint32_t i = 0; i < r.count; ++i)
                 wideBase += (bp.blas[r.first + i].count == 0 && r.count > 1) ? 1u : 0u;
         const uint32_t first = (uint32_t)bp.blas.size();
-        if (staged && cloud->build(pts, n, wideBase, bp.blas, bp.perm, cloudDepth)) {
+        if (staged && cloud->build(pts, n, wideBase, bp.blas, bp.perm, cloudDepth, bp.cloudWide)) {
             bp.cloudOnDevice = true;
         } else {
             std::vector<RefNode> nodes;
@@ -613,24 +616,23 @@ void makeDeviceImage(const BuildProducts& bp, const std::vector<HostMesh>& meshe
         img.tris[i] = TriGeo{a.x, a.y, a.z, 0.f, b.x, b.y, b.z, 0.f, c.x, c.y, c.z, 0.f};
     }
     // Wide nodes: every internal reference node becomes one WideNode holding
-    // both child boxes; leaves become references.
-    std::vector<uint32_t> compact(bp.blas.size(), kInvalid);
+    // both child boxes; leaves become references.  The cloud's come last; a
+    // device build has written them, and of its tree only the root is needed.
+    const Range& cloudRange = bp.blasRanges.back();
+    const size_t listed = bp.cloudOnDevice ? (size_t)cloudRange.first + 1 : bp.blas.size();
+    std::vector<uint32_t> compact(listed, kInvalid);
     uint32_t next = 0;
     for (const Range& r : bp.blasRanges) {
-        for (uint32_t i = 0; i < r.count; ++i) {
+        if (&r == &cloudRange) img.meshWide = next;
+        for (uint32_t i = 0; i < r.count && r.first + i < listed; ++i) {
             const RefNode& n = bp.blas[r.first + i];
             const bool internal = n.count == 0 && r.count > 1;
             if (internal) compact[r.first + i] = next++;
         }
     }
-    // the cloud's wide nodes come last; a device build has written them
-    const Range& cloudRange = bp.blasRanges.back();
-    uint32_t meshWide = next;
-    for (uint32_t i = 0; i < cloudRange.count; ++i)
-        if (compact[cloudRange.first + i] != kInvalid) meshWide = std::min(meshWide, compact[cloudRange.first + i]);
-    img.meshWide = meshWide;
+    if (bp.cloudOnDevice) next = img.meshWide + bp.cloudWide;
     img.wideCount = next;
-    img.nodes.resize(bp.cloudOnDevice ? meshWide : next);
+    img.nodes.resize(bp.cloudOnDevice ? img.meshWide : next);
     auto refOf = [&](const Range& r, uint32_t local) -> uint32_t {
         const RefNode& n = bp.blas[r.first + local];
         if (n.count > 0) return leafRef(n.leftFirst, n.count);

@@ -105,8 +105,13 @@ class DeviceCloudBuild final : public CloudBuild {
    public:
     static constexpr uint32_t kSubtree = 32;      // subtrees this small: one thread each
     static constexpr uint32_t kFitChunk = 16384;  // surfels per fit workgroup
-    static constexpr uint32_t kWideMin = 65536;   // larger nodes take their first steps on many workgroups
-    static constexpr uint32_t kWideTile = 8192;   // positions per workgroup in those steps
+    // Nodes larger than kWideMin take their first steps on many workgroups, of
+    // kWideTile positions each: one workgroup takes 300 us for a level of nodes
+    // of 16k to 64k surfels, a step of many about 20 us.  Rebuild at 65536 and
+    // 8192, 16384 and 4096, 8192 and 4096: 100k surfels 2.9, 2.6, 2.6 ms; 400k 5.6,
+    // 4.9, 4.9 ms; 1M 8.8, 8.1, 8.1 ms.
+    static constexpr uint32_t kWideMin = 16384;
+    static constexpr uint32_t kWideTile = 4096;
 
     hipStream_t stream = nullptr;
     uint32_t minCount = 65536;  // smaller clouds are built on the host

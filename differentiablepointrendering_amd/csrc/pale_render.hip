@@ -677,6 +677,7 @@ struct pale_handle {
         static constexpr bool kDry = false;
         void operator()(DevMem& m, size_t b) const { m.reserve(b); }
     };
+    static constexpr uint32_t kAdjointBatch = 4u << 20;  // rays of a small default adjoint batch
     struct Probe {
         static constexpr bool kDry = true;
         uint64_t add = 0;
@@ -728,8 +729,10 @@ struct pale_handle {
         sizeQueues(cap, a);
     }
 
+    // Adjoint of npx rays at a time; pass: rays of the largest sample when the
+    // default batch holds several (else npx).
     template <typename A>
-    void sizeAdjoint(uint32_t npx, A& a) {
+    void sizeAdjoint(uint32_t npx, uint32_t pass, A& a) {
         sizeQueues(nextPow2(npx), a);
         a(entStart, ((size_t)grid.total + 1) * 4);
         uint32_t have = adjCap;
@@ -739,8 +742,10 @@ struct pale_handle {
         a(pend1, (size_t)npx * sizeof(float4));
         a(pend2, (size_t)npx * sizeof(uint2));
         // Event pool: the events of up to 24 bounces of npx paths wait for
-        // one cell-sorted transport launch.
-        const uint32_t pool = (uint32_t)std::min<uint64_t>((uint64_t)npx * 24u, 1u << 28);
+        // one cell-sorted transport launch; in a batch of more than 4 Mi rays
+        // those of 19 bounces of 4 Mi or of its largest sample.
+        const uint32_t small = std::min(npx, std::max(kAdjointBatch, pass));
+        const uint32_t pool = (uint32_t)std::min<uint64_t>((uint64_t)small * (npx > small ? 19u : 24u), 1u << 28);
         const int arrays = eventRays() ? 6 : 4;
         for (int k = 0; k < arrays; ++k) a(evCmp[k], (size_t)pool * sizeof(float4));
         if (S.full_gradients) {
@@ -757,7 +762,7 @@ struct pale_handle {
     }
     void ensureAdjoint(uint32_t npx) {
         Allocate a;
-        sizeAdjoint(npx, a);
+        sizeAdjoint(npx, npx, a);
     }
 
     // Device bytes a W x H view of spp passes (with its adjoint) would add:
@@ -771,7 +776,7 @@ struct pale_handle {
             p(viewFb, (size_t)npx * sizeof(float4));
             p(viewLdr, (size_t)npx * sizeof(float4));
             if (adjoint) {
-                sizeAdjoint(npx, p);
+                sizeAdjoint(npx, npx, p);
                 p(dloss, (size_t)npx * 3 * sizeof(float));
                 if (S.full_gradients) p(gradFull, std::max<size_t>(1, bp.points.size() * 16) * sizeof(float));
             }
@@ -1451,14 +1456,14 @@ struct pale_handle {
     struct BackwardPlan {
         std::vector<HostBatch> batches;
         std::vector<size_t> pixOff, off;  // pixel and dL/dI float offsets of the views
-        uint32_t maxTiles = 0, maxSlots = 1;
+        uint32_t maxTiles = 0, maxSlots = 1, maxPass = 1;
         size_t maxSegs = 1;
     };
 
     // Buffers of a backward plan (A = Allocate or Probe, as sizeForward).
     template <typename A>
     void sizeBackward(const BackwardPlan& plan, size_t nViews, A& a) {
-        sizeAdjoint(plan.maxSlots, a);
+        sizeAdjoint(plan.maxSlots, plan.maxPass, a);
         a(bTiles, (size_t)plan.maxTiles * sizeof(uint4));
         a(bSegs, plan.maxSegs * sizeof(BatchSeg));
         a(bRuns, sizeof(BatchRun));
@@ -1474,7 +1479,13 @@ struct pale_handle {
     }
 
     // (view, sample) segments in sample-major order cut into batches like
-    // the forward's.
+    // the forward's.  Default batch (slots_per_batch = 0): 16 samples of the
+    // largest view, between 4 Mi and 16 Mi rays.  A batch traces the samples of
+    // a pixel side by side, and each of its bounces ends with a tail of long
+    // rays: the adjoint of 16 samples of 800x800 on 1M surfels takes 19.8 ms in
+    // batches of 4 Mi rays, 16.5 ms in one.  Queues and paths of 16 Mi rays take
+    // 2.6 GB, 2.1 GB more than those of 4 Mi; the event pool gives 1.5 GB of it
+    // back (no more flushes: 6 bounces of 10 Mi rays fit).
     BackwardPlan cutBackward(const std::vector<HostCamera>& vc, const std::vector<uint32_t>& spp) const {
         BackwardPlan plan;
         const uint32_t n = (uint32_t)vc.size();
@@ -1489,7 +1500,12 @@ struct pale_handle {
             maxSpp = std::max(maxSpp, spp[v]);
         }
         if (pixOff[n] > 0x7FFFFFFFull) throw StatusError(PALE_ERR_INVALID_ARG, "render_views_backward: too many pixels");
-        const uint64_t budget = tune.slots_per_batch ? tune.slots_per_batch : (4u << 20);
+        for (const HostCamera& c : vc) plan.maxPass = std::max(plan.maxPass, c.W * c.H);
+        const uint64_t budget =
+            tune.slots_per_batch
+                ? tune.slots_per_batch
+                : std::min<uint64_t>(std::max<uint64_t>((uint64_t)plan.maxPass * 16u, kAdjointBatch), 4u * kAdjointBatch);
+        if (tune.slots_per_batch) plan.maxPass = (uint32_t)std::min<uint64_t>(budget, 0xFFFFFFFFu);
         std::vector<HostBatch>& batches = plan.batches;
         uint64_t cur = budget + 1;
         for (uint32_t p = 0; p < maxSpp; ++p) {

@@ -203,3 +203,29 @@ def test_scans_and_sort_buckets(size, radius):
                                 adjoint_passes=1, gather_radius=radius, spp_decorrelate=1))
     gpu, orc = _pair(spec, {})
     _check(gpu, orc)
+
+
+@pytest.mark.parametrize("full", [0, 1])
+def test_default_adjoint_batches(full):
+    """The default batch of several samples of a large view (16 x 640x512 rays,
+    an event pool of fewer bounces than the samples have) gives the gradients
+    of one sample per batch: sums in another order, 1e-4 of the largest."""
+    from differentiablepointrendering_amd.pale import Renderer
+
+    pts = scene.uniform_surfels(3000, seed=4, scale_lo=0.05, scale_hi=0.15)[0]
+    spec = scene.SceneSpec([scene.light_quad()], [scene.default_camera(64, 64)], pts,
+                           dict(photons=20_000, bounces=3, forward_passes=1, gather_passes=1, adjoint_bounces=20,
+                                adjoint_passes=1, gather_radius=0.05, full_gradients=full, adjoint_decorrelate=1))
+    print(f"case: full={full}", flush=True)
+    r = Renderer.from_spec(spec, {})
+    r.render_forward()
+    cam = scene.default_camera(640, 512)
+    rng = np.random.default_rng(1)
+    dl = rng.normal(size=(512, 640, 3)).astype(np.float32)
+    grads = []
+    for slots in (0, 640 * 512):
+        r.set_batch_tuning(slots_per_batch=slots)
+        grads.append(r.render_view_backward(cam, 16, dl))
+    for k in grads[0]:
+        a, b = grads[0][k], grads[1][k]
+        assert np.allclose(a, b, rtol=1e-4, atol=1e-4 * (float(np.abs(b).max()) or 1.0)), k

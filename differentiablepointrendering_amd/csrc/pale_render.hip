@@ -730,22 +730,27 @@ struct pale_handle {
     }
 
     // Adjoint of npx rays at a time; pass: rays of the largest sample when the
-    // default batch holds several (else npx).
+    // default batch holds several (else npx); events: most that the call makes.
     template <typename A>
-    void sizeAdjoint(uint32_t npx, uint32_t pass, A& a) {
-        sizeQueues(nextPow2(npx), a);
+    void sizeAdjoint(uint32_t npx, uint32_t pass, uint64_t events, A& a) {
+        // (queues in powers of two up to 4 Mi rays, then in steps of 1 Mi)
+        constexpr uint32_t step = kAdjointBatch / 4;
+        sizeQueues(npx <= kAdjointBatch ? nextPow2(npx) : (npx + step - 1) / step * step, a);
         a(entStart, ((size_t)grid.total + 1) * 4);
-        uint32_t have = adjCap;
-        if (eventRays() && !adjFull) have = 0;  // also allocate the event rays
-        if (npx <= have) return;
-        a(pend0, (size_t)npx * sizeof(float4));
-        a(pend1, (size_t)npx * sizeof(float4));
-        a(pend2, (size_t)npx * sizeof(uint2));
         // Event pool: the events of up to 24 bounces of npx paths wait for
         // one cell-sorted transport launch; in a batch of more than 4 Mi rays
         // those of 19 bounces of 4 Mi or of its largest sample.
         const uint32_t small = std::min(npx, std::max(kAdjointBatch, pass));
-        const uint32_t pool = (uint32_t)std::min<uint64_t>((uint64_t)small * (npx > small ? 19u : 24u), 1u << 28);
+        const uint64_t most = std::min<uint64_t>((uint64_t)small * (npx > small ? 19u : 24u), 1u << 28);
+        uint32_t pool = (uint32_t)std::max<uint64_t>(npx, std::min(most, events));
+        uint32_t have = adjCap;
+        if (eventRays() && !adjFull) have = 0;  // also allocate the event rays
+        if (npx <= have && pool <= poolCap) return;
+        npx = std::max(npx, adjCap);
+        pool = std::max(pool, poolCap);
+        a(pend0, (size_t)npx * sizeof(float4));
+        a(pend1, (size_t)npx * sizeof(float4));
+        a(pend2, (size_t)npx * sizeof(uint2));
         const int arrays = eventRays() ? 6 : 4;
         for (int k = 0; k < arrays; ++k) a(evCmp[k], (size_t)pool * sizeof(float4));
         if (S.full_gradients) {
@@ -762,7 +767,7 @@ struct pale_handle {
     }
     void ensureAdjoint(uint32_t npx) {
         Allocate a;
-        sizeAdjoint(npx, npx, a);
+        sizeAdjoint(npx, npx, ~0ull, a);
     }
 
     // Device bytes a W x H view of spp passes (with its adjoint) would add:
@@ -776,7 +781,7 @@ struct pale_handle {
             p(viewFb, (size_t)npx * sizeof(float4));
             p(viewLdr, (size_t)npx * sizeof(float4));
             if (adjoint) {
-                sizeAdjoint(npx, npx, p);
+                sizeAdjoint(npx, npx, ~0ull, p);
                 p(dloss, (size_t)npx * 3 * sizeof(float));
                 if (S.full_gradients) p(gradFull, std::max<size_t>(1, bp.points.size() * 16) * sizeof(float));
             }
@@ -1457,13 +1462,14 @@ struct pale_handle {
         std::vector<HostBatch> batches;
         std::vector<size_t> pixOff, off;  // pixel and dL/dI float offsets of the views
         uint32_t maxTiles = 0, maxSlots = 1, maxPass = 1;
+        uint64_t rays = 0;  // of all batches
         size_t maxSegs = 1;
     };
 
     // Buffers of a backward plan (A = Allocate or Probe, as sizeForward).
     template <typename A>
     void sizeBackward(const BackwardPlan& plan, size_t nViews, A& a) {
-        sizeAdjoint(plan.maxSlots, plan.maxPass, a);
+        sizeAdjoint(plan.maxSlots, plan.maxPass, plan.rays * S.adjoint_bounces, a);
         a(bTiles, (size_t)plan.maxTiles * sizeof(uint4));
         a(bSegs, plan.maxSegs * sizeof(BatchSeg));
         a(bRuns, sizeof(BatchRun));
@@ -1534,6 +1540,7 @@ struct pale_handle {
             b.hdr = BatchHeader{(uint32_t)b.tiles.size(), slots, (uint32_t)b.segs.size(), 0u, 0u, {0, 0, 0}};
             plan.maxTiles = std::max(plan.maxTiles, b.hdr.nTiles);
             plan.maxSlots = std::max(plan.maxSlots, slots);
+            plan.rays += slots;
             plan.maxSegs = std::max(plan.maxSegs, b.segs.size());
         }
         return plan;

@@ -728,19 +728,21 @@ __device__ bool intersectScene(const DevScene& S, F3 o, F3 d, const LaneStack& s
 // Camera walk of 16 passes at 800x800, shared and independent: 41.6 and 87.5 ms
 // before; 36.9 and 56.5 so; 33.4 and 50.6 with the walk's hits shaded elsewhere
 // and 5 waves per SIMD; 30.6 and 49.0 with quad nodes.  Photon trace 10.1 -> 6.1
-// -> 5.1 ms, adjoint trace 31.2 -> 23.2 -> 19.4 ms (independent).  Of the walk's
-// cycles with waves on a CU, vector instructions now take 90 % and L1 accesses
-// 88 %; a sixth of its time passes after the last pixel is drawn, while the
-// longest pixels end.  kLeafMin 6, 8, 10, 16: 5 % slower to 2 % slower; kEndShare
-// 1 and 3: 40 % and 5 % slower.
+// -> 5.1 -> 4.5 ms, adjoint trace 31.2 -> 23.2 -> 19.4 -> 11.5 ms (independent; the
+// last with its shading elsewhere, first rays given and batches of 10 Mi rays).
+// Vector instructions now take 95 % of the walk's cycles with shared samples, 80 %
+// with independent ones, where L1 accesses take 79 %; a sixth of its time passes
+// after the last pixel is drawn, while the longest pixels end.  kLeafMin 6, 8, 10,
+// 16: 5 % slower to 2 % slower; kEndShare 1 and 3: 40 % and 5 % slower.  The photon
+// and adjoint traces run the same with other values (within 1 %).
 //
 // Job: bool finish(bool done, const JobHit&, const Work&, F3& o, F3& d) takes
 // the hits of the lanes with done set (and the work of their queries in
 // counting mode) and returns whether the lane goes on with a new ray (o, d),
 // bool fetch(bool idle, F3& o, F3& d) gives idle lanes new work; both are
 // called by every lane of the wave.  drained(): no more work to fetch
-// (uniform over the wave).  kGoesOn: finish may give a lane a new ray.  Counting mode runs the counting traversal, query
-// by query.
+// (uniform over the wave).  kGoesOn: finish may give a lane a new ray.
+// Counting mode runs the counting traversal, query by query.
 struct JobHit {
     F3 pos;
     uint32_t inst, prim;  // inst kInvalid: miss

@@ -292,10 +292,8 @@ class DeviceCloudBuild final : public CloudBuild {
 // once per device (noAllocScratch) and kept in the handle.
 constexpr uint32_t kNoAllocMaxPixels = 65536;  // 256 x 256
 // Per pixel: 6 queue arrays (16 B), hits 16 + 4 B, pending 16 + 16 + 8 B, 4
-// event arrays (16 B), 4 B of transport order; plus the compaction's tiles.
-constexpr size_t kNoAllocScratchBytes =
-    (size_t)kNoAllocMaxPixels * (6 * 16 + 16 + 4 + 16 + 16 + 8 + 4 * 16 + 4) +
-    ((kNoAllocMaxPixels / kTile + 1) * 8 + 255) / 256 * 256;
+// event arrays (16 B), 4 B of transport order.
+constexpr size_t kNoAllocScratchBytes = (size_t)kNoAllocMaxPixels * (6 * 16 + 16 + 4 + 16 + 16 + 8 + 4 * 16 + 4);
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
 namespace {
@@ -711,7 +709,9 @@ struct pale_handle {
         }
         a(hitPos, (size_t)cap * sizeof(float4));
         a(hitPrim, (size_t)cap * sizeof(uint32_t));
-        a(tileState, ((size_t)cap / kTile + 1) * sizeof(uint64_t));
+        // (also the no-allocation adjoint's: tiles wait for each other, so no two
+        // handles may share their states)
+        a(tileState, ((size_t)std::max(cap, kNoAllocMaxPixels) / kTile + 1) * sizeof(uint64_t));
         if (reservoirOn) {
             a(depStg[0], (size_t)cap * sizeof(float4));
             a(depStg[1], (size_t)cap * sizeof(float4));
@@ -1712,7 +1712,7 @@ struct pale_handle {
         float4* q[7];
         for (float4*& x : q) x = reinterpret_cast<float4*>(take(M * sizeof(float4)));
         const HitArrays hit{q[6], reinterpret_cast<uint32_t*>(take(M * sizeof(uint32_t)))};
-        const TileStates ts{reinterpret_cast<unsigned long long*>(take((M / kTile + 1) * sizeof(uint64_t)))};
+        const TileStates ts = tileStates();
         const PendingArrays pend{reinterpret_cast<float4*>(take(M * sizeof(float4))),
                                  reinterpret_cast<float4*>(take(M * sizeof(float4))),
                                  reinterpret_cast<uint2*>(take(M * sizeof(uint2))), nullptr, nullptr};

@@ -267,8 +267,8 @@ def pmc_summary(dirs, cal_dirs=None):
                                              if "hbm_bytes_per_launch" in k and k.get("launches"))
             out["totals"]["kernel_ms"] = round(sum(k.get("total_ms", 0.0) for k in out["kernels"].values()), 3)
     # What the counters say bounds each kernel, as fractions of the kernel's
-    # cycles on every CU (GRBM_GUI_ACTIVE sums the 8 XCDs' GPU-busy cycles;
-    # the _sum counters sum 256 CUs).
+    # cycles on every CU or SIMD (GRBM_GUI_ACTIVE sums the 8 XCDs' GPU-busy
+    # cycles; the _sum counters sum 256 CUs, the SQ counters 1024 SIMDs).
     for k in out["kernels"].values():
         c = k.get("counters_per_launch", {})
         if c.get("GRBM_GUI_ACTIVE"):
@@ -280,6 +280,13 @@ def pmc_summary(dirs, cal_dirs=None):
                     u[key] = c[name] / 256.0 / cyc
             if "TCP_TOTAL_CACHE_ACCESSES_sum" in c and "TCP_TCC_READ_REQ_sum" in c:
                 u["l1_hit"] = 1.0 - c["TCP_TCC_READ_REQ_sum"] / max(c["TCP_TOTAL_CACHE_ACCESSES_sum"], 1.0)
+                u["l1_accesses"] = c["TCP_TOTAL_CACHE_ACCESSES_sum"] / 256.0 / cyc
+            if "SQ_ACTIVE_INST_VALU" in c:
+                # A vector instruction of a wave takes a SIMD four cycles.  (The
+                # cycles are another pass's: a little above 1 can come out.)
+                u["valu_busy"] = min(1.0, c["SQ_ACTIVE_INST_VALU"] * 4.0 / 1024.0 / cyc)
+                if "SQ_THREAD_CYCLES_VALU" in c:
+                    u["valu_lanes"] = c["SQ_THREAD_CYCLES_VALU"] / max(c["SQ_ACTIVE_INST_VALU"], 1.0) / 64.0
             k["utilisation"] = u
         if c.get("SQ_WAVE_CYCLES"):
             u = k.setdefault("utilisation", {})
@@ -847,7 +854,7 @@ def counter_roofline(form, kernel, avg_launch_ms, algorithmic_bytes=None):
     calibrated FETCH_SIZE + WRITE_SIZE bytes per launch of the same workload
     (its summary in profiles/, rocprofv3 --pmc) over the launch duration
     measured here with HIP events.  What bounds the kernel comes from the
-    same profile's unit counters (TD / TA busy, L1 hit rate, issue), with
+    same profile's unit counters (VALU / TD / TA busy, L1 hit rate), with
     HBM's own fraction beside them.  The reference byte model per work unit
     (every lane charged for its own node and surfel loads, most of which
     the L1 serves) is kept as an informational rate."""
@@ -870,10 +877,10 @@ def counter_roofline(form, kernel, avg_launch_ms, algorithmic_bytes=None):
         lim = {kk: round(v, 3) for kk, v in u.items()}
         if out["frac"] is not None:
             lim["hbm"] = out["frac"]
-        busy = {kk: v for kk, v in lim.items() if kk in ("td_busy", "ta_busy", "hbm")}
+        busy = {kk: v for kk, v in lim.items() if kk in ("valu_busy", "td_busy", "ta_busy", "hbm")}
         top = max(busy, key=busy.get) if busy else None
-        names = {"td_busy": "vector-memory data return (TD)", "ta_busy": "vector-memory addressing (TA)",
-                 "hbm": "HBM bandwidth"}
+        names = {"valu_busy": "vector instruction issue (VALU)", "td_busy": "vector-memory data return (TD)",
+                 "ta_busy": "vector-memory addressing (TA)", "hbm": "HBM bandwidth"}
         out["limiter"] = {"unit": names.get(top, top), "fractions": lim}
     for key in ("vgpr_field", "agpr", "sgpr", "scratch_bytes_per_lane", "lds_bytes"):
         if key in k:

@@ -1085,8 +1085,10 @@ struct GridRows {
         const float d = gap(ylo, yhi, cy, g.ry);
         const float rest = left - d * d;
         const float hw = __builtin_amdgcn_sqrtf(fmaxf(rest, 0.0f)) * inv;
-        ax = max((int)floorf(x0 - hw), lx);
-        bx = min((int)floorf(x1 + hw), hx);
+        // The first and last cells have no outer face (photons beyond the grid
+        // are stored there): a point beyond it keeps them.
+        ax = min(max((int)floorf(x0 - hw), lx), g.rx - 1);
+        bx = max(min((int)floorf(x1 + hw), hx), 0);
         return rest >= 0.0f && ax <= bx;
     }
 };

@@ -162,6 +162,9 @@ struct alignas(16) QuadNode {
     uint32_t pad[4];
 };
 
+// Stack entries of a lane that a traversal workgroup can hold in 64 KB of LDS.
+constexpr uint32_t kStackLimit = 64;
+
 PALE_HD uint32_t leafRef(uint32_t first, uint32_t count) { return kLeafBit | (first << 2) | (count - 1u); }
 PALE_HD uint32_t leafFirst(uint32_t ref) { return (ref & ~kLeafBit) >> 2; }
 PALE_HD uint32_t leafCount(uint32_t ref) { return (ref & 3u) + 1u; }

@@ -335,8 +335,10 @@ struct DevPointArrays {
 // per surfel: p, t_u, t_v, s_u, s_v, albedo, opacity, beta).
 void launchApplyPoints(hipStream_t s, SurfelGeo* geo, SurfelShade* shade, float* raw, DevPointArrays a, uint32_t n);
 
-// Quad nodes first .. first + count - 1 from the wide nodes of the same index.
-void launchQuadNodes(hipStream_t s, const WideNode* nodes, QuadNode* quads, uint32_t first, uint32_t count);
+// Quad nodes first .. first + count - 1 from the wide nodes of the same index,
+// of one or two levels.
+void launchQuadNodes(hipStream_t s, const WideNode* nodes, QuadNode* quads, uint32_t first, uint32_t count,
+                     uint32_t levels);
 
 // Device build of the surfel BVH (pale_bvh.hip).  boxes / refBox: 6 floats
 // (min xyz, max xyz) per surfel / per reference node; acc: 6 order-

@@ -2039,9 +2039,10 @@ __global__ __launch_bounds__(256) void k_gather_points(DevGrid G, uint32_t n, co
 // A node's quad node.  The children's own boxes are not stored: the traversal
 // takes their entries from the union of their children's, so a node is written
 // two levels deep only where those unions are the children's boxes (always,
-// unless a box has NaN or no extent); otherwise its two children take a slot
-// each.
-__global__ __launch_bounds__(256) void k_quad_nodes(const WideNode* nodes, QuadNode* quads, uint32_t first, uint32_t n) {
+// unless a box has NaN or no extent); otherwise, and where `levels` is 1, its two
+// children take a slot each.
+__global__ __launch_bounds__(256) void k_quad_nodes(const WideNode* nodes, QuadNode* quads, uint32_t first, uint32_t n,
+                                                    uint32_t levels) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const WideNode w = nodes[first + i];
@@ -2053,7 +2054,7 @@ __global__ __launch_bounds__(256) void k_quad_nodes(const WideNode* nodes, QuadN
     const uint32_t ref[2] = {w.left, w.right};
     Box box[4];
     uint32_t refs[4];
-    bool whole = true;
+    bool whole = levels == 2u;
     for (int c = 0; c < 2; ++c) {
         box[2 * c] = box[2 * c + 1] = child[c];
         refs[2 * c] = ref[c];
@@ -2365,8 +2366,9 @@ void launchGatherPoints(hipStream_t s, const DevGrid& G, uint32_t n, const float
     if (n) k_gather_points<<<blocks(n, 256), 256, 0, s>>>(G, n, q, nrm, out);
 }
 
-void launchQuadNodes(hipStream_t s, const WideNode* nodes, QuadNode* quads, uint32_t first, uint32_t count) {
-    if (count) k_quad_nodes<<<blocks(count, 256), 256, 0, s>>>(nodes, quads, first, count);
+void launchQuadNodes(hipStream_t s, const WideNode* nodes, QuadNode* quads, uint32_t first, uint32_t count,
+                     uint32_t levels) {
+    if (count) k_quad_nodes<<<blocks(count, 256), 256, 0, s>>>(nodes, quads, first, count, levels);
 }
 
 void launchSetOpacity(hipStream_t s, SurfelShade* shade, const float* opacity, uint32_t n) {

@@ -578,7 +578,8 @@ struct pale_handle {
         scene.shade = shade.as<SurfelShade>();
         scene.nodes = nodes.as<WideNode>();
         quads.reserve((size_t)img.wideCount * sizeof(QuadNode));
-        launchQuadNodes(stream, nodes.as<WideNode>(), quads.as<QuadNode>(), img.meshWide, img.wideCount - img.meshWide);
+        launchQuadNodes(stream, nodes.as<WideNode>(), quads.as<QuadNode>(), img.meshWide, img.wideCount - img.meshWide,
+                        img.quadLevels);
         scene.quads = quads.as<QuadNode>();
         scene.tris = tris.as<TriGeo>();
         scene.inst = inst.as<DevInstance>();
@@ -593,7 +594,8 @@ struct pale_handle {
         scene.nTlas = (uint32_t)img.tlas.size();
         scene.nLights = (uint32_t)img.lights.size();
         scene.stackDepth = img.stackDepth;
-        if ((size_t)img.stackDepth * sizeof(uint2) * kTraceBlock > 65536)
+        static_assert(kStackLimit * sizeof(uint2) * kTraceBlock == 65536);
+        if (img.stackDepth > kStackLimit)
             throw StatusError(PALE_ERR_INVALID_ARG, "BVH too deep for the LDS traversal stack");
         ensureWalkSpill();
         gradOpacity.reserve(std::max<size_t>(1, bp.points.size()) * sizeof(float));

@@ -201,6 +201,7 @@ struct DeviceImage {
     std::vector<DevLight> lights;
     std::vector<DevEmTri> emTris;
     uint32_t stackDepth = 0;  // stack entries one lane needs
+    uint32_t quadLevels = 2;  // levels of the cloud's tree in a quad node
     uint32_t wideCount = 0;   // wide nodes of all trees, the cloud's from meshWide on
     // With BuildProducts::cloudOnDevice: surfGeo / surfShade are sized but
     // not filled, and only nodes[0, meshWide) (the meshes' wide nodes) are;

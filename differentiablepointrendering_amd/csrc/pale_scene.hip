@@ -686,8 +686,12 @@ void makeDeviceImage(const BuildProducts& bp, const std::vector<HostMesh>& meshe
     for (const HostEmTri& e : bp.emTris) img.emTris.push_back(DevEmTri{e.tri, e.cdf});
     // Near-far depth-first traversal keeps at most one pending sibling per
     // level, or three per two levels of quad nodes; tlasDepth + 1 entries below
-    // a BLAS's.
-    img.stackDepth = (bp.tlasMaxDepth + 1) + std::max(bp.blasMaxDepth + 1, 3 * ((bp.blasMaxDepth + 1) / 2));
+    // a BLAS's.  Where two levels at a time would pass the limit (a very deep
+    // top level), the quad nodes hold one.
+    const uint32_t top = bp.tlasMaxDepth + 1, levels = bp.blasMaxDepth + 1;
+    const uint32_t two = top + std::max(levels, 3 * (levels / 2));
+    img.quadLevels = two <= kStackLimit ? 2u : 1u;
+    img.stackDepth = img.quadLevels == 2u ? two : top + levels;
 }
 
 }  // namespace pale

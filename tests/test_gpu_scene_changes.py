@@ -69,3 +69,27 @@ def test_gather_beyond_the_grid(radius):
     want = orc.gather(q, n)
     assert np.count_nonzero(want.any(axis=1)) > len(q) // 4
     assert np.array_equal(gpu.gather_irradiance(q, n), want)
+
+
+@pytest.mark.parametrize("quads", [62, 64])
+def test_deep_top_level(quads):
+    """Instances on a geometric row make the top level as deep as there are
+    instances (its midpoint partition takes one off at a time), so that little
+    of the 64 stack entries is left to a cloud whose tree, two levels per step,
+    would need 21 of them and node by node needs 15."""
+    pts = scene.uniform_surfels(40_000, seed=9, scale_lo=0.01, scale_hi=0.03)[0]
+    spec = scene.SceneSpec([scene.light_quad()], [scene.default_camera(40, 32)], pts,
+                           dict(photons=4000, bounces=3, forward_passes=1, gather_passes=2, adjoint_bounces=3,
+                                adjoint_passes=1, seed=5, gather_radius=0.05, spp_decorrelate=1))
+    along_x = ((0, 0, 1), (0, 1, 0), (-1, 0, 0))  # normal +x
+    for i in range(quads):
+        spec.meshes.append(scene.quad_mesh(f"q{i}", (2.0 ** -i, 0.0, 0.0), along_x, 0.01, (0.6, 0.5, 0.4)))
+    gpu, orc = _pair(spec, {})
+    _check(gpu, orc)
+    rng = np.random.default_rng(3)
+    o = rng.uniform(-1.2, 1.2, size=(2000, 3)).astype(np.float32)
+    d = rng.normal(size=(2000, 3))
+    d = (d / np.linalg.norm(d, axis=1, keepdims=True)).astype(np.float32)
+    a, b = gpu.trace_rays(o, d), orc.trace(o, d)
+    for k in ("instance", "primitive", "t", "position"):
+        assert np.array_equal(a[k], b[k]), k

@@ -360,15 +360,23 @@ struct pale_handle {
     // the 5 waves per SIMD their registers allow (8 or 16 entries: within 2 %).
     static constexpr uint32_t kTraceLdsEntries = 12;
     DevMem traceSpill;
-    size_t traceSpillBytes(uint32_t rays) const {
-        if (img.stackDepth <= kTraceLdsEntries || !rays) return 0;
-        const size_t lanes = queueTraceLanes(scene, rays, kTraceLdsEntries);
-        return (size_t)(img.stackDepth - kTraceLdsEntries) * lanes * sizeof(uint2);
+    uint32_t traceLanes = 0;  // lanes of the largest launch over queueCap rays
+    size_t traceSpillBytes(size_t lanes) const {
+        return scene.stackDepth > kTraceLdsEntries
+                   ? (size_t)(scene.stackDepth - kTraceLdsEntries) * lanes * sizeof(uint2)
+                   : 0;
     }
-    // t with the split stack when the spill area (sized with the queues)
-    // covers a launch of `rays` lanes; else the whole stack in LDS.
-    TraceParams withTraceSpill(TraceParams t, uint32_t rays) const {
-        const size_t need = traceSpillBytes(rays);
+    // The spill area for the current scene and queues: its size changes with
+    // both (a cloud that grows gets a deeper tree).
+    void ensureTraceSpill() {
+        if (!queueCap) return;
+        traceLanes = queueTraceLanes(scene, queueCap, kTraceLdsEntries);
+        if (const size_t sb = traceSpillBytes(traceLanes)) traceSpill.reserve(sb);
+    }
+    // t with the split stack where there is an area for it (it covers every
+    // launch over a queue); else the whole stack in LDS.
+    TraceParams withTraceSpill(TraceParams t) const {
+        const size_t need = traceSpillBytes(traceLanes);
         if (need && traceSpill.p && traceSpill.bytes >= need) {
             t.spill = traceSpill.as<uint2>();
             t.inLds = kTraceLdsEntries;
@@ -598,6 +606,7 @@ struct pale_handle {
         if (img.stackDepth > kStackLimit)
             throw StatusError(PALE_ERR_INVALID_ARG, "BVH too deep for the LDS traversal stack");
         ensureWalkSpill();
+        ensureTraceSpill();
         gradOpacity.reserve(std::max<size_t>(1, bp.points.size()) * sizeof(float));
         HIPCHECK(hipStreamSynchronize(stream));
     }
@@ -723,8 +732,12 @@ struct pale_handle {
             a(resvAttempt, (size_t)cap * sizeof(uint32_t));
             a(resvSlot, (size_t)cap * sizeof(uint32_t));
         }
-        if (const size_t sb = traceSpillBytes(cap)) a(traceSpill, sb);
-        if (!A::kDry) queueCap = cap;
+        if (A::kDry) {
+            if (const size_t sb = traceSpillBytes(queueTraceLanes(scene, cap, kTraceLdsEntries))) a(traceSpill, sb);
+        } else {
+            queueCap = cap;
+            ensureTraceSpill();
+        }
     }
     void ensureQueues(uint32_t cap) {
         Allocate a;
@@ -1054,7 +1067,7 @@ struct pale_handle {
             for (uint32_t b = 0; b < S.bounces; ++b) {
                 launchPhotonNext(stream, st, table, tlen, (int)b, resvCap, ts, P);
                 const size_t te = tBegin(kTPhoton);
-                launchQueueTrace(stream, scene, st, P, rq(in), hits(), withTraceSpill(tp(), P), false, countWork);
+                launchQueueTrace(stream, scene, st, P, rq(in), hits(), withTraceSpill(tp()), false, countWork);
                 tEnd(te);
                 launchPhotonShade(stream, scene, st, P, rq(in), hits(), rq(out), queueCap,
                                   pa(rawPosPow, rawDirPow, rawPowZ), pa(depStg[0], depStg[1], depStg[2]), tp(), rs,
@@ -1611,7 +1624,7 @@ struct pale_handle {
                     pooledBound = 0;
                 }
                 tpb.segFirst = segs;
-                const TraceParams t = withTraceSpill(tpb, nr);
+                const TraceParams t = withTraceSpill(tpb);
                 const size_t ta = tBegin(kTAdjTrace);
                 launchQueueTrace(stream, scene, st, nr, rq(in), hits(), t, true, countWork);
                 tEnd(ta);
@@ -1681,7 +1694,7 @@ struct pale_handle {
                     if (pooledBound + npx > poolCap) flush();
                     TraceParams tpc = tp(invSpp, nullptr, nullptr, adjointSeed(spp));
                     tpc.debugBase = (uint32_t)(off[k] / 3);
-                    tpc = withTraceSpill(tpc, npx);
+                    tpc = withTraceSpill(tpc);
                     const size_t ta = tBegin(kTAdjTrace);
                     launchQueueTrace(stream, scene, st, npx, rq(in), hits(), tpc, true, countWork);
                     tEnd(ta);

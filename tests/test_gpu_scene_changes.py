@@ -93,3 +93,39 @@ def test_deep_top_level(quads):
     a, b = gpu.trace_rays(o, d), orc.trace(o, d)
     for k in ("instance", "primitive", "t", "position"):
         assert np.array_equal(a[k], b[k]), k
+
+
+def test_grown_cloud_keeps_its_stacks_split():
+    """A renderer whose cloud grew (a deeper tree, more stack entries than a
+    lane has in LDS) holds the device buffers of one made with that cloud, the
+    traces' spill area among them, and gives its results."""
+    from differentiablepointrendering_amd.pale import Renderer
+
+    pts = scene.uniform_surfels(20_000, seed=7, scale_lo=0.02, scale_hi=0.06)[0]
+    ends = {k: np.concatenate([v[[0, 0]], v[2:]]) for k, v in pts.items()}
+    ends["position"][:2] = (-1.2, -1.2, -1.2), (1.2, 1.2, 1.2)  # both clouds span the same box, and grid
+    ends["scale"][:2] = 0.06
+    st = dict(photons=20_000, bounces=4, forward_passes=1, gather_passes=2, adjoint_bounces=3, adjoint_passes=1,
+              seed=5, gather_radius=0.05)
+    few = scene.SceneSpec([scene.light_quad()], [scene.default_camera(60, 44)],
+                          {k: v[:40] for k, v in ends.items()}, st)
+    all_ = scene.SceneSpec(few.meshes, few.cameras, ends, st)
+    print("case: cloud of 40 surfels grown to 20000", flush=True)
+
+    def bytes_of(make):
+        before = Renderer.device_bytes()
+        r = make()
+        return r, Renderer.device_bytes() - before
+
+    def grown():
+        r = Renderer.from_spec(few, {})
+        r.add_points({"new": {k: v[40:] for k, v in ends.items() if k != "shape"}})
+        return r
+
+    a, held_a = bytes_of(grown)
+    b, held_b = bytes_of(lambda: Renderer.from_spec(all_, {}))
+    assert a.point_count == b.point_count == 20_000
+    assert held_a == held_b
+    x, y = a.render_forward()["camera1_raw"], b.render_forward()["camera1_raw"]
+    assert np.array_equal(x, y)
+    assert np.array_equal(a.photons()["position"], b.photons()["position"])

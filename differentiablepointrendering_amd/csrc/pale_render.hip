@@ -675,7 +675,7 @@ struct pale_handle {
             HIPCHECK(hipStreamSynchronize(stream));
             gridConfigured = true;
         }
-        ensureQueues(nextPow2(std::max(S.photons, 1u)));
+        ensureQueues(photonQueue());
     }
     HitArrays hits() const { return HitArrays{hitPos.as<float4>(), hitPrim.as<uint32_t>()}; }
     TileStates tileStates() const { return TileStates{tileState.as<unsigned long long>()}; }
@@ -711,9 +711,38 @@ struct pale_handle {
         }
     };
 
+    // The other two uses of the sizing: what buffers hold beyond a size, and
+    // smaller ones in their place (made before any is exchanged, so that a
+    // failure leaves all as they were).
+    struct Excess {
+        static constexpr bool kDry = true;
+        uint64_t bytes = 0;
+        void operator()(const DevMem& m, size_t b) {
+            b = std::max<size_t>(b, 16);
+            if (m.p && m.bytes > b) bytes += m.bytes - b;
+        }
+    };
+    struct Shrink {
+        static constexpr bool kDry = false;
+        std::vector<std::pair<DevMem*, DevMem>> smaller;
+        void operator()(DevMem& m, size_t b) {
+            if (!m.p || m.bytes <= std::max<size_t>(b, 16)) return;
+            smaller.emplace_back(&m, DevMem{});
+            smaller.back().second.reserve(b);
+        }
+        void exchange() {
+            for (auto& [m, s] : smaller) {
+                std::swap(m->p, s.p);
+                std::swap(m->bytes, s.bytes);
+            }
+            smaller.clear();
+        }
+    };
+
+    // Queue capacity of the photon stage; a large adjoint batch needs more.
+    uint32_t photonQueue() const { return nextPow2(std::max(S.photons, 1u)); }
     template <typename A>
-    void sizeQueues(uint32_t cap, A& a) {
-        if (cap <= queueCap) return;
+    void queueBuffers(uint32_t cap, A& a) {
         for (int k = 0; k < 3; ++k) {
             a(qA[k], (size_t)cap * sizeof(float4));
             a(qB[k], (size_t)cap * sizeof(float4));
@@ -732,9 +761,13 @@ struct pale_handle {
             a(resvAttempt, (size_t)cap * sizeof(uint32_t));
             a(resvSlot, (size_t)cap * sizeof(uint32_t));
         }
-        if (A::kDry) {
-            if (const size_t sb = traceSpillBytes(queueTraceLanes(scene, cap, kTraceLdsEntries))) a(traceSpill, sb);
-        } else {
+        if (const size_t sb = traceSpillBytes(queueTraceLanes(scene, cap, kTraceLdsEntries))) a(traceSpill, sb);
+    }
+    template <typename A>
+    void sizeQueues(uint32_t cap, A& a) {
+        if (cap <= queueCap) return;
+        queueBuffers(cap, a);
+        if (!A::kDry) {
             queueCap = cap;
             ensureTraceSpill();
         }
@@ -825,13 +858,15 @@ struct pale_handle {
     }
 
     // Frees the buffers that grow with the image size (camera gather, view
-    // images, adjoint); the scene, BVH, photon map and photon-stage queues
-    // stay.  They are allocated again by the next view.
+    // images, adjoint) and takes the ray queues back to the photon stage's
+    // size; the scene, BVH and photon map stay.  They are allocated again by
+    // the next view.
     std::vector<DevMem*> viewBuffers() {
         std::vector<DevMem*> v = {&pxOt,    &pxDl,    &pxCs,    &pxCnt,  &pxOff, &pxScan, &entQa,  &entQb,
                                   &entQs, &entContrib, &entPos, &entCell, &entSorted, &viewFb, &viewLdr, &pend0,
                                   &pend1,   &pend2,   &pend3,   &pend4,  &evCell, &evSorted, &dloss,
-                                  &bTiles,  &bSegs,   &bRuns,   &bHdr,   &bCams, &bSegFirst[0], &viewsFb, &viewsLdr};
+                                  &bTiles,  &bSegs,   &bRuns,   &bHdr,   &bCams, &bSegFirst[0], &bSegFirst[1], &bSegEnd,
+                                  &bGroups, &bGroupSegs, &viewsFb, &viewsLdr};
         for (int k = 0; k < 6; ++k) {
             v.push_back(&evCmp[k]);
         }
@@ -840,6 +875,11 @@ struct pale_handle {
     uint64_t viewBufferBytes() {
         uint64_t b = 0;
         for (DevMem* m : viewBuffers()) b += m->p ? m->bytes : 0;
+        if (queueCap > photonQueue()) {
+            Excess e;
+            queueBuffers(photonQueue(), e);
+            b += e.bytes;
+        }
         return b;
     }
     void releaseViewBuffers() {
@@ -847,6 +887,13 @@ struct pale_handle {
         pxCap = entryCap = 0;
         adjCap = poolCap = 0;
         adjFull = false;
+        if (queueCap > photonQueue()) {
+            Shrink s;
+            queueBuffers(photonQueue(), s);
+            s.exchange();
+            queueCap = photonQueue();
+            ensureTraceSpill();
+        }
     }
 
     void resetState() {

@@ -377,11 +377,13 @@ int pale_views_bytes(pale_handle* h, uint32_t n, const uint32_t* widths,
                      const int32_t* adjoint, uint64_t* out);
 
 /* Device bytes of this renderer's image-sized buffers (camera gather, view
- * images, adjoint): what pale_release_view_buffers frees. */
+ * images, adjoint, ray queues beyond the photon stage's): what
+ * pale_release_view_buffers frees. */
 int pale_view_buffer_bytes(pale_handle* h, uint64_t* out);
 
 /* Frees the buffers that grow with the image size (camera gather, view
- * images, adjoint); scene, BVH and photon map stay resident. */
+ * images, adjoint, ray queues beyond the photon stage's); scene, BVH and photon
+ * map stay resident. */
 int pale_release_view_buffers(pale_handle* h);
 
 /* Photon stage of render_forward only (emission, bounces, grid). */

@@ -400,6 +400,49 @@ __device__ __forceinline__ void cloudLeaf(const DevScene& S, const LaneStack& st
     cloudPop(st, c);
 }
 
+// The lane's traversal from the start, by the binary tree's steps and the tests
+// in leaf order: for a ray whose two-level walk accepted a NaN distance (a
+// degenerate surfel's).  After one, the next surfel is accepted at any
+// distance, so the best rises, and boxes tested two levels early against the
+// smaller one are missing from the stack.  On the lane's own state and surfel by
+// surfel: it runs hardly ever, and its registers would count for every wave (a
+// second kind of step in the waves' loop cost 3 to 5 % of every case).
+__device__ __forceinline__ void cloudAgain(const DevScene& S, uint32_t rootRef, const LaneStack& st, CloudLane& c) {
+    c.best = __builtin_huge_valf();
+    c.bestIdx = kInvalid;
+    c.sp = c.base;
+    c.ref = rootRef;
+    while (c.ref != kRefDone) {
+        if (c.ref & kLeafBit) {
+            const uint32_t first = leafFirst(c.ref), cnt = leafCount(c.ref);
+#pragma unroll 1
+            for (uint32_t k = 0; k < cnt; ++k) {
+                const SurfelGeo& g = S.geo[first + k];
+                const F3 n = mk3(g.nx, g.ny, g.nz);
+                const float nd = dot(n, c.d);
+                if (fabsf(nd) < 1e-6f) continue;
+                const float t = dot(n, mk3(g.px, g.py, g.pz) - c.o) / nd;
+                if (t <= 1e-5f || t >= c.best) continue;
+                if (surfelR2(g, c.o + c.d * t) >= 1.0f) continue;
+                c.best = t;
+                c.bestIdx = first + k;
+            }
+            cloudPop(st, c);
+        } else {
+            const float4* n = reinterpret_cast<const float4*>(S.nodes + c.ref);
+            const float4 p = n[0], q = n[1], r = n[2];
+            const uint2 refs = reinterpret_cast<const uint2*>(S.nodes + c.ref)[6];  // left, right (not the padding)
+            float tl = __builtin_huge_valf(), tr = __builtin_huge_valf();
+            const bool hl = slab(c.o, c.inv, p.x, p.y, p.z, p.w, q.x, q.y, c.best, 1e-6f, tl);
+            const bool hr = slab(c.o, c.inv, q.z, q.w, r.x, r.y, r.z, r.w, c.best, 1e-6f, tr);
+            const bool left = hl && (!hr || tl <= tr);
+            if (hl && hr) st.pushBounded(c.sp, left ? refs.y : refs.x, left ? tr : tl);
+            c.ref = left ? refs.x : refs.y;
+            if (!hl && !hr) cloudPop(st, c);
+        }
+    }
+}
+
 // A wave's leaf tests, packed: the (lane, surfel) pairs of up to 16 lanes at
 // a leaf take one test each on all 64 lanes, four neighbouring lanes (a quad)
 // per leaf.  A step of four tests one after the other costs the wave the same
@@ -440,7 +483,7 @@ __device__ __forceinline__ bool cloudLeafRound(const DevScene& S, CloudLane& c, 
     const F3 d = mk3(laneGetF(c.d.x, from), laneGetF(c.d.y, from), laneGetF(c.d.z, from));
     const float best = laneGetF(c.best, from);
     float t = 0.0f;
-    bool ok = false;
+    bool inside = false;  // hit, in front, in the support: all tests but that against best
     if (r < n && k < leafCount(ref)) {
         const float4* g = reinterpret_cast<const float4*>(S.geo + (leafFirst(ref) + k));
         const float4 g0 = g[0], g1 = g[1], g2 = g[2], g3 = g[3];
@@ -452,13 +495,14 @@ __device__ __forceinline__ bool cloudLeafRound(const DevScene& S, CloudLane& c, 
         const float a = dot(mk3(g2.x, g2.y, g2.z), q), b = dot(mk3(g3.x, g3.y, g3.z), q);
         const float as = a * g1.w, bs = b * g0.w, ss = g0.w * g1.w;
         const float lhs = as * as + bs * bs, rhs = ss * ss;
-        bool inside = lhs < rhs * (1.0f - 4e-6f);
+        inside = lhs < rhs * (1.0f - 4e-6f);
         if (!(inside || lhs > rhs * (1.0f + 4e-6f)) || !(rhs > 1e-30f) || !(lhs < 1e30f)) {
             const float uu = a / g0.w, vv = b / g1.w;
             inside = !(uu * uu + vv * vv >= 1.0f);
         }
-        ok = inside && !(fabsf(nd) < 1e-6f) && !(t <= 1e-5f) && !(t >= best);
+        inside = inside && !(fabsf(nd) < 1e-6f) && !(t <= 1e-5f);
     }
+    const bool ok = inside && !(t >= best);
     unsigned long long wins;
     float nt;
     if (__builtin_amdgcn_ballot_w64(ok && !(t < best)) == 0ull) {
@@ -469,18 +513,23 @@ __device__ __forceinline__ bool cloudLeafRound(const DevScene& S, CloudLane& c, 
         nt = laneGetF(q, (below << 2) & 63u);
     } else {
         // A NaN distance (a degenerate surfel or ray) was accepted: the tests
-        // one after the other, each against the best before it.
-        const unsigned long long oks = __builtin_amdgcn_ballot_w64(ok);
-        const uint32_t mine = (uint32_t)(oks >> (lane & 60u));
+        // one after the other, each against the best before it (none is beyond
+        // a NaN best).  A lane that accepted one, also if another took its
+        // place, ends here with a NaN best (traceWave).
+        const unsigned long long in = __builtin_amdgcn_ballot_w64(inside);
+        const uint32_t mine = (uint32_t)(in >> (lane & 60u));
         const float t0 = quadGet<0x00>(t), t1 = quadGet<0x55>(t), t2 = quadGet<0xAA>(t), t3 = quadGet<0xFF>(t);
         float now = best;
         uint32_t win = 4u;
-        if ((mine & 1u) && !(t0 >= now)) { now = t0; win = 0u; }
-        if ((mine & 2u) && !(t1 >= now)) { now = t1; win = 1u; }
-        if ((mine & 4u) && !(t2 >= now)) { now = t2; win = 2u; }
-        if ((mine & 8u) && !(t3 >= now)) { now = t3; win = 3u; }
+        bool was = false;
+        if ((mine & 1u) && !(t0 >= now)) { now = t0; win = 0u; was = was || now != now; }
+        if ((mine & 2u) && !(t1 >= now)) { now = t1; win = 1u; was = was || now != now; }
+        if ((mine & 4u) && !(t2 >= now)) { now = t2; win = 2u; was = was || now != now; }
+        if ((mine & 8u) && !(t3 >= now)) { now = t3; win = 3u; was = was || now != now; }
+        if (was) now = __builtin_nanf("");
         wins = __builtin_amdgcn_ballot_w64(win == k);
         nt = laneGetF(now, (below << 2) & 63u);
+        if (leaf && below < kLeafLanes && nt != nt) c.sp = c.base;
     }
     const bool tested = leaf && below < kLeafLanes;
     const uint32_t won = (uint32_t)(wins >> ((below << 2) & 63u)) & 15u;
@@ -786,6 +835,7 @@ __device__ __forceinline__ void traceWave(const DevScene& S, const Top& top, con
         // the cloud (a ray that misses it ends here at once).
         while (true) {
             if (state == kCloud && c.ref == kRefDone) {
+                if (c.best != c.best) cloudAgain(S, top.inst[inst].rootRef, st, c);  // a NaN distance was accepted
                 if (c.bestIdx != kInvalid) {
                     const F3 x = c.o + c.d * c.best;
                     const float tw = dot(x - o, d);

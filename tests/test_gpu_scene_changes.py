@@ -163,3 +163,21 @@ def test_release_gives_back_a_large_adjoints_queues(capacity):
     assert np.array_equal(r.render_view(scene.default_camera(256, 200), 16, 3)["raw"], img)
     again = r.render_view_backward(scene.default_camera(256, 200), 16, dl)["opacity"]
     assert np.allclose(again, grad, rtol=1e-4, atol=1e-4 * float(np.abs(grad).max()))
+
+
+@pytest.mark.parametrize("n", [40, 400])
+def test_degenerate_surfels_in_leaves(n):
+    """A surfel without a plane accepts a NaN distance, and after it the next
+    surfel of its leaf is accepted at any distance: where photons go and what a
+    camera sees follow the tests in leaf order."""
+    pts = scene.uniform_surfels(n, seed=4, scale_lo=0.2, scale_hi=0.4)[0]
+    pts["tangent_v"][::6] = pts["tangent_u"][::6]  # normalize(0)
+    spec = scene.SceneSpec([scene.light_quad()], [scene.default_camera(64, 48)], pts, {})
+    gpu, orc = _pair(spec, dict(photons=100_000, bounces=3, forward_passes=1, gather_passes=2, gather_radius=0.05,
+                                spp_decorrelate=1))
+    a, b = gpu.render_forward()["camera1_raw"], orc.render_forward()["camera1_raw"]
+    pa, pb = gpu.photons(), orc.photons()
+    assert pa["count"] == pb["count"] > 1000
+    for k in ("position", "power", "direction"):
+        assert np.array_equal(pa[k], pb[k], equal_nan=True), k
+    assert np.array_equal(a, b, equal_nan=True)

@@ -52,10 +52,7 @@ struct DevGrid {
 
 struct Hit {
     F3 pos;
-    float t;
-    float alpha;
-    uint32_t inst;  // kInvalid: miss
-    uint32_t prim;
+    uint32_t inst, prim;  // inst kInvalid: miss
 };
 
 // Per-thread work counters of the counting mode (the per-query units of the
@@ -146,44 +143,38 @@ struct LaneStack {
 
 struct LocalHit {
     F3 pos;
-    float t;
-    float alpha;
     uint32_t prim;
 };
 
 // intersectBLASPointCloudFirstHit (IntersectionKernels.h:585-675) with
-// intersectSurfel (KernelHelpers.h:637-669); alpha_geom is evaluated once for
-// the final hit (it is a pure function of the hit).
-template <bool kCount>
+// intersectSurfel (KernelHelpers.h:637-669), its work counted; alpha_geom is
+// left to who needs it (a pure function of the hit, surfelAlpha).
 __device__ bool traverseCloud(const DevScene& S, const DevInstance& I, F3 o, F3 d, const LaneStack& st,
                               uint32_t base, LocalHit& out, Work& w) {
     const F3 inv = safeInvDir(d);
     float best = __builtin_huge_valf();
     float te;
-    if (kCount) w.aabb++;  // the reference slab-tests the root when it pops it
+    w.aabb++;  // the reference slab-tests the root when it pops it
     if (!slab(o, inv, I.rmnx, I.rmny, I.rmnz, I.rmxx, I.rmxy, I.rmxz, best, 1e-6f, te)) {
-        if (kCount) w.pops++;
+        w.pops++;
         return false;
     }
     bool firstPop = true;
     uint32_t sp = base;
     st.push(sp, I.rootRef, te);
     uint32_t bestIdx = 0;
-    float bestR2 = 0.0f;
     F3 bestX = mk3(0, 0, 0);
     bool any = false;
     while (sp > base) {
         const uint2 e = st.get(--sp);
-        if (kCount) {
-            w.pops++;
-            if (!firstPop) w.aabb++;  // re-test of a popped box (root already counted)
-            firstPop = false;
-        }
+        w.pops++;
+        if (!firstPop) w.aabb++;  // re-test of a popped box (root already counted)
+        firstPop = false;
         if (__uint_as_float(e.y) > best) continue;
         const uint32_t ref = e.x;
         if (ref & kLeafBit) {
             const uint32_t first = leafFirst(ref), cnt = leafCount(ref);
-            if (kCount) w.prims += cnt;
+            w.prims += cnt;
             for (uint32_t k = 0; k < cnt; ++k) {
                 const uint32_t si = first + k;
                 const float4* g = reinterpret_cast<const float4*>(S.geo + si);
@@ -205,14 +196,13 @@ __device__ bool traverseCloud(const DevScene& S, const DevInstance& I, F3 o, F3 
                 best = t;
                 bestIdx = si;
                 bestX = x;
-                bestR2 = r2;
             }
             continue;
         }
         const float4* nd4 = reinterpret_cast<const float4*>(S.nodes + ref);
         const float4 a = nd4[0], b = nd4[1], c = nd4[2];
         const uint2 refs = reinterpret_cast<const uint2*>(S.nodes + ref)[6];  // left, right (not the padding)
-        if (kCount) w.aabb += 2;
+        w.aabb += 2;
         float tl = __builtin_huge_valf(), tr = __builtin_huge_valf();
         const bool hl = slab(o, inv, a.x, a.y, a.z, a.w, b.x, b.y, best, 1e-6f, tl);
         const bool hr = slab(o, inv, b.z, b.w, c.x, c.y, c.z, c.w, best, 1e-6f, tr);
@@ -231,10 +221,8 @@ __device__ bool traverseCloud(const DevScene& S, const DevInstance& I, F3 o, F3 
         }
     }
     if (!any) return false;
-    out.t = best;
     out.prim = bestIdx;
     out.pos = bestX;
-    out.alpha = pow_r(1.0f - bestR2, S.geo[bestIdx].e4b);
     return true;
 }
 
@@ -363,41 +351,6 @@ __device__ __forceinline__ void cloudNode(const DevScene& S, const LaneStack& st
     if (h1 && h0) st.pushBounded(c.sp, r1, t1);
     c.ref = h0 ? r0 : (h1 ? r1 : (h2 ? r2 : r3));
     if (!any2 && !h3) cloudPop(st, c);
-}
-
-__device__ __forceinline__ void cloudLeaf(const DevScene& S, const LaneStack& st, CloudLane& c) {
-    // A leaf holds at most four surfels: their records are loaded together
-    // before the first test.  The tests run in leaf order.
-    const uint32_t first = leafFirst(c.ref), cnt = leafCount(c.ref);
-    const float4* g = reinterpret_cast<const float4*>(S.geo + first);
-    float4 w[4][4];
-#pragma unroll
-    for (uint32_t k = 0; k < 4; ++k) {
-        if (k < cnt) {
-#pragma unroll
-            for (uint32_t j = 0; j < 4; ++j) w[k][j] = g[4 * k + j];
-        }
-    }
-#pragma unroll
-    for (uint32_t k = 0; k < 4; ++k) {
-        if (k >= cnt) break;
-        const float4 g0 = w[k][0], g1 = w[k][1], g2 = w[k][2], g3 = w[k][3];
-        const F3 n = mk3(g1.x, g1.y, g1.z);
-        const float nd = dot(n, c.d);
-        if (fabsf(nd) < 1e-6f) continue;
-        const F3 p = mk3(g0.x, g0.y, g0.z);
-        const float t = dot(n, p - c.o) / nd;
-        if (t <= 1e-5f || t >= c.best) continue;
-        const F3 x = c.o + c.d * t;
-        const F3 r = x - p;
-        const float uu = dot(mk3(g2.x, g2.y, g2.z), r) / g0.w;
-        const float vv = dot(mk3(g3.x, g3.y, g3.z), r) / g1.w;
-        const float r2 = uu * uu + vv * vv;
-        if (r2 >= 1.0f) continue;
-        c.best = t;
-        c.bestIdx = first + k;
-    }
-    cloudPop(st, c);
 }
 
 // The lane's traversal from the start, by the binary tree's steps and the tests
@@ -540,24 +493,6 @@ __device__ __forceinline__ bool cloudLeafRound(const DevScene& S, CloudLane& c, 
     return tested;
 }
 
-__device__ bool traverseCloudFast(const DevScene& S, const DevInstance& I, F3 o, F3 d, const LaneStack& st,
-                                  uint32_t base, LocalHit& out) {
-    CloudLane c;
-    if (!cloudBegin(I, o, d, base, c)) return false;
-    while (c.ref != kRefDone) {
-        if (c.ref & kLeafBit)
-            cloudLeaf(S, st, c);
-        else
-            cloudNode(S, st, c);
-    }
-    if (c.bestIdx == kInvalid) return false;
-    out.t = c.best;
-    out.prim = c.bestIdx;
-    out.pos = c.o + c.d * c.best;
-    out.alpha = surfelAlpha(S.geo[c.bestIdx], out.pos);
-    return true;
-}
-
 // intersectTriangle (KernelHelpers.h:248-277)
 __device__ __forceinline__ bool intersectTri(F3 o, F3 d, F3 v0, F3 v1, F3 v2, float tMin, float& tOut) {
     const F3 e1 = v1 - v0, e2 = v2 - v0;
@@ -641,10 +576,8 @@ __device__ bool traverseMesh(const DevScene& S, const DevInstance& I, F3 o, F3 d
         }
     }
     if (!any) return false;
-    out.t = best;
     out.prim = bestTri;
     out.pos = toWorldPoint(I.o2w, o + d * best);
-    out.alpha = 0.0f;
     return true;
 }
 
@@ -678,31 +611,25 @@ __device__ inline void loadTopLds(const DevScene& S, TopLds& t) {
     __syncthreads();
 }
 
-template <bool kCount>
-__device__ bool intersectScene(const DevScene& S, F3 o, F3 d, const LaneStack& st, Hit& h, Work& w);
-
-template <bool kCount, typename Top>
-__device__ bool intersectSceneTop(const DevScene& S, const Top& top, F3 o, F3 d, const LaneStack& st, Hit& h,
-                                  Work& w) {
+// One query, its work counted as the reference's.
+template <typename Top>
+__device__ void intersectScene(const DevScene& S, const Top& top, F3 o, F3 d, const LaneStack& st, Hit& h, Work& w) {
     h.inst = kInvalid;
-    if (S.nTlas == 0) return false;
+    if (S.nTlas == 0) return;
     const F3 inv = safeInvDir(d);
     float bestW = __builtin_huge_valf();
-    bool found = false;
     uint32_t sp = 0;
     st.push(sp, 0u, 0.0f);
     while (sp > 0) {
         const uint32_t ni = st.get(--sp).x;
         const TlasNode nd = top.tlas[ni];
-        if (kCount) {
-            w.pops++;
-            w.aabb++;
-        }
+        w.pops++;
+        w.aabb++;
         float te;
         if (!slab(o, inv, nd.mnx, nd.mny, nd.mnz, nd.mxx, nd.mxy, nd.mxz, bestW, 0.0f, te)) continue;
         if (nd.count == 0) {
             const TlasNode L = top.tlas[nd.left], R = top.tlas[nd.right];
-            if (kCount) w.aabb += 2;
+            w.aabb += 2;
             float tl = __builtin_huge_valf(), tr = __builtin_huge_valf();
             const bool hl = slab(o, inv, L.mnx, L.mny, L.mnz, L.mxx, L.mxy, L.mxz, bestW, 0.0f, tl);
             const bool hr = slab(o, inv, R.mnx, R.mny, R.mnz, R.mxx, R.mxy, R.mxz, bestW, 0.0f, tr);
@@ -733,30 +660,19 @@ __device__ bool intersectSceneTop(const DevScene& S, const Top& top, F3 o, F3 d,
         LocalHit lh;
         bool acc;
         if (I.type == kGeoMesh)
-            acc = traverseMesh<kCount>(S, I, oo, od, st, sp, lh, w);
-        else if (kCount)
-            acc = traverseCloud<kCount>(S, I, oo, od, st, sp, lh, w);
+            acc = traverseMesh<true>(S, I, oo, od, st, sp, lh, w);
         else
-            acc = traverseCloudFast(S, I, oo, od, st, sp, lh);
+            acc = traverseCloud(S, I, oo, od, st, sp, lh, w);
         if (acc) {
             const float tw = dot(lh.pos - o, d);
             if (tw > 0.0f && tw < bestW) {
                 bestW = tw;
-                found = true;
-                h.t = tw;
                 h.pos = lh.pos;
                 h.inst = ii;
                 h.prim = lh.prim;
-                h.alpha = lh.alpha;
             }
         }
     }
-    return found;
-}
-
-template <bool kCount>
-__device__ bool intersectScene(const DevScene& S, F3 o, F3 d, const LaneStack& st, Hit& h, Work& w) {
-    return intersectSceneTop<kCount>(S, TopGlobal{S.tlas, S.inst}, o, d, st, h, w);
 }
 
 // Queries of a whole wave (intersectScene for every lane, FirstHit mode), by
@@ -785,26 +701,21 @@ __device__ bool intersectScene(const DevScene& S, F3 o, F3 d, const LaneStack& s
 // 16: 5 % slower to 2 % slower; kEndShare 1 and 3: 40 % and 5 % slower.  The photon
 // and adjoint traces run the same with other values (within 1 %).
 //
-// Job: bool finish(bool done, const JobHit&, const Work&, F3& o, F3& d) takes
+// Job: bool finish(bool done, const Hit&, const Work&, F3& o, F3& d) takes
 // the hits of the lanes with done set (and the work of their queries in
 // counting mode) and returns whether the lane goes on with a new ray (o, d),
 // bool fetch(bool idle, F3& o, F3& d) gives idle lanes new work; both are
 // called by every lane of the wave.  drained(): no more work to fetch
 // (uniform over the wave).  kGoesOn: finish may give a lane a new ray.
 // Counting mode runs the counting traversal, query by query.
-struct JobHit {
-    F3 pos;
-    uint32_t inst, prim;  // inst kInvalid: miss
-};
-
 constexpr uint32_t kLeafMin = 12, kLeafShare = 2, kEndShare = 2;
 
 template <bool kCount, typename Top, typename Job>
 __device__ __forceinline__ void traceWave(const DevScene& S, const Top& top, const LaneStack& st, Job& job) {
-    if (kCount) {
+    if constexpr (kCount) {
         F3 o = mk3(0, 0, 0), d = mk3(0, 0, 1);
         bool has = false;
-        JobHit h{};
+        Hit h{};
         Work w{};
         while (true) {
             has = job.finish(has, h, w, o, d);
@@ -815,10 +726,7 @@ __device__ __forceinline__ void traceWave(const DevScene& S, const Top& top, con
             }
             if (has) {
                 w = Work{};
-                Hit q;
-                h.inst = intersectSceneTop<kCount>(S, top, o, d, st, q, w) ? q.inst : kInvalid;
-                h.prim = q.prim;
-                h.pos = q.pos;
+                intersectScene(S, top, o, d, st, h, w);
             }
         }
     }
@@ -827,7 +735,7 @@ __device__ __forceinline__ void traceWave(const DevScene& S, const Top& top, con
     F3 o = mk3(0, 0, 0), d = mk3(0, 0, 1);
     CloudLane c{};
     c.ref = kRefDone;
-    JobHit h{};
+    Hit h{};
     float bestW = 0.0f;
     uint32_t inst = 0;  // instance being traversed
     while (true) {
@@ -981,8 +889,7 @@ __device__ bool alphaGradient(const SurfelGeo& s, F3 o, F3 d, float g[12]) {
 }
 
 // buildIntersectionNormal (KernelHelpers.h:480-503)
-template <typename H>
-__device__ __forceinline__ F3 hitNormal(const DevScene& S, const H& h) {
+__device__ __forceinline__ F3 hitNormal(const DevScene& S, const Hit& h) {
     const DevInstance& I = S.inst[h.inst];
     if (I.type == kGeoMesh) {
         const TriGeo tg = S.tris[h.prim];

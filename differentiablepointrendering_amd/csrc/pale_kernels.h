@@ -377,7 +377,7 @@ void launchBvhWide(hipStream_t s, const uint4* wide, uint32_t nWide, const float
 void launchBvhRecords(hipStream_t s, const HostPoint* pts, const uint32_t* ord, uint32_t n, SurfelGeo* geo,
                       SurfelShade* shade);
 void launchGatherPoints(hipStream_t s, const DevGrid& G, uint32_t n, const float* q, const float* nrm, float* out);
-void launchTraceRays(hipStream_t s, const DevScene& S, uint32_t n, const float* o, const float* d, int32_t* inst,
-                     int32_t* prim, float* t, float* pos, float* alpha);
+void launchTraceRays(hipStream_t s, const DevScene& S, DevState* st, uint32_t n, const float* o, const float* d,
+                     int32_t* inst, int32_t* prim, float* t, float* pos, float* alpha);
 
 }  // namespace pale

@@ -2621,8 +2621,8 @@ int pale_trace_rays(pale_handle* h, uint32_t n, const float* origins, const floa
         al.reserve((size_t)n * 4);
         HIPCHECK(hipMemcpy(o.p, origins, (size_t)n * 12, hipMemcpyHostToDevice));
         HIPCHECK(hipMemcpy(d.p, directions, (size_t)n * 12, hipMemcpyHostToDevice));
-        launchTraceRays(h->stream, h->scene, n, o.as<float>(), d.as<float>(), ii.as<int32_t>(), pp.as<int32_t>(),
-                        tt.as<float>(), ps.as<float>(), al.as<float>());
+        launchTraceRays(h->stream, h->scene, h->st(), n, o.as<float>(), d.as<float>(), ii.as<int32_t>(),
+                        pp.as<int32_t>(), tt.as<float>(), ps.as<float>(), al.as<float>());
         HIPCHECK(hipStreamSynchronize(h->stream));
         HIPCHECK(hipGetLastError());
         HIPCHECK(hipMemcpy(instance_out, ii.p, (size_t)n * 4, hipMemcpyDeviceToHost));

@@ -181,3 +181,23 @@ def test_degenerate_surfels_in_leaves(n):
     for k in ("position", "power", "direction"):
         assert np.array_equal(pa[k], pb[k], equal_nan=True), k
     assert np.array_equal(a, b, equal_nan=True)
+
+
+@pytest.mark.parametrize("rays", [1, 63, 64, 65, 4097, 700_001])
+def test_probe_rays(rays):
+    """Rays of a caller, by the traversal that the renderer uses: fewer than a
+    wave, at a wave's edges, and more than the device holds lanes."""
+    spec = scene.config_scene(0, n=1500, width=8, height=8)
+    spec.meshes.append(scene.quad_mesh("floor", (0.0, -1.1, 0.0), scene.FACING_UP, 0.8, (0.6, 0.5, 0.4)))
+    gpu, orc = _pair(spec, dict(photons=100))
+    rng = np.random.default_rng(rays)
+    o = rng.uniform(-1.5, 1.5, size=(rays, 3)).astype(np.float32)
+    d = rng.normal(size=(rays, 3))
+    d = (d / np.linalg.norm(d, axis=1, keepdims=True)).astype(np.float32)
+    if rays == 4097:  # rays that are none among the others
+        o[5::40, 0], o[6::40, 1], o[7::40] = np.nan, np.inf, 1e30
+        d[8::40, 2], d[9::40, 0], d[10::40] = np.nan, -np.inf, 0.0
+    a, b = gpu.trace_rays(o, d), orc.trace(o, d)
+    for k in ("instance", "primitive", "t", "position"):
+        assert np.array_equal(a[k], b[k], equal_nan=a[k].dtype.kind == "f"), k
+    np.testing.assert_allclose(a["alpha"], b["alpha"], rtol=1e-6, atol=0)

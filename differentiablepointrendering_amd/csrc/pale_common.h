@@ -26,6 +26,18 @@ constexpr uint32_t kInvalid = 0xFFFFFFFFu;
 constexpr uint32_t kLeafBit = 0x80000000u;
 constexpr uint32_t kMaxLeafPrims = 4u;  // BuildOptions (SceneBuild.ixx:72-75)
 
+// Counts and indexes of up to 2^32 - 1 items (a photon grid may have nearly as
+// many cells), none of which may wrap.
+PALE_HD constexpr uint32_t ceilDiv(uint32_t n, uint32_t d) { return n / d + (n % d != 0u ? 1u : 0u); }
+// Items i .. i + 3 are below n.
+PALE_HD constexpr bool wholeFour(uint32_t i, uint32_t n) { return i < n && n - i >= 4u; }
+// The next item of a strided loop at item i < n; false: none.
+PALE_HD bool nextItem(uint32_t& i, uint32_t stride, uint32_t n) {
+    if (n - i <= stride) return false;
+    i += stride;
+    return true;
+}
+
 struct F3 {
     float x, y, z;
 };

@@ -110,13 +110,25 @@ __device__ __forceinline__ uint32_t f2u(float f) { return __float_as_uint(f); }
 
 // ---------------------------------------------------------------- small --
 __global__ void k_fill(uint32_t* p, uint32_t n, uint32_t v) {
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = v;
+    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    do {
+        p[i] = v;
+    } while (nextItem(i, gridDim.x * blockDim.x, n));
 }
 __global__ void k_fillf(float* p, uint32_t n, float v) {
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = v;
+    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    do {
+        p[i] = v;
+    } while (nextItem(i, gridDim.x * blockDim.x, n));
 }
 __global__ void k_iota(uint32_t* p, uint32_t n) {
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = i;
+    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    do {
+        p[i] = i;
+    } while (nextItem(i, gridDim.x * blockDim.x, n));
 }
 
 // Between the launches of the photon stage.  Seed schedule of
@@ -770,7 +782,6 @@ __global__ __launch_bounds__(256) void k_cell_count(GridParams g, const DevState
     atomicAdd(&cellCount[c], 1u);
 }
 
-// Exclusive scan, pass 1: per-tile scan of `in` into `out`, tile sums.
 // Exclusive scan of the counts of a grid's cells (or of an image's pixels) in
 // one pass: the tiles' sums by look-back, 16 bytes per lane and load; out[n] =
 // the sum of all.  in and out are the starts of their allocations.  Every count
@@ -792,7 +803,7 @@ __global__ __launch_bounds__(kScanBlock) void k_scan(const uint32_t* in, uint32_
 #pragma unroll
     for (uint32_t k = 0; k < kLoads; ++k) {
         const uint32_t i = first + k * (kScanBlock * 4u);
-        if (i + 4u <= n)
+        if (wholeFour(i, n))
             v[k] = *reinterpret_cast<const uint4*>(in + i);
         else
             v[k] = make_uint4(i < n ? in[i] : 0u, i + 1u < n ? in[i + 1u] : 0u, i + 2u < n ? in[i + 2u] : 0u, 0u);
@@ -846,7 +857,7 @@ __global__ __launch_bounds__(kScanBlock) void k_scan(const uint32_t* in, uint32_
         o.y = o.x + v[k].x;
         o.z = o.y + v[k].y;
         o.w = o.z + v[k].z;
-        if (i + 4u <= n) {
+        if (wholeFour(i, n)) {
             *reinterpret_cast<uint4*>(out + i) = o;
         } else {
             if (i < n) out[i] = o.x;
@@ -2112,7 +2123,7 @@ __global__ __launch_bounds__(256) void k_quad_nodes(const WideNode* nodes, QuadN
 }
 
 // ------------------------------------------------------------ launchers --
-static inline uint32_t blocks(uint32_t n, uint32_t b) { return (n + b - 1) / b; }
+static inline uint32_t blocks(uint32_t n, uint32_t b) { return ceilDiv(n, b); }
 // Grid of the light per-item kernels (keys and scatters of the entry and
 // event sorts) that stride over buffers whose count is known only on the
 // device: 256 CUs x 32 workgroups of 256 lanes.

@@ -8,7 +8,7 @@
 
 namespace pale {
 
-constexpr uint32_t kTile = 1024;       // compaction / scan tile (256 threads x 4)
+constexpr uint32_t kTile = 1024;       // items of a compaction tile, one per thread (reservoir ranks: four)
 constexpr uint32_t kScanBlock = 512;    // threads of an exclusive scan's workgroup
 constexpr uint32_t kScanTile = 16384;   // its items
 // Scratch bytes of an exclusive scan of n items: a ticket and the tiles' states.

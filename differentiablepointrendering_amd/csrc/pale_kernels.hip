@@ -712,7 +712,7 @@ __global__ __launch_bounds__(256) void k_resv_write(const DevState* st, Reservoi
     raw.powZ[sl] = dep.powZ[i];
 }
 
-// --------------------------------------------------------- tile scans --
+// ------------------------------------------- ranks of a full map's deposits --
 __global__ __launch_bounds__(kScanThreads) void k_tile_count(const uint8_t* flags, const uint32_t* count,
                                                              uint32_t maxItems, uint32_t* tiles) {
     const uint32_t n = loadCount(count, maxItems);
@@ -726,14 +726,10 @@ __global__ __launch_bounds__(kScanThreads) void k_tile_count(const uint8_t* flag
     if (threadIdx.x == 0) tiles[blockIdx.x] = total;
 }
 
-// Exclusive scan of the tile sums (one workgroup); *total = sum, clamped to
-// `cap`.  The number of tiles is ceil(n / kTile) for n = *count (or
-// `fixedN` if count is null).
-__global__ __launch_bounds__(1024) void k_tile_scan(uint32_t* tiles, const uint32_t* count, uint32_t fixedN,
-                                                    uint32_t maxItems, uint32_t* total, uint32_t cap) {
+// Exclusive scan of the tile sums (one workgroup).
+__global__ __launch_bounds__(1024) void k_tile_scan(uint32_t* tiles, const uint32_t* count, uint32_t maxItems) {
     __shared__ uint32_t sums[1024 / 64 + 1];
-    const uint32_t n = count ? loadCount(count, maxItems) : fixedN;
-    const uint32_t numTiles = (n + kTile - 1) / kTile;
+    const uint32_t numTiles = ceilDiv(loadCount(count, maxItems), kTile);
     uint32_t carry = 0;
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     for (uint32_t base = 0; base < numTiles; base += 1024) {
@@ -761,7 +757,6 @@ __global__ __launch_bounds__(1024) void k_tile_scan(uint32_t* tiles, const uint3
         carry += sums[1024 / 64];
         __syncthreads();
     }
-    if (threadIdx.x == 0) *total = carry < cap ? carry : cap;
 }
 
 // ------------------------------------------------------ photon grid --
@@ -2215,7 +2210,7 @@ void launchPhotonShade(hipStream_t s, const DevScene& S, DevState* st, uint32_t 
         const uint32_t nt = blocks(maxRays, kTile);
         k_photon_probe<<<blocks(maxRays, 256), 256, 0, s>>>(S, st, hits, depFlags, tp);
         k_tile_count<<<nt, kScanThreads, 0, s>>>(depFlags, qCount, maxRays, tiles);
-        k_tile_scan<<<1, 1024, 0, s>>>(tiles, qCount, 0u, maxRays, tiles + nt, 0xFFFFFFFFu);
+        k_tile_scan<<<1, 1024, 0, s>>>(tiles, qCount, maxRays);
         k_resv_rank<<<nt, kScanThreads, 0, s>>>(depFlags, st, tiles, rs.attempt);
     }
     k_photon_shade<<<tilesOf(maxRays), kTile, 0, s>>>(S, st, in, hits, out, outCap, map, staged, tp, rs, ts);

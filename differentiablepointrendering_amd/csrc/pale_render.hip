@@ -757,7 +757,7 @@ struct pale_handle {
             a(depStg[1], (size_t)cap * sizeof(float4));
             a(depStg[2], (size_t)cap * sizeof(float));
             a(depFlags, cap);
-            a(tiles, ((size_t)cap / kTile + 4) * sizeof(uint32_t));
+            a(tiles, ((size_t)cap / kTile + 1) * sizeof(uint32_t));
             a(resvAttempt, (size_t)cap * sizeof(uint32_t));
             a(resvSlot, (size_t)cap * sizeof(uint32_t));
         }

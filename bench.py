@@ -283,8 +283,9 @@ def pmc_summary(dirs, cal_dirs=None):
                 u["l1_accesses"] = c["TCP_TOTAL_CACHE_ACCESSES_sum"] / 256.0 / cyc
             if "SQ_ACTIVE_INST_VALU" in c:
                 # A vector instruction of a wave takes a SIMD four cycles.  (The
-                # cycles are another pass's: a little above 1 can come out.)
-                u["valu_busy"] = min(1.0, c["SQ_ACTIVE_INST_VALU"] * 4.0 / 1024.0 / cyc)
+                # cycles are another pass's: a saturated kernel can come out a
+                # little above 1.)
+                u["valu_busy"] = c["SQ_ACTIVE_INST_VALU"] * 4.0 / 1024.0 / cyc
                 if "SQ_THREAD_CYCLES_VALU" in c:
                     u["valu_lanes"] = c["SQ_THREAD_CYCLES_VALU"] / max(c["SQ_ACTIVE_INST_VALU"], 1.0) / 64.0
             k["utilisation"] = u

@@ -674,24 +674,21 @@ __device__ void intersectScene(const DevScene& S, const Top& top, F3 o, F3 d, co
 //
 // With one query per lane run to the wave's longest, and each iteration
 // stepping the lanes at a leaf and the lanes at a node, the traversals were bound
-// by vector instructions: issued in 70-80 % of a SIMD's cycles, with 16 % (photon
-// trace), 21 % (adjoint trace), 23 % and 49 % (camera walk, independent and
-// shared samples) of their lanes enabled; 1M clustered surfels, 50 nodes of the
-// binary tree and 7.5 leaves per query.  So a wave takes one kind of step at a
-// time, for the lanes that are at that kind: a leaf round (cloudLeafRound, 100
-// vector instructions; a node step has 170) once kLeafMin lanes or 1 /
-// kLeafShare of those that traverse wait at a leaf, and the ends and starts of
-// queries once 1 / kEndShare of the lanes that were traversing have ended.
-// Camera walk of 16 passes at 800x800, shared and independent: 41.6 and 87.5 ms
-// before; 36.9 and 56.5 so; 33.4 and 50.6 with the walk's hits shaded elsewhere
-// and 5 waves per SIMD; 30.6 and 49.0 with quad nodes.  Photon trace 10.1 -> 6.1
-// -> 5.1 -> 4.5 ms, adjoint trace 31.2 -> 23.2 -> 19.4 -> 11.5 ms (independent; the
-// last with its shading elsewhere, first rays given and batches of 10 Mi rays).
-// Vector instructions now take 95 % of the walk's cycles with shared samples, 80 %
-// with independent ones, where L1 accesses take 79 %; a sixth of its time passes
-// after the last pixel is drawn, while the longest pixels end.  kLeafMin 6, 8, 10,
-// 16: 5 % slower to 2 % slower; kEndShare 1 and 3: 40 % and 5 % slower.  The photon
-// and adjoint traces run the same with other values (within 1 %).
+// by vector instructions of which 16 % (photon trace) to 49 % (camera walk, shared
+// samples) of the lanes took part; a query of 1M clustered surfels visits 50 nodes
+// of the binary tree and 7.5 leaves.  So a wave takes one kind of step at a time,
+// for the lanes that are at that kind: a leaf round (cloudLeafRound, 100 vector
+// instructions; a node step has 170) once kLeafMin lanes or 1 / kLeafShare of those
+// that traverse wait at a leaf, and the ends and starts of queries once 1 /
+// kEndShare of the lanes that were traversing have ended.
+//
+// Camera walk of 16 passes at 800x800 on 1M surfels: 41.6 ms before, 28.4 now (87.5
+// and 45.4 with independent samples).  Vector instructions take all of its cycles
+// with shared samples, 84 % with independent ones, where L1 accesses take 80 %; a
+// sixth of its time passes after the last pixel is drawn, while the longest pixels
+// end.  kLeafMin 6, 8, 10, 16: 5 % slower to 2 % slower; kEndShare 1 and 3: 40 % and
+// 5 % slower.  The photon and adjoint traces run the same with other values (within
+// 1 %).
 //
 // Job: bool finish(bool done, const Hit&, const Work&, F3& o, F3& d) takes
 // the hits of the lanes with done set (and the work of their queries in

@@ -1371,9 +1371,9 @@ __global__ __launch_bounds__(256) void k_entry_scatter(const DevState* st, uint3
 // the slot's layer list (the products the reference's loop forms,
 // PrimalKernels.cpp:583-585, :620, :626-628).
 //
-// Bound by vector instructions (issued in 80-89 % of the cycles with shared
-// seeds, 60-64 % with independent samples), then by the latency of the rows'
-// dependent loads: 5 waves per SIMD (at most 96 VGPRs) instead of 4.  12.2 ->
+// Bound by vector instructions with shared seeds (issued in all of the cycles;
+// 72 % with independent samples, 48 GB a launch at 0.39 of the HBM rate), then
+// by the latency of the rows' dependent loads: 5 waves per SIMD (at most 96 VGPRs) instead of 4.  12.2 ->
 // 8.8 ms and 18.1 -> 14.0 ms for the 102 M gathers of the 1M-surfel step: row
 // bounds without IEEE divisions and square roots (GridRows; -1.0, -1.8 ms),
 // photons two at a time instead of four (-1.6 ms), the fifth wave (-0.6 ms).

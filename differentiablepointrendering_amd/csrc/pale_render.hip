@@ -283,10 +283,11 @@ class DeviceCloudBuild final : public CloudBuild {
 };
 
 // ------------------------------------------- no-allocation adjoint --
-// pale_render_view_backward_noalloc keeps every intermediate of the adjoint
-// of one view (ray queues, pending states, event staging and pool, flags,
-// compaction tiles) in this file-scope device array instead of buffers the
-// library allocates: views of at most kNoAllocMaxPixels pixels.  Each GPU
+// pale_render_view_backward_noalloc keeps the intermediates of the adjoint of
+// one view (ray queues, hits, pending states, event pool) in this file-scope
+// device array instead of buffers the library allocates: views of at most
+// kNoAllocMaxPixels pixels.  (The tile states of its compactions are the
+// handle's, made with the photon stage's queues.)  Each GPU
 // holds its own copy for the life of the process.  In host code `scratch` is
 // only a symbol: its device address comes from hipGetSymbolAddress, resolved
 // once per device (noAllocScratch) and kept in the handle.
@@ -787,7 +788,10 @@ struct pale_handle {
         a(entStart, ((size_t)grid.total + 1) * 4);
         // Event pool: the events of up to 24 bounces of npx paths wait for
         // one cell-sorted transport launch; in a batch of more than 4 Mi rays
-        // those of 19 bounces of 4 Mi or of its largest sample.
+        // those of 19 bounces of 4 Mi or of its largest sample: five fewer than
+        // a batch of 4 Mi keeps, which gives back 1.5 of the 2.1 GB that the
+        // larger queues take (cutBackward) and still holds 7 bounces of 16
+        // samples of 800x800.
         const uint32_t small = std::min(npx, std::max(kAdjointBatch, pass));
         const uint64_t most = std::min<uint64_t>((uint64_t)small * (npx > small ? 19u : 24u), 1u << 28);
         uint32_t pool = (uint32_t)std::max<uint64_t>(npx, std::min(most, events));

@@ -302,13 +302,15 @@ class Renderer:
         return v.value
 
     def view_buffer_bytes(self) -> int:
-        """Device bytes of the image-sized buffers (what release_view_buffers frees)."""
+        """Device bytes of the image-sized buffers and of the ray queues beyond the photon
+        stage's (what release_view_buffers frees)."""
         v = C.c_uint64()
         check(self._L.pale_view_buffer_bytes(self._h, C.byref(v)))
         return v.value
 
     def release_view_buffers(self) -> None:
-        """Frees the image-sized buffers; scene and photon map stay."""
+        """Frees the image-sized buffers and takes the ray queues back to the photon
+        stage's size; scene and photon map stay."""
         check(self._L.pale_release_view_buffers(self._h))
 
     def render_view(self, camera: _abi.Camera, spp: int, seed: int) -> dict:

@@ -1443,12 +1443,12 @@ struct pale_handle {
             outLdr = viewsLdr.as<float4>();
             return;
         }
-        outFb = viewFb.as<float4>();
-        outLdr = viewLdr.as<float4>();
         const uint32_t npx = c.W * c.H;
         ensureCamera(npx);
         viewFb.reserve((size_t)npx * sizeof(float4));
         viewLdr.reserve((size_t)npx * sizeof(float4));
+        outFb = viewFb.as<float4>();
+        outLdr = viewLdr.as<float4>();
         tReset();
         camRounds = 0;
         HIPCHECK(hipEventRecord(ev0, stream));

@@ -201,3 +201,20 @@ def test_probe_rays(rays):
     for k in ("instance", "primitive", "t", "position"):
         assert np.array_equal(a[k], b[k], equal_nan=a[k].dtype.kind == "f"), k
     np.testing.assert_allclose(a["alpha"], b["alpha"], rtol=1e-6, atol=0)
+
+
+@pytest.mark.parametrize("batched", [0, 1])
+def test_views_that_grow(batched):
+    """The first view of a renderer and views larger than those before it, pass
+    by pass and batched, also after a release, come from the buffers that they
+    were rendered into."""
+    spec = scene.config_scene(0, n=600, width=16, height=16)
+    gpu, orc = _pair(spec, dict(photons=3000, batch_passes=batched))
+    gpu.build_photon_map()
+    orc.build_photon_map()
+    for w, h in ((5, 3), (40, 30), (90, 70), (17, 9)):
+        got, want = gpu.render_view(scene.default_camera(w, h), 2, 7), orc.render_view(scene.default_camera(w, h), 2, 7)
+        assert np.array_equal(got["raw"], want["raw"]), (w, h)
+        np.testing.assert_allclose(got["ldr"], want["ldr"], rtol=1e-4, atol=1e-6)
+        if w == 90:
+            gpu.release_view_buffers()

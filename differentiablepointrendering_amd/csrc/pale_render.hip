@@ -424,6 +424,22 @@ struct pale_handle {
     std::vector<uint32_t> debugCams;
     // Device address of this GPU's no-allocation scratch array.
     char* scratchBase = nullptr;
+    // Point i into the asset's place i, as an update leaves it (shape is not
+    // mirrored, as in the reference, pale_bindings.cpp:1025-1040).  The points are
+    // in tree order, the asset's in another until the first update after a build.
+    bool assetInTreeOrder = false;
+    void mirrorPoint(size_t i) {
+        const HostPoint& q = bp.points[i];
+        AssetPoint& a = asset[i];
+        a.p = q.p;
+        a.tu = q.tu;
+        a.tv = q.tv;
+        a.su = q.su;
+        a.sv = q.sv;
+        a.albedo = q.albedo;
+        a.opacity = q.opacity;
+        a.beta = q.beta;
+    }
     void syncHostPoints() {
         if (!hostStale) return;
         const size_t n = bp.points.size();
@@ -441,16 +457,9 @@ struct pale_handle {
             q.albedo = mk3(v[11], v[12], v[13]);
             q.opacity = v[14];
             q.beta = v[15];
-            AssetPoint& a = asset[i];
-            a.p = q.p;
-            a.tu = q.tu;
-            a.tv = q.tv;
-            a.su = q.su;
-            a.sv = q.sv;
-            a.albedo = q.albedo;
-            a.opacity = q.opacity;
-            a.beta = q.beta;
+            mirrorPoint(i);
         }
+        assetInTreeOrder = true;
         refreshSurfels(bp.points, img);
         hostStale = false;
     }
@@ -619,6 +628,7 @@ struct pale_handle {
         cloudBuild.shade = &shade;
         cloudBuild.nodes = &nodes;
         cloudBuild.minCount = S.bvh_build == 1 ? 0u : 65536u;
+        assetInTreeOrder = false;
         buildScene(meshes, asset, bp, S.bvh_build == 2 ? nullptr : &cloudBuild);
         makeDeviceImage(bp, meshes, img);
         uploadScene();
@@ -2212,11 +2222,18 @@ int pale_set_opacity_device(pale_handle* h, const float* opacity_dev, uint32_t n
         // (the host image is rebuilt before any upload; after a device BVH
         // build it is not kept)
         const bool img = h->img.surfShade.size() == n;
-        for (uint32_t i = 0; i < n; ++i) {
-            h->bp.points[i].opacity = v[i];
-            h->asset[i].opacity = v[i];
-            if (img) h->img.surfShade[i].opacity = v[i];
-        }
+        constexpr size_t kChunk = 1u << 14;
+        parallelFor((n + kChunk - 1) / kChunk, [&](size_t c) {
+            for (size_t i = c * kChunk; i < std::min<size_t>(n, (c + 1) * kChunk); ++i) {
+                h->bp.points[i].opacity = v[i];
+                if (h->assetInTreeOrder)
+                    h->asset[i].opacity = v[i];
+                else
+                    h->mirrorPoint(i);
+                if (img) h->img.surfShade[i].opacity = v[i];
+            }
+        });
+        h->assetInTreeOrder = true;
     });
 }
 
@@ -2477,22 +2494,13 @@ int pale_apply_points(pale_handle* h, const pale_points_desc* points) {
                     q.opacity = p.opacity[i];
                     q.beta = p.beta[i];
                     if (stage) stage[i] = q;
-                    // Mirror into the asset (shape is not mirrored, as in the
-                    // reference, pale_bindings.cpp:1025-1040).
-                    AssetPoint& a = h->asset[i];
-                    a.p = q.p;
-                    a.tu = q.tu;
-                    a.tv = q.tv;
-                    a.su = q.su;
-                    a.sv = q.sv;
-                    a.albedo = q.albedo;
-                    a.opacity = q.opacity;
-                    a.beta = q.beta;
+                    h->mirrorPoint(i);
                 }
             },
             [&](size_t done) {
                 if (stage) h->cloudBuild.staged((uint32_t)done);
             });
+        h->assetInTreeOrder = true;
         if (stage) {
             h->cloudBuild.records((uint32_t)p.count);
         } else {

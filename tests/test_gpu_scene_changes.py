@@ -218,3 +218,25 @@ def test_views_that_grow(batched):
         np.testing.assert_allclose(got["ldr"], want["ldr"], rtol=1e-4, atol=1e-6)
         if w == 90:
             gpu.release_view_buffers()
+
+
+def test_opacities_set_on_the_device_outlive_a_rebuild():
+    """set_opacity_device is an update of the points in tree order: a rebuild
+    after it gives what apply_point_optimization with those opacities gives."""
+    import torch
+
+    from differentiablepointrendering_amd.pale import Renderer
+
+    spec = scene.config_scene(0, n=3000, width=48, height=40)
+    print("case: opacities set on the device, then a rebuild", flush=True)
+    a, b = (Renderer.from_spec(spec, dict(photons=10_000)) for _ in range(2))
+    p = {k: v for k, v in b.get_point_parameters().items() if k in KEYS}
+    p["opacity"] = np.random.default_rng(4).uniform(0.1, 0.9, size=p["opacity"].shape).astype(np.float32)
+    b.apply_point_optimization(p)
+    a.set_opacity_device(torch.from_numpy(p["opacity"]).cuda())
+    for r in (a, b):
+        r.rebuild_bvh()
+    x, y = a.get_point_parameters(), b.get_point_parameters()
+    for k in KEYS:
+        assert np.array_equal(x[k], y[k]), k
+    assert np.array_equal(a.render_forward()["camera1_raw"], b.render_forward()["camera1_raw"])
